@@ -266,11 +266,12 @@ size_t spyre_sdpa_fwd_workspace_bytes(int B, int Hkv, int Skv, int D);
  * grid fills at least half the device: when a sequence spans several
  * chunks, their fp32 partials B * Hkv * chunks * g * (D + 2) * 4 bytes and a
  * 4-byte arrival flag per (sequence, KV head, chunk), also without
- * initialisation (the chunks merge in the one kernel).  With a mask: 0 for fp16 / bool masks with
- * key stride 1, a 16-byte aligned pointer, b / h / i strides and Skv of
- * whole 16 bytes (staged in LDS beside K and V as they lie); for other fp16 / bool
- * masks, a copy with 16-byte rows of the mask's non-broadcast extent (then
- * staged the same way); for fp32 masks, spyre_sdpa_fwd_workspace_bytes.  A
+ * initialisation (the chunks merge in the one kernel).  With a mask: a key
+ * split's partials as above, and before them (its size rounded up to 256
+ * bytes) for fp16 / bool masks other than those with key stride 1, a 16-byte
+ * aligned pointer, b / h / i strides and Skv of whole 16 bytes (staged in
+ * LDS beside K and V as they lie) a copy with 16-byte rows of the mask's
+ * non-broadcast extent (then staged the same way); for fp32 masks, spyre_sdpa_fwd_workspace_bytes.  A
  * call whose fp16 / bool mask needs a copy but whose workspace holds only
  * spyre_sdpa_fwd_workspace_bytes runs the fp32-mask kernel instead (same
  * results within the SDPA tolerance, slower).  No reference counterpart:
@@ -279,6 +280,15 @@ size_t spyre_sdpa_fwd_workspace_bytes(int B, int Hkv, int Skv, int D);
 size_t spyre_sdpa_fwd_call_workspace_bytes(const void* attn_mask, int mask_kind,
                                            const int64_t* mask_strides, int B, int Hq, int Hkv,
                                            int Sq, int Skv, int D);
+
+/* The least workspace spyre_sdpa_fwd_f16 accepts for the call (same
+ * arguments): 0 without a mask or for a mask staged as it lies; the smaller
+ * of its copy and V's relayout for other fp16 / bool masks; V's relayout for
+ * fp32 masks.  What spyre_sdpa_fwd_call_workspace_bytes asks beyond it only
+ * makes the call faster. */
+size_t spyre_sdpa_fwd_min_workspace_bytes(const void* attn_mask, int mask_kind,
+                                          const int64_t* mask_strides, int B, int Hq, int Hkv,
+                                          int Sq, int Skv, int D);
 
 /* Scaled dot-product attention forward (prefill, any Sq):
  *   out[b,h,i,:] = softmax_j(scale * q[b,h,i,:] . k[b,h/g,j,:] + bias[b,h,i,j]) v[b,h/g,j,:]

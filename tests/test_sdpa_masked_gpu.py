@@ -1,0 +1,110 @@
+"""Masked SDPA calls on the grids of unmasked ones -- the q heads of a KV
+head packed into one block's rows, keys split over blocks, blocks of at most
+128 rows in half steps -- against torch's CPU SDPA in fp32 and the fp64
+logsumexp.
+
+Bars: out within 2e-3 + 1e-2 |ref| (tests/test_sdpa_gpu.py); LSE within 2e-3
+of fp64 (scores of fp16 products of a prescaled fp16 q).
+"""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import attention as OA
+from tests.conftest import SEED
+from tests.test_sdpa_gpu import LSE_ATOL, assert_close, randn
+
+pytestmark = pytest.mark.gpu
+
+
+def make_mask(kind, shape, B, Hq, Sq, Skv, seed):
+    """tail: query i sees keys up to Skv - Sq + i; pad: each sequence's own
+    number of keys; the other shapes: random, key 0 kept."""
+    g = torch.Generator().manual_seed(seed)
+    if shape == "tail":
+        keep = torch.ones((Sq, Skv), dtype=torch.bool).tril(Skv - Sq)
+    elif shape == "pad":
+        lens = torch.randint(1, Skv + 1, (B, 1, 1, 1), generator=g)
+        keep = torch.arange(Skv)[None, None, None, :] < lens
+    else:
+        dims = {"qk": (Sq, Skv), "bhqk": (B, Hq, Sq, Skv), "1h1k": (1, Hq, 1, Skv)}[shape]
+        keep = torch.rand(dims, generator=g) > 0.3
+        keep[..., 0] = True
+        if kind != "bool":
+            return (torch.randn(dims, generator=g) * 2).to(torch.float16).masked_fill(~keep, -float("inf"))
+    if kind == "bool":
+        return keep
+    low = torch.finfo(torch.float16).min if shape == "pad" else -float("inf")
+    return torch.zeros(keep.shape, dtype=torch.float16).masked_fill_(~keep, low)
+
+
+# Rows per block: 4 (decode), 60, 128 (a whole half-step block), 132 (just
+# past it: full steps), 512 (two packed blocks); keys: one step, a step and
+# one key, splits of 256 and of 512 with a ragged last one, copied masks
+# (odd rows) with a split's partials behind the copy.
+CASES = [(3, 8, 2, 1, 64, 128), (2, 32, 8, 1, 1000, 128), (1, 8, 8, 1, 2048, 64), (2, 8, 2, 15, 65, 64),
+         (1, 32, 8, 32, 1040, 128), (2, 16, 4, 33, 784, 128), (1, 32, 8, 128, 1536, 128), (1, 16, 16, 130, 640, 64),
+         (1, 8, 8, 300, 1100, 128)]
+
+
+@pytest.mark.parametrize("shape", ["tail", "pad", "bhqk", "1h1k"])
+@pytest.mark.parametrize("kind", ["bool", "f16"])
+@pytest.mark.parametrize("case", CASES, ids=str)
+def test_masked_grids(cuda, case, kind, shape):
+    import torch_spyre_amd as tsa
+
+    B, Hq, Hkv, Sq, Skv, D = case
+    q = randn((B, Hq, Sq, D), SEED + 300)
+    k, v = randn((B, Hkv, Skv, D), SEED + 301), randn((B, Hkv, Skv, D), SEED + 302)
+    mask = make_mask(kind, shape, B, Hq, Sq, Skv, SEED + 303 + Sq + Skv)
+    out, lse = tsa.scaled_dot_product_attention(q.to(cuda), k.to(cuda), v.to(cuda), attn_mask=mask.to(cuda),
+                                                enable_gqa=True, return_lse=True)
+    assert_close(out, OA.sdpa_cpu_fp32(q, k, v, attn_mask=mask))
+    _, lse64 = OA.sdpa_decomposition_fp64(q, k, v, attn_mask=mask.numpy(), return_lse=True)
+    assert np.allclose(lse.cpu().numpy(), lse64, atol=LSE_ATOL, rtol=0)
+
+
+@pytest.mark.parametrize("kind", ["bool", "f16"])
+@pytest.mark.parametrize("Sq,Skv", [(1, 2048), (40, 1536)])
+def test_masked_rows_and_splits(cuda, kind, Sq, Skv):
+    """Rows with every key masked give zeros and LSE -inf beside live rows of
+    the same block, and a split in which some rows see no key adds nothing to
+    them: head 0's rows keep only the last 7 keys, head 1's none."""
+    import torch_spyre_amd as tsa
+
+    B, Hq, Hkv, D = 2, 8, 2, 128
+    q = randn((B, Hq, Sq, D), SEED + 310)
+    k, v = randn((B, Hkv, Skv, D), SEED + 311), randn((B, Hkv, Skv, D), SEED + 312)
+    keep = torch.ones((1, Hq, Sq, Skv), dtype=torch.bool)
+    keep[:, 0, :, :-7] = False
+    keep[:, 1] = False
+    mask = keep if kind == "bool" else torch.zeros(keep.shape, dtype=torch.float16).masked_fill_(~keep, -float("inf"))
+    out, lse = tsa.scaled_dot_product_attention(q.to(cuda), k.to(cuda), v.to(cuda), attn_mask=mask.to(cuda),
+                                                enable_gqa=True, return_lse=True)
+    assert not out[:, 1].float().abs().sum() and bool(torch.isneginf(lse[:, 1]).all())
+    live = [h for h in range(Hq) if h != 1]
+    ref = OA.sdpa_cpu_fp32(q, k, v, attn_mask=mask)
+    assert_close(out[:, live], ref[:, live])
+    _, lse64 = OA.sdpa_decomposition_fp64(q, k, v, attn_mask=mask.numpy(), return_lse=True)
+    assert np.allclose(lse[:, live].cpu().numpy(), lse64[:, live], atol=LSE_ATOL, rtol=0)
+
+
+def test_masked_call_with_less_workspace(cuda):
+    """A masked call whose workspace holds no split's partials (staged mask:
+    16 bytes; copied mask: its copy alone) runs unsplit, within the bar."""
+    import torch_spyre_amd as tsa
+    from torch_spyre_amd import _lib
+
+    B, Hq, Hkv, Sq, D = 1, 8, 2, 16, 128
+    for Skv, room in ((1600, 16), (1603, Sq * 1616)):
+        q = randn((B, Hq, Sq, D), SEED + 320).to(cuda)
+        k, v = randn((B, Hkv, Skv, D), SEED + 321).to(cuda), randn((B, Hkv, Skv, D), SEED + 322).to(cuda)
+        mask = make_mask("bool", "tail", B, Hq, Sq, Skv, 0).to(cuda)
+        m = mask.view(torch.uint8).expand(B, Hq, Sq, Skv)
+        args = (m.data_ptr(), 3, _lib.i64_array(m.stride()), B, Hq, Hkv, Sq, Skv, D)
+        assert _lib.lib().spyre_sdpa_fwd_call_workspace_bytes(*args) > room
+        assert _lib.lib().spyre_sdpa_fwd_min_workspace_bytes(*args) <= room
+        out = tsa.scaled_dot_product_attention(q, k, v, attn_mask=mask, enable_gqa=True,
+                                               workspace=torch.empty(room, dtype=torch.uint8, device=cuda))
+        assert_close(out, OA.sdpa_cpu_fp32(q.cpu(), k.cpu(), v.cpu(), attn_mask=mask.cpu()))

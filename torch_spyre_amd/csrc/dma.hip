@@ -36,8 +36,7 @@
 // nothing is predicated.
 //
 // Index decomposition uses multiply-high division by loop-invariant divisors
-// (Granlund & Montgomery, "Division by Invariant Integers using
-// Multiplication", PLDI 1994, round-up variant), valid for 0 <= n, d < 2^31.
+// (fast_div.h).
 
 #include <hip/hip_runtime.h>
 
@@ -47,6 +46,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "fast_div.h"
 #include "spyre_common.h"
 #include "transpose8.h"
 
@@ -55,16 +55,9 @@ namespace {
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
-struct FastDiv {
-  uint32_t d, mul, shift;
-};
-
-FastDiv make_fastdiv(uint32_t d) {
-  uint32_t l = 0;
-  while ((uint64_t{1} << l) < d) ++l;
-  const uint64_t m = ((uint64_t{1} << 32) * ((uint64_t{1} << l) - d)) / d + 1;
-  return FastDiv{d, static_cast<uint32_t>(m), l};
-}
+using spyre_hip::FastDiv;
+using spyre_hip::fdiv;
+using spyre_hip::make_fastdiv;
 
 // Reads a kernel argument into scalar registers here and keeps it there.
 // Arguments are read from memory where they are used (the compiler may
@@ -75,10 +68,6 @@ template <typename T>
 __device__ __forceinline__ T pinned(T x) {
   asm volatile("" : "+s"(x));
   return x;
-}
-
-__device__ __forceinline__ uint32_t fdiv(uint32_t n, const FastDiv& f) {
-  return (__umulhi(n, f.mul) + n) >> f.shift;
 }
 
 constexpr int kMaxLoops = SPYRE_MAX_RANK;

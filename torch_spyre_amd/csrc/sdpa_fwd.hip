@@ -46,6 +46,7 @@
 #include <type_traits>
 
 #include "decode_dense.h"
+#include "fast_div.h"
 #include "spyre_common.h"
 #include "transpose8.h"
 
@@ -55,6 +56,7 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+using spyre_hip::fdiv;
 using spyre_hip::u32x4_t;
 
 constexpr int kWaves = 4;
@@ -396,18 +398,18 @@ struct Fwd2Args {
   const _Float16* v;
   const void* mask;          // fp16 bias or uint8 keep-mask, keys contiguous
   int64_t m_sb, m_sh, m_sq;  // elements
-  uint32_t m_bytes;          // extent of one (sequence, q head) of the mask
+  uint32_t m_bytes;          // extent of one block's `pack` q heads of the mask
   int64_t q_sb, q_sh, q_ss;
   int64_t k_sb, k_sh, k_ss;
   int64_t v_sb, v_sh, v_ss;
   _Float16* out;
   float* lse;
   int B, Hq, Hkv, g, Sq, Skv, causal, qblocks;
-  // Rows per query: 1, or (calls without a mask, Sq < 256) the g q heads of
-  // a KV head, which then share each K / V tile; gp = g / pack.
+  // Rows per query: 1, or (Sq < 256) the g q heads of a KV head, which then
+  // share each K / V tile; gp = g / pack.
   int pack, gp;
-  // Key split (calls without a mask or causal flag whose blocks would not
-  // fill the device): block sp attends keys sp * split_keys .. + split_keys
+  // Key split (calls without the causal flag whose blocks would not fill
+  // the device): block sp attends keys sp * split_keys .. + split_keys
   // - 1 and writes its fp32 partial (O, row max, row sum) to part; a merge
   // pass combines them.  nsplit == 1: no split.
   int nsplit, split_keys;
@@ -418,20 +420,24 @@ struct Fwd2Args {
   uint32_t n_items;
   int xcd_remap;
   float scale_log2;
+  // The divisors of the block index and of a row's (query, head), as
+  // multiply-high divisions: as integer divisions they cost ~30 instructions
+  // each before a block's first load.
+  spyre_hip::FastDiv by_split, by_gp, by_qblocks, by_hkv, by_pack;
 };
 
-// A wavefront's mask block for one step: its 32 queries x the step's 64 keys,
-// rows padded by 16 bytes, staged in LDS by buffer loads like the K / V
-// tiles (whole 1 KB loads; units past the block arrive as zeros in a spare
-// tail).
-template <int MK> struct MaskTile {
-  static constexpr int kRowU = 0, kDataU = 0, kLoads = 0, kBytes = 0, kEsz = 1;
+// A wavefront's mask block for one step: its 32 rows x the step's 64 keys
+// (HALF: the 32 keys of its half), rows padded by 16 bytes, staged in LDS by
+// buffer loads like the K / V tiles (whole 1 KB loads; units past the block
+// arrive as zeros in a spare tail).
+template <int ESZ, int KEYS> struct MaskRows {
+  static constexpr int kEsz = ESZ;
+  static constexpr int kDataU = KEYS * ESZ / 16, kRowU = kDataU + 1;  // 16-byte units of a row
+  static constexpr int kLoads = (32 * kRowU + 63) / 64, kBytes = kLoads * 1024;
 };
-template <> struct MaskTile<kMaskF16> {  // 128 + 16 bytes per row
-  static constexpr int kRowU = 9, kDataU = 8, kLoads = 5, kBytes = kLoads * 1024, kEsz = 2;
-};
-template <> struct MaskTile<kMaskBool> {  // 64 + 16 bytes per row
-  static constexpr int kRowU = 5, kDataU = 4, kLoads = 3, kBytes = kLoads * 1024, kEsz = 1;
+template <int MK, bool HALF> struct MaskTile : MaskRows<MK == kMaskF16 ? 2 : 1, HALF ? 32 : 64> {};
+template <bool HALF> struct MaskTile<kNoMask, HALF> {
+  static constexpr int kEsz = 1, kDataU = 0, kRowU = 1, kLoads = 0, kBytes = 0;
 };
 
 // PRESCALED (|scale log2 e| <= 1, so q * that never overflows fp16): Q is
@@ -443,15 +449,14 @@ template <> struct MaskTile<kMaskBool> {  // 64 + 16 bytes per row
 // ahead, a barrier per step.  Four (calls without a mask whose blocks have
 // fewer than 256 rows, e.g. decode, where one wavefront computes and the
 // step waits on its loads): loads two steps ahead, a barrier per two steps.
-// HALF (blocks of at most 128 rows without a mask, e.g. decode): wavefronts
-// 2r and 2r + 1 share row tile r and take one 32-key half of every step
-// each; the pair's partials are folded in LDS at the end.
+// HALF (blocks of at most 128 rows, e.g. decode): wavefronts 2r and 2r + 1
+// share row tile r and take one 32-key half of every step each; the pair's
+// partials are folded in LDS at the end.
 template <int D, bool PRESCALED, int MK, int SLOTS = 2, bool HALF = false>
 __global__ __launch_bounds__(kThreads2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   static_assert(SLOTS == 2 || (SLOTS == 4 && MK == kNoMask), "four slots leave no room for a mask");
-  static_assert(!HALF || MK == kNoMask, "half steps serve calls without a mask");
   using L = Lds2<D>;
-  using MT = MaskTile<MK>;
+  using MT = MaskTile<MK, HALF>;
   constexpr int DK = D / 16;  // QK k-steps
   constexpr int DM = D / 32;  // O row tiles
   // Two K / V slots, then (masked calls) two mask blocks per wavefront.
@@ -464,29 +469,28 @@ __global__ __launch_bounds__(kThreads2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   // row = query * pack + head in group.
   uint32_t item = blockIdx.x;
   if (a.xcd_remap) item = (item % 8) * (a.n_items / 8) + item / 8;
-  const int pack = MK == kNoMask ? a.pack : 1;
-  const int sp = MK == kNoMask ? static_cast<int>(item % a.nsplit) : 0;
-  if (MK == kNoMask) item /= a.nsplit;
-  const int gi = static_cast<int>(item % a.gp);
-  uint32_t r = item / a.gp;
-  const int qb = a.qblocks - 1 - static_cast<int>(r % a.qblocks);
-  r /= a.qblocks;
-  const int kvh = static_cast<int>(r % a.Hkv);
-  const int b = static_cast<int>(r / a.Hkv);
+  const int pack = a.pack;
+  const uint32_t i1 = fdiv(item, a.by_split), i2 = fdiv(i1, a.by_gp), i3 = fdiv(i2, a.by_qblocks);
+  const uint32_t bq = fdiv(i3, a.by_hkv);
+  const int sp = static_cast<int>(item - i1 * a.nsplit);
+  const int gi = static_cast<int>(i1 - i2 * a.gp);
+  const int qb = a.qblocks - 1 - static_cast<int>(i2 - i3 * a.qblocks);
+  const int kvh = static_cast<int>(i3 - bq * a.Hkv);
+  const int b = static_cast<int>(bq);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
   __builtin_assume(wave >= 0 && wave < kWaves2);  // lets the compiler drop always-true load guards
   const int hw = HALF ? (wave & 1) : 0;  // HALF: the key half of each step
   const int qw0 = qb * kQB, q0 = qw0 + (HALF ? (wave >> 1) : wave) * kQW;  // rows
   const int col = lane & 31, half = lane >> 5;
   const int qrow = q0 + col;
-  const int qi = pack == 1 ? qrow : qrow / pack;  // this lane's query
+  const int qi = static_cast<int>(fdiv(qrow, a.by_pack));  // this lane's query
   // Block gi of the KV head holds q heads gi * pack .. gi * pack + pack - 1.
   const int h = kvh * a.g + gi * pack + (qrow - qi * pack);
   const bool q_ok = qi < a.Sq;
   // The wavefront's first and last query, and the block's last.
-  const int q_lo = pack == 1 ? q0 : q0 / pack;
-  const int q_hi = pack == 1 ? q0 + kQW - 1 : (q0 + kQW - 1) / pack;
-  const int qb_hi = pack == 1 ? qw0 + kQB - 1 : (qw0 + kQB - 1) / pack;
+  const int q_lo = static_cast<int>(fdiv(q0, a.by_pack));
+  const int q_hi = static_cast<int>(fdiv(q0 + kQW - 1, a.by_pack));
+  const int qb_hi = static_cast<int>(fdiv(qw0 + kQB - 1, a.by_pack));
 
   // Q^T operand: lane (query column, half) holds features 16ks + 8half .. +8.
   f16x8 qv[DK];
@@ -575,29 +579,33 @@ __global__ __launch_bounds__(kThreads2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
     v_cur += v_tile;
     v_left -= v_step;
   };
-  // The wavefront's mask block of keys kb .. kb + 63 into its slot `slot`:
-  // rows past Sq and bytes past the (sequence, head) slice arrive as zeros.
-  // Offsets are from the wavefront's first query row; the descriptor's range
-  // ends with the (sequence, head) slice.
+  // The wavefront's mask block of keys kb .. kb + 63 (HALF: its 32 of them)
+  // into its slot `slot`: rows past Sq and bytes past the block's heads
+  // arrive as zeros.  Offsets are from the first of the block's `pack` q
+  // heads (a row is a (query, head) pair); the descriptor's range ends with
+  // the last of them.
   uint32_t m_off[MT::kLoads > 0 ? MT::kLoads : 1];
   const char* mbase = nullptr;
-  uint32_t m_left = 0;  // bytes of the slice from row q0, key 0
   if constexpr (MK != kNoMask) {
-    const int64_t row0 = static_cast<int64_t>(min(q0, a.Sq - 1)) * a.m_sq * MT::kEsz;
-    mbase = static_cast<const char*>(a.mask) + (b * a.m_sb + h * a.m_sh) * MT::kEsz + row0;
-    m_left = a.m_bytes - static_cast<uint32_t>(row0);
+    mbase = static_cast<const char*>(a.mask) + (b * a.m_sb + (kvh * a.g + gi * pack) * a.m_sh) * MT::kEsz;
 #pragma unroll
     for (int j = 0; j < MT::kLoads; ++j) {
       const int u = 64 * j + lane, row = u / MT::kRowU, ch = u % MT::kRowU;
-      const bool ok = row < kQW && ch < MT::kDataU && q0 + row < a.Sq;
-      m_off[j] = ok ? static_cast<uint32_t>((row * a.m_sq) * MT::kEsz + 16 * ch) : kOob;
+      // a valid row's offset lies below m_bytes < 2^31, so 32 bits of each product do
+      uint32_t mq = q0 + row, at = mq * static_cast<uint32_t>(a.m_sq);
+      if (pack > 1) {
+        mq = fdiv(q0 + row, a.by_pack);
+        at = mq * static_cast<uint32_t>(a.m_sq) + (q0 + row - mq * pack) * static_cast<uint32_t>(a.m_sh);
+      }
+      const bool ok = row < kQW && ch < MT::kDataU && static_cast<int>(mq) < a.Sq;
+      m_off[j] = ok ? (at + 32 * hw) * MT::kEsz + 16 * ch : kOob;
     }
   }
   auto mask_block = [&](int slot) { return lds + SLOTS * L::kSlot + (slot * kWaves2 + wave) * (MT::kBytes / 2); };
   auto dma_m = [&](int kb, int slot) {
     if constexpr (MK != kNoMask) {
-      const uint32_t done = static_cast<uint32_t>(kb) * MT::kEsz;  // < Skv esz <= m_left
-      const Rsrc r = make_rsrc(reinterpret_cast<const _Float16*>(mbase + done), m_left - done);
+      const uint32_t done = static_cast<uint32_t>(kb) * MT::kEsz;  // < Skv esz <= m_bytes
+      const Rsrc r = make_rsrc(reinterpret_cast<const _Float16*>(mbase + done), a.m_bytes - done);
 #pragma unroll
       for (int j = 0; j < MT::kLoads; ++j) load_lds16(r, mask_block(slot) + 512 * j, m_off[j]);
     }
@@ -657,26 +665,28 @@ __global__ __launch_bounds__(kThreads2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   // units (PRESCALED: log2 units, else divided by |scale|), a keep-mask
   // sends dropped scores to -inf.
   const float bias_mul = PRESCALED ? kLog2e : kLog2e / scale_abs;
-  auto apply_mask = [&](int t, f32x16 (&s)[2]) {
+  // Half mt of the mask block (HALF: its one half, mt 0) onto S half s.
+  auto apply_mask_half = [&](int t, int mt, f32x16& s) {
     if constexpr (MK != kNoMask) {
       const char* row = reinterpret_cast<const char*>(mask_block(t & 1)) + col * (16 * MT::kRowU);
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt)
+      for (int i = 0; i < 4; ++i) {
+        const int k4 = 32 * mt + 16 * (i >> 1) + 8 * half + 4 * (i & 1);
+        if constexpr (MK == kMaskF16) {
+          const f16x4 m4 = *reinterpret_cast<const f16x4*>(row + 2 * k4);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int k4 = 32 * mt + 16 * (i >> 1) + 8 * half + 4 * (i & 1);
-          if constexpr (MK == kMaskF16) {
-            const f16x4 m4 = *reinterpret_cast<const f16x4*>(row + 2 * k4);
+          for (int v = 0; v < 4; ++v) s[4 * i + v] = __builtin_fmaf(static_cast<float>(m4[v]), bias_mul, s[4 * i + v]);
+        } else {
+          const uint32_t m4 = *reinterpret_cast<const uint32_t*>(row + k4);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) s[mt][4 * i + v] = __builtin_fmaf(static_cast<float>(m4[v]), bias_mul, s[mt][4 * i + v]);
-          } else {
-            const uint32_t m4 = *reinterpret_cast<const uint32_t*>(row + k4);
-#pragma unroll
-            for (int v = 0; v < 4; ++v)
-              s[mt][4 * i + v] = ((m4 >> (8 * v)) & 0xffu) != 0 ? s[mt][4 * i + v] : -INFINITY;
-          }
+          for (int v = 0; v < 4; ++v) s[4 * i + v] = ((m4 >> (8 * v)) & 0xffu) != 0 ? s[4 * i + v] : -INFINITY;
         }
+      }
     }
+  };
+  auto apply_mask = [&](int t, f32x16 (&s)[2]) {
+    apply_mask_half(t, 0, s[0]);
+    apply_mask_half(t, 1, s[1]);
   };
   // The running max (log2 domain) moves only when a score of the step
   // exceeds it by more than 2^8, so P <= 256 (fine in fp16) and most steps
@@ -862,6 +872,7 @@ __global__ __launch_bounds__(kThreads2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
     if constexpr (SLOTS == 2) {
       if (t + 2 < n_tiles) dma_k(t & 1);
       if (t + 1 < n_tiles) dma_v((t + 1) & 1);
+      if (t + 1 < n_tiles) dma_m(kb0 + (t + 1) * kKT, (t + 1) & 1);
     } else if ((t & 1) == 0) {
       if (t + 3 < n_tiles) dma_k((t + 3) % 4);
       if (t + 4 < n_tiles) dma_k(t % 4);
@@ -878,6 +889,7 @@ __global__ __launch_bounds__(kThreads2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
         acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[i], b, acc, 0, 0, 0);
         if (i + kPrefetch < kNFH) fr[i + kPrefetch] = frag_h(k1, i + kPrefetch);
       };
+      if constexpr (MK != kNoMask) apply_mask_half(t, 0, cur);
       if (edge(t)) {  // the key test on this half
         const int kl = key_last - (kb0 + t * kKT) - 32 * hw - 8 * half;
 #pragma unroll
@@ -892,7 +904,9 @@ __global__ __launch_bounds__(kThreads2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
 #pragma unroll
       for (int rr = 0; rr < 16; ++rr) mx = fmaxf(mx, cur[rr]);
       mx = PRESCALED ? max_xor32(mx) + m_use : max_xor32(mx) * scale_abs;
-      if (__builtin_amdgcn_ballot_w64(mx > m_run + 8.f) != 0) {
+      // A step the mask blanks for every real row adds nothing (see step).
+      const bool live = MK == kNoMask || __builtin_amdgcn_ballot_w64(q_ok && mx > -INFINITY && mx >= m_run - 32.f) != 0;
+      if (live && __builtin_amdgcn_ballot_w64(mx > m_run + 8.f) != 0) {
         const float m_new = fmaxf(m_run, mx);
         const float alpha = m_new == -INFINITY ? 1.f : fast_exp2(m_run - m_new);
         l_run *= alpha;
@@ -911,16 +925,18 @@ __global__ __launch_bounds__(kThreads2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
           }
         }
       }
-      const float neg_m = m_run == -INFINITY ? 0.f : -m_run;
-      f16x8 p[2];
-      softmax_half(cur, neg_m, p);
-      __builtin_amdgcn_sched_barrier(0);
+      if (live) {
+        const float neg_m = m_run == -INFINITY ? 0.f : -m_run;
+        f16x8 p[2];
+        softmax_half(cur, neg_m, p);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int dm = 0; dm < DM; ++dm) mfma(DK + j * DM + dm, p[j], o[dm]);
-      interleave_h(DK, kNFH);
-      __builtin_amdgcn_sched_barrier(0);
+          for (int dm = 0; dm < DM; ++dm) mfma(DK + j * DM + dm, p[j], o[dm]);
+        interleave_h(DK, kNFH);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
     if (SLOTS == 2 || (t & 1)) {
       dma_wait();
@@ -1021,13 +1037,13 @@ __global__ __launch_bounds__(kThreads2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
       } else {
 
         // A mask can leave a step nothing to add: every score of the
-        // wavefront's block -inf or more than 32 below its row's running
+        // wavefront's real rows -inf or more than 32 below its row's running
         // max, so every P rounds to 0 in fp16.  Such a step computes only
         // S(t+1); S(t+1) is therefore computed whole before the softmax.
         apply_mask(t, cur);
         if (edge(t)) mask_step(t, cur);
         const float mx = row_max(cur);
-        const bool live = __builtin_amdgcn_ballot_w64(mx > -INFINITY && mx >= m_run - 32.f) != 0;
+        const bool live = __builtin_amdgcn_ballot_w64(q_ok && mx > -INFINITY && mx >= m_run - 32.f) != 0;
         nxt[0] = PRESCALED ? neg_m_tile : f32x16{};
         nxt[1] = PRESCALED ? neg_m_tile : f32x16{};
 #pragma unroll
@@ -1128,7 +1144,7 @@ __global__ __launch_bounds__(kThreads2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
 
   const float l = sum_xor32(l_run);
   if (!q_ok) return;
-  if (MK == kNoMask && a.nsplit > 1) {
+  if (a.nsplit > 1) {
     // The partial: O unnormalised (relative to m_run), then m_run and l.
     const int64_t prow = ((static_cast<int64_t>(b) * a.Hq + h) * a.Sq + qi) * a.nsplit + sp;
     float* po = a.part + prow * D;
@@ -1201,17 +1217,17 @@ __global__ __launch_bounds__(W * 64) void sdpa_decode_short_kernel(Fwd2Args a) {
   // item = ((b * Hkv + kvh) * gp + gi) * nsplit + sp (one query block).
   uint32_t item = blockIdx.x;
   if (a.xcd_remap) item = (item % 8) * (a.n_items / 8) + item / 8;
-  const int sp = static_cast<int>(item % a.nsplit);
-  item /= a.nsplit;
-  const int gi = static_cast<int>(item % a.gp);
-  const uint32_t r = item / a.gp;
-  const int kvh = static_cast<int>(r % a.Hkv);
-  const int b = static_cast<int>(r / a.Hkv);
+  const uint32_t i1 = fdiv(item, a.by_split), i2 = fdiv(i1, a.by_gp), bq = fdiv(i2, a.by_hkv);
+  const int sp = static_cast<int>(item - i1 * a.nsplit);
+  item = i1;
+  const int gi = static_cast<int>(i1 - i2 * a.gp);
+  const int kvh = static_cast<int>(i2 - bq * a.Hkv);
+  const int b = static_cast<int>(bq);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
   __builtin_assume(wave >= 0 && wave < W);
   const int col = lane & 31, half = lane >> 5;
   const int pack = a.pack;
-  const int qi = col / pack;  // this lane's row: query qi, q head h
+  const int qi = static_cast<int>(fdiv(col, a.by_pack));  // this lane's row: query qi, q head h
   const int h = kvh * a.g + gi * pack + (col - qi * pack);
   const bool q_ok = qi < a.Sq;
 
@@ -1383,7 +1399,7 @@ __global__ __launch_bounds__(W * 64) void sdpa_decode_short_kernel(Fwd2Args a) {
       lsum += (mlw[w][1] + l1[w]) * wt;
       acc += val[w] * wt;
     }
-    const int jq = j / pack, jh = kvh * a.g + gi * pack + (j - jq * pack);
+    const int jq = static_cast<int>(fdiv(j, a.by_pack)), jh = kvh * a.g + gi * pack + (j - jq * pack);
     const int64_t r = (static_cast<int64_t>(b) * a.Hq + jh) * a.Sq + jq;
     if (a.nsplit == 1) {
       const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
@@ -1435,7 +1451,7 @@ __global__ __launch_bounds__(W * 64) void sdpa_decode_short_kernel(Fwd2Args a) {
   const int d4 = static_cast<int>(threadIdx.x) % D4;
   const uint32_t last = static_cast<uint32_t>(a.nsplit - 1);
   for (int j = static_cast<int>(threadIdx.x) / D4; j < nv; j += RP) {
-    const int jq = j / pack, jh = kvh * a.g + gi * pack + (j - jq * pack);
+    const int jq = static_cast<int>(fdiv(j, a.by_pack)), jh = kvh * a.g + gi * pack + (j - jq * pack);
     const int64_t r = (static_cast<int64_t>(b) * a.Hq + jh) * a.Sq + jq;
     const uint32_t r0 = static_cast<uint32_t>(r * a.nsplit);
     float Mr = -INFINITY, Lr = 0.f;
@@ -1627,7 +1643,7 @@ __global__ __launch_bounds__(256) void sdpa_split_merge_rows_kernel(MergeArgs a)
 
 int device_cus();
 
-// Key split of a call without a mask or causal flag: splits enough that the
+// Key split of a call without the causal flag: splits enough that the
 // grid gives every compute unit a block, each split at least 8 steps (512
 // keys; shorter splits lose more to the merge pass than they gain) -- or,
 // when the unsplit grid would use at most an eighth of the compute units,
@@ -1658,11 +1674,16 @@ int64_t blocks_for(int B, int Hkv, int g, int Sq, int pack) {
   return static_cast<int64_t>(B) * Hkv * (g / pack) * ((static_cast<int64_t>(pack) * Sq + kQB - 1) / kQB);
 }
 
-// The grid of a call without a mask: short query runs pack all g q heads of
-// a KV head into one block's rows and split the keys until the grid fills
-// the device, if the workspace (ws_bytes) holds the split's partials;
-// otherwise the heads are packed only as far as the unsplit grid still
-// fills the device (pack_heads).
+// The grid of a call: short query runs pack all g q heads of a KV head into
+// one block's rows and split the keys until the grid fills the device, if
+// the workspace (ws_bytes) holds the split's partials; otherwise the heads
+// are packed only as far as the unsplit grid still fills the device
+// (pack_heads).  Masked calls take the same grid, less the short-decode
+// kernel; one block per q head and 256 queries, unsplit, left most units or
+// wavefronts idle for short query runs: 128 queries x 4096 keys with the
+// chunk's causal boolean mask (B 4, 32 / 8 heads) 94.0 us, packed and split
+// 54.3; one query x 2048 keys with a padding mask (B 16) 98.6 and 33.6; 512
+// queries x 512 keys (B 2) the same grid and time.
 struct GridPlan {
   int pack = 1, nsplit = 1, split_keys = 0;
   size_t part_bytes = 0;
@@ -1670,14 +1691,18 @@ struct GridPlan {
   int waves = kWaves2;         // its wavefronts per block
 };
 
-GridPlan plan_grid(int B, int Hq, int Hkv, int Sq, int Skv, int D, bool causal, size_t ws_bytes) {
+// masked: a staged or copied mask, can_pack: its rows of a KV head's q heads
+// fit one buffer descriptor (else heads stay apart).
+GridPlan plan_grid(int B, int Hq, int Hkv, int Sq, int Skv, int D, bool causal, size_t ws_bytes,
+                   bool masked = false, bool can_pack = true) {
   GridPlan gp;
-  const int g = Hq / Hkv;
+  const int g = can_pack ? Hq / Hkv : 1;
+  const int Hb = Hq / g;  // the (KV head, pack group) pairs of a sequence
   gp.split_keys = Skv;
   // Short decode: one row tile (the g q heads of a KV head times Sq <= 32
   // rows) whose keys fit one block (kWaves2 slices), or a split of them
   // over blocks that all run in one round of the device.
-  if (!causal && Sq > 0 && static_cast<int64_t>(g) * Sq <= 32) {
+  if (!causal && !masked && Sq > 0 && static_cast<int64_t>(g) * Sq <= 32) {
     const int kw = D == 64 ? ShortLds<64>::kKW : ShortLds<128>::kKW;
     const int64_t cus = device_cus() > 0 ? device_cus() : 256;
     int waves = kWaves2;
@@ -1706,7 +1731,7 @@ GridPlan plan_grid(int B, int Hq, int Hkv, int Sq, int Skv, int D, bool causal, 
   if (!causal && Sq > 0) {
     const int p0 = Sq < kQB ? g : 1;
     int keys = Skv;
-    const int ns = plan_split(blocks_for(B, Hkv, g, Sq, p0), Skv, &keys);
+    const int ns = plan_split(blocks_for(B, Hb, g, Sq, p0), Skv, &keys);
     const size_t pb = split_bytes(static_cast<int64_t>(B) * Hq * Sq, ns, D);
     if (ns > 1 && ws_bytes >= pb) {
       gp.pack = p0;
@@ -1716,7 +1741,7 @@ GridPlan plan_grid(int B, int Hq, int Hkv, int Sq, int Skv, int D, bool causal, 
       return gp;
     }
   }
-  gp.pack = pack_heads(B, Hkv, g, Sq);
+  gp.pack = pack_heads(B, Hb, g, Sq);
   return gp;
 }
 
@@ -1751,7 +1776,7 @@ void launch_short(const Fwd2Args& f2, int D, bool prescaled, int waves, hipStrea
     launch_short_w<kWaves2>(f2, D, prescaled, st);
 }
 
-template <int MK, int SLOTS = 2, bool HALF = false>
+template <int MK, int SLOTS, bool HALF = false>
 void launch_lds(const Fwd2Args& f2, int D, bool prescaled, hipStream_t st) {
   const dim3 grid(f2.n_items);
   if (D == 128 && prescaled)
@@ -1820,6 +1845,8 @@ enum MaskRoute { kRouteNone, kRouteStaged, kRouteCopied, kRouteVt };
 
 struct MaskPlan {
   MaskRoute route = kRouteNone;
+  int64_t esz = 1;
+  int64_t sb = 0, sh = 0, sq = 0;        // strides as staged, elements
   int64_t span = 0;                      // bytes of one (sequence, head) slice as staged
   int64_t bm = 1, hm = 1, qm = 1, pitch = 0;  // kRouteCopied: extents kept, row pitch (bytes)
   size_t copy_bytes = 0;
@@ -1832,7 +1859,7 @@ MaskPlan plan_mask(const void* mask, int kind, const int64_t* ms, int B, int Hq,
     p.route = kRouteVt;
     return p;
   }
-  const int64_t esz = kind == kMaskF16 ? 2 : 1;
+  const int64_t esz = p.esz = kind == kMaskF16 ? 2 : 1;
   if (Sq == 0 || Skv == 0) {  // nothing of the mask is read
     p.route = kRouteStaged;
     return p;
@@ -1845,6 +1872,9 @@ MaskPlan plan_mask(const void* mask, int kind, const int64_t* ms, int B, int Hq,
       (ms[2] * esz) % 16 == 0 && (Skv * esz) % 16 == 0 && span <= kBufRange) {
     p.route = kRouteStaged;
     p.span = span;
+    p.sb = ms[0];
+    p.sh = ms[1];
+    p.sq = ms[2];
     return p;
   }
   p.bm = ms[0] != 0 ? B : 1;
@@ -1858,7 +1888,25 @@ MaskPlan plan_mask(const void* mask, int kind, const int64_t* ms, int B, int Hq,
   }
   p.route = kRouteCopied;
   p.copy_bytes = static_cast<size_t>(p.bm * p.hm * p.qm * p.pitch);
+  const int64_t pe = p.pitch / esz;  // row pitch, elements
+  p.sq = p.qm > 1 ? pe : 0;
+  p.sh = p.hm > 1 ? p.qm * pe : 0;
+  p.sb = p.bm > 1 ? p.hm * p.qm * pe : 0;
   return p;
+}
+
+// Bytes of a mask's rows of `pack` consecutive q heads as staged.
+int64_t mask_extent(const MaskPlan& mp, int pack) { return mp.span + (pack - 1) * mp.sh * mp.esz; }
+
+// The workspace of a copied mask: the copy, then (256-byte aligned) a key
+// split's partials.
+size_t copy_room(const MaskPlan& mp) {
+  return mp.route == kRouteCopied ? (mp.copy_bytes + 255) / 256 * 256 : 0;
+}
+
+// The grid of a staged or copied mask's call given ws_bytes beyond the copy.
+GridPlan masked_grid(const MaskPlan& mp, int B, int Hq, int Hkv, int Sq, int Skv, int D, size_t ws_bytes) {
+  return plan_grid(B, Hq, Hkv, Sq, Skv, D, false, ws_bytes, true, mask_extent(mp, Hq / Hkv) <= kBufRange);
 }
 
 // Compute units of the current device, cached per device; 0 if the runtime
@@ -1910,8 +1958,20 @@ extern "C" size_t spyre_sdpa_fwd_call_workspace_bytes(const void* attn_mask, int
   }
   if (!mask_strides || mask_kind < kNoMask || mask_kind > kMaskBool) return 0;
   const MaskPlan mp = plan_mask(attn_mask, mask_kind, mask_strides, B, Hq, Sq, Skv);
-  if (mp.route == kRouteCopied) return mp.copy_bytes;
-  return mp.route == kRouteVt ? spyre_sdpa_fwd_workspace_bytes(B, Hkv, Skv, D) : 0;
+  if (mp.route == kRouteVt) return spyre_sdpa_fwd_workspace_bytes(B, Hkv, Skv, D);
+  const size_t part = masked_grid(mp, B, Hq, Hkv, Sq, Skv, D, SIZE_MAX).part_bytes;
+  return part ? copy_room(mp) + part : mp.copy_bytes;
+}
+
+extern "C" size_t spyre_sdpa_fwd_min_workspace_bytes(const void* attn_mask, int mask_kind,
+                                                     const int64_t* mask_strides, int B, int Hq, int Hkv,
+                                                     int Sq, int Skv, int D) {
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || Sq < 0 || Skv < 0 || (D != 64 && D != 128)) return 0;
+  if (!mask_strides || mask_kind <= kNoMask || mask_kind > kMaskBool) return 0;
+  const MaskPlan mp = plan_mask(attn_mask, mask_kind, mask_strides, B, Hq, Sq, Skv);
+  if (mp.route == kRouteStaged) return 0;
+  const size_t vt = spyre_sdpa_fwd_workspace_bytes(B, Hkv, Skv, D);
+  return mp.route == kRouteCopied ? std::min(mp.copy_bytes, vt) : vt;
 }
 
 extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const void* k,
@@ -1965,12 +2025,6 @@ extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int s64 = static_cast<int>(s64_of(Skv));
   const void* mask_ptr = attn_mask;
-  int64_t m_sb = 0, m_sh = 0, m_sq = 0;
-  if (mask_kind != kNoMask) {
-    m_sb = mask_strides[0];
-    m_sh = mask_strides[1];
-    m_sq = mask_strides[2];
-  }
   if (mp.route == kRouteCopied) {
     const int esz = mask_kind == kMaskF16 ? 2 : 1;
     MaskPadArgs pa{static_cast<const char*>(attn_mask), static_cast<char*>(workspace), mask_strides[0],
@@ -1982,11 +2036,7 @@ extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const
     mask_pad_kernel<<<dim3(static_cast<unsigned>(blocks)), 256, 0, st>>>(pa);
     const hipError_t e = hipGetLastError();
     SPYRE_REQUIRE(e == hipSuccess, SPYRE_EHIP, "mask copy launch failed: %s", hipGetErrorString(e));
-    const int64_t pe = mp.pitch / esz;  // row pitch, elements
     mask_ptr = workspace;
-    m_sq = mp.qm > 1 ? pe : 0;
-    m_sh = mp.hm > 1 ? mp.qm * pe : 0;
-    m_sb = mp.bm > 1 ? mp.hm * mp.qm * pe : 0;
   }
   if (Skv > 0 && !lds_path) {
     VtArgs va{static_cast<const _Float16*>(v), v_strides[0], v_strides[1], v_strides[2],
@@ -2067,47 +2117,56 @@ extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const
     f2.Sq = Sq;
     f2.Skv = Skv;
     f2.causal = fa.causal;
-    // Without a mask, short query runs pack q heads of a KV head into one
-    // block's rows, so they share each K / V tile (decode: one block per
-    // (sequence, KV head) instead of g mostly idle ones).
+    // Short query runs pack q heads of a KV head into one block's rows, so
+    // they share each K / V tile (decode: one block per (sequence, KV head)
+    // instead of g mostly idle ones).
     // And (plan_grid) a key split when the blocks would not fill the device
-    // and the workspace holds its partials.
-    GridPlan gpl;
-    if (mask_kind == kNoMask)
-      gpl = plan_grid(B, Hq, Hkv, Sq, Skv, D, is_causal != 0, workspace && aligned16(workspace) ? workspace_bytes : 0);
+    // and the workspace holds its partials (after a mask's copy).
+    const size_t ws_room = workspace && aligned16(workspace) ? workspace_bytes : 0;
+    const size_t part_at = copy_room(mp);
+    const size_t part_room = ws_room > part_at ? ws_room - part_at : 0;
+    const GridPlan gpl = mask_kind == kNoMask ? plan_grid(B, Hq, Hkv, Sq, Skv, D, is_causal != 0, part_room)
+                                              : masked_grid(mp, B, Hq, Hkv, Sq, Skv, D, part_room);
     f2.pack = gpl.pack;
     f2.gp = fa.g / f2.pack;
     f2.qblocks = static_cast<int>((static_cast<int64_t>(f2.pack) * Sq + kQB - 1) / kQB);
     f2.nsplit = gpl.nsplit;
     f2.split_keys = gpl.nsplit > 1 ? gpl.split_keys : Skv;
-    f2.part = gpl.nsplit > 1 ? static_cast<float*>(workspace) : nullptr;
+    f2.part = gpl.nsplit > 1 ? reinterpret_cast<float*>(static_cast<char*>(workspace) + part_at) : nullptr;
     const int64_t items = blocks_for(B, Hkv, fa.g, Sq, f2.pack) * f2.nsplit;
     SPYRE_REQUIRE(items < (int64_t{1} << 31), SPYRE_EUNSUPPORTED, "too many query blocks");
     f2.n_items = static_cast<uint32_t>(items);
+    f2.by_split = spyre_hip::make_fastdiv(static_cast<uint32_t>(f2.nsplit));
+    f2.by_gp = spyre_hip::make_fastdiv(static_cast<uint32_t>(f2.gp));
+    f2.by_qblocks = spyre_hip::make_fastdiv(static_cast<uint32_t>(f2.qblocks));
+    f2.by_hkv = spyre_hip::make_fastdiv(static_cast<uint32_t>(Hkv));
+    f2.by_pack = spyre_hip::make_fastdiv(static_cast<uint32_t>(f2.pack));
     f2.xcd_remap = items % 8 == 0;
     f2.scale_log2 = fa.scale_log2;
     // |scale log2 e| <= 1: q times it stays within fp16, so Q is prescaled.
     const bool prescaled = fabsf(f2.scale_log2) <= 1.f;
     f2.mask = mask_ptr;
-    f2.m_sb = m_sb;
-    f2.m_sh = m_sh;
-    f2.m_sq = m_sq;
-    f2.m_bytes = static_cast<uint32_t>(mp.span);
+    f2.m_sb = mp.sb;
+    f2.m_sh = mp.sh;
+    f2.m_sq = mp.sq;
+    f2.m_bytes = static_cast<uint32_t>(mask_extent(mp, f2.pack));
+    // Blocks of at most 128 rows: half steps (two wavefronts per row tile).
+    const bool half = static_cast<int64_t>(f2.pack) * Sq <= kQB / 2;
     if (gpl.short_decode) {
       // One row tile, its keys all in flight at once; a key split merges in
       // the same kernel.
       f2.ticket = spyre_hip::next_call_ticket();
       launch_short(f2, D, prescaled, gpl.waves, st);
     } else if (mask_kind == kMaskF16) {
-      launch_lds<kMaskF16>(f2, D, prescaled, st);
+      half ? launch_lds<kMaskF16, 2, true>(f2, D, prescaled, st) : launch_lds<kMaskF16, 2>(f2, D, prescaled, st);
     } else if (mask_kind == kMaskBool) {
-      launch_lds<kMaskBool>(f2, D, prescaled, st);
-    } else if (static_cast<int64_t>(f2.pack) * Sq <= kQB / 2) {
-      launch_lds<kNoMask, 4, true>(f2, D, prescaled, st);  // half steps: two wavefronts per row tile
+      half ? launch_lds<kMaskBool, 2, true>(f2, D, prescaled, st) : launch_lds<kMaskBool, 2>(f2, D, prescaled, st);
+    } else if (half) {
+      launch_lds<kNoMask, 4, true>(f2, D, prescaled, st);
     } else if (static_cast<int64_t>(f2.pack) * Sq < kQB) {
       launch_lds<kNoMask, 4>(f2, D, prescaled, st);  // blocks with fewer rows than wavefronts can fill
     } else {
-      launch_lds<kNoMask>(f2, D, prescaled, st);
+      launch_lds<kNoMask, 2>(f2, D, prescaled, st);
     }
     if (f2.nsplit > 1 && !gpl.short_decode) {
       const hipError_t e0 = hipGetLastError();

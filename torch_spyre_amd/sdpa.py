@@ -89,10 +89,10 @@ def _geometry_plan(q, k, v, mask, kind: int, is_causal: bool):
     B, Hq, Sq, D = q.shape
     _, Hkv, Skv, _ = k.shape
     mstrides = _lib.i64_array(mask.stride()) if mask is not None else None
-    # The call's workspace: without a mask, a key split's partials when the
-    # blocks would not fill the device (none for causal calls); none for
-    # masks the kernel stages as they lie, a copy with 16-byte rows for other
-    # fp16 / bool masks, V's relayout for fp32 masks.
+    # The call's workspace: a key split's partials when the blocks would not
+    # fill the device (none for causal calls), a copy with 16-byte rows of
+    # fp16 / bool masks the kernel cannot stage as they lie, V's relayout for
+    # fp32 masks.
     need = 0
     if kind != MASK_NONE or not is_causal:
         need = int(_lib.lib().spyre_sdpa_fwd_call_workspace_bytes(
@@ -144,8 +144,9 @@ def _prepare(query, key, value, attn_mask, dropout_p, is_causal, scale, enable_g
     if workspace is None and need:
         workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
     elif workspace is not None and need and kind != MASK_NONE:
-        # a workspace that holds V's relayout also serves (the fp32-mask kernel runs)
-        floor = min(need, workspace_bytes(B, Hkv, Skv, D))
+        # less than the call asks for also serves (no key split; V's relayout instead of the mask's copy)
+        floor = int(_lib.lib().spyre_sdpa_fwd_min_workspace_bytes(mask.data_ptr(), kind, mstrides, B, Hq, Hkv, Sq,
+                                                                  Skv, D))
         if workspace.numel() * workspace.element_size() < floor:
             raise ValueError(f"workspace holds {workspace.numel() * workspace.element_size()} bytes, need {floor}")
     ws_ptr = workspace.data_ptr() if workspace is not None else None
