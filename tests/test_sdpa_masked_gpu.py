@@ -1,6 +1,7 @@
 """Masked SDPA calls on the grids of unmasked ones -- the q heads of a KV
 head packed into one block's rows, keys split over blocks, blocks of at most
-128 rows in half steps -- against torch's CPU SDPA in fp32 and the fp64
+128 rows in half steps -- and the workgroup shapes of the SDPA forward kernel
+(64, 128 or 256 rows), against torch's CPU SDPA in fp32 and the fp64
 logsumexp.
 
 Bars: out within 2e-3 + 1e-2 |ref| (tests/test_sdpa_gpu.py); LSE within 2e-3
@@ -108,3 +109,37 @@ def test_masked_call_with_less_workspace(cuda):
         out = tsa.scaled_dot_product_attention(q, k, v, attn_mask=mask, enable_gqa=True,
                                                workspace=torch.empty(room, dtype=torch.uint8, device=cuda))
         assert_close(out, OA.sdpa_cpu_fp32(q.cpu(), k.cpu(), v.cpu(), attn_mask=mask.cpu()))
+
+
+# Grids on both sides of the workgroup shapes' lines, for a 256-unit device
+# (the numbers of 64-, 128- and 256-row blocks decide): one step of keys; 64
+# and 65 rows; 256 and 260 64-row blocks (2 x 32 heads x 256 / 257 queries);
+# the same for causal at twice that; whole and partial rounds of 256-row
+# blocks; ragged last blocks and steps throughout.
+SHAPES = [(1, 8, 8, 64, 64, False), (1, 8, 8, 64, 65, False), (1, 8, 8, 65, 200, False), (2, 32, 8, 256, 130, False),
+          (2, 32, 8, 257, 130, False), (2, 32, 32, 512, 512, True), (2, 32, 8, 513, 513, True),
+          (4, 32, 8, 500, 90, False), (5, 32, 8, 300, 190, False), (1, 4, 4, 3400, 3400, True)]
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("kind", [None, "bool", "f16"])
+@pytest.mark.parametrize("case", SHAPES, ids=str)
+def test_workgroup_shapes(cuda, case, kind, D):
+    import torch_spyre_amd as tsa
+
+    B, Hq, Hkv, Sq, Skv, causal = case
+    if causal and kind is not None:
+        pytest.skip("causal calls take no mask")
+    q = randn((B, Hq, Sq, D), SEED + 330)
+    k, v = randn((B, Hkv, Skv, D), SEED + 331), randn((B, Hkv, Skv, D), SEED + 332)
+    mask = None if kind is None else make_mask(kind, "qk", B, Hq, Sq, Skv, SEED + 333)
+    out, lse = tsa.scaled_dot_product_attention(
+        q.to(cuda), k.to(cuda), v.to(cuda), attn_mask=None if mask is None else mask.to(cuda), is_causal=causal,
+        enable_gqa=True, return_lse=True)
+    heads = sorted({0, Hq // 2, Hq - 1})  # sampled heads: the reference runs on the CPU
+    qs, ks, vs = q[:, heads], k[:, [h // (Hq // Hkv) for h in heads]], v[:, [h // (Hq // Hkv) for h in heads]]
+    assert_close(out[:, heads], OA.sdpa_cpu_fp32(qs, ks, vs, attn_mask=mask, is_causal=causal))
+    _, lse64 = OA.sdpa_decomposition_fp64(qs, ks, vs, attn_mask=None if mask is None else mask.numpy(),
+                                          is_causal=causal, return_lse=True)
+    assert np.allclose(lse[:, heads].cpu().numpy(), lse64, atol=LSE_ATOL, rtol=0)
+    assert not torch.isnan(out).any()

@@ -13,10 +13,10 @@
 // Kernels, on the caller's stream:
 //  * sdpa_fwd_lds_kernel serves calls without a mask (plain or causal) and
 //    fp16 / boolean masks whose rows are whole 16-byte units.  A workgroup
-//    of 8 wavefronts takes 256 queries of one (sequence, q head); wavefront w
-//    takes 32.  Per 64-key step the K and V tiles (row-major, padded) move
-//    from L2 straight into LDS (buffer loads with the LDS flag), once for all
-//    8 wavefronts:
+//    of 4 or 8 wavefronts takes 32 queries of one (sequence, q head) per
+//    wavefront or pair of wavefronts (pick_shape).  Per 64-key step the K and
+//    V tiles (row-major, padded) move from L2 straight into LDS (buffer loads
+//    with the LDS flag), once for all its wavefronts:
 //       S^T[key, q] = K[key, :] Q^T[:, q]     2 x D/16 MFMA 32x32x16
 //       online softmax in fp32 (exp2 domain), lazy rescaling of the max;
 //       O^T[d, q] += V^T[d, key] P^T[key, q]  4 x D/32 MFMA 32x32x16
@@ -325,8 +325,9 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_fwd_kernel(FwdArgs a) {
 
 // ---- 3. attention with K/V tiles shared through LDS (no mask) -------------
 //
-// One workgroup of kWaves2 wavefronts per 256 queries of one (sequence, q
-// head); wavefront w takes 32 of them.  Per 64-key step t the workgroup
+// A workgroup of W = 8 or 4 wavefronts takes W x 32 queries of one (sequence,
+// q head), wavefront w 32 of them (or, in half steps, W / 2 x 32 queries;
+// which of them a call runs: pick_shape).  Per 64-key step t the workgroup
 // stages the K tile and the V tile, both [64 keys][D] as K and V lie in
 // memory, in LDS, and every wavefront reads its MFMA operands from there:
 //   S^T[key, q] = K Q^T   2 x D/16 MFMA 32x32x16 (M = 32 keys, N = 32 queries)
@@ -351,7 +352,7 @@ typedef short v4i16 __attribute__((ext_vector_type(4)));
 constexpr int kWaves2 = 8;
 constexpr int kThreads2 = kWaves2 * 64;
 constexpr int kQW = 32;             // queries per wavefront
-constexpr int kQB = kWaves2 * kQW;  // queries per workgroup
+constexpr int kQB = kWaves2 * kQW;  // rows of the largest workgroup
 constexpr int kKT = 64;             // keys per step
 static_assert(kStick % kKT == 0, "the Vt padding must cover whole steps");
 constexpr int kPadH = 8;            // LDS row padding, halves (16 bytes)
@@ -452,15 +453,15 @@ template <bool HALF> struct MaskTile<kNoMask, HALF> {
 // HALF (blocks of at most 128 rows, e.g. decode): wavefronts 2r and 2r + 1
 // share row tile r and take one 32-key half of every step each; the pair's
 // partials are folded in LDS at the end.
-template <int D, bool PRESCALED, int MK, int SLOTS = 2, bool HALF = false>
-__global__ __launch_bounds__(kThreads2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
+template <int D, bool PRESCALED, int MK, int SLOTS, bool HALF, int W>
+__global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   static_assert(SLOTS == 2 || (SLOTS == 4 && MK == kNoMask), "four slots leave no room for a mask");
   using L = Lds2<D>;
   using MT = MaskTile<MK, HALF>;
   constexpr int DK = D / 16;  // QK k-steps
   constexpr int DM = D / 32;  // O row tiles
   // Two K / V slots, then (masked calls) two mask blocks per wavefront.
-  __shared__ __align__(16) _Float16 lds[SLOTS * L::kSlot + kWaves2 * MT::kBytes];
+  __shared__ __align__(16) _Float16 lds[SLOTS * L::kSlot + W * MT::kBytes];
 
   // item = ((b * Hkv + kvh) * qblocks + (qblocks - 1 - qb)) * gp + gi: the
   // blocks of one (sequence, KV head) are consecutive, latest query block
@@ -478,9 +479,10 @@ __global__ __launch_bounds__(kThreads2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   const int kvh = static_cast<int>(i3 - bq * a.Hkv);
   const int b = static_cast<int>(bq);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
-  __builtin_assume(wave >= 0 && wave < kWaves2);  // lets the compiler drop always-true load guards
+  __builtin_assume(wave >= 0 && wave < W);  // lets the compiler drop always-true load guards
   const int hw = HALF ? (wave & 1) : 0;  // HALF: the key half of each step
-  const int qw0 = qb * kQB, q0 = qw0 + (HALF ? (wave >> 1) : wave) * kQW;  // rows
+  constexpr int kRows = (HALF ? W / 2 : W) * kQW;
+  const int qw0 = qb * kRows, q0 = qw0 + (HALF ? (wave >> 1) : wave) * kQW;  // rows
   const int col = lane & 31, half = lane >> 5;
   const int qrow = q0 + col;
   const int qi = static_cast<int>(fdiv(qrow, a.by_pack));  // this lane's query
@@ -490,7 +492,7 @@ __global__ __launch_bounds__(kThreads2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   // The wavefront's first and last query, and the block's last.
   const int q_lo = static_cast<int>(fdiv(q0, a.by_pack));
   const int q_hi = static_cast<int>(fdiv(q0 + kQW - 1, a.by_pack));
-  const int qb_hi = static_cast<int>(fdiv(qw0 + kQB - 1, a.by_pack));
+  const int qb_hi = static_cast<int>(fdiv(qw0 + kRows - 1, a.by_pack));
 
   // Q^T operand: lane (query column, half) holds features 16ks + 8half .. +8.
   f16x8 qv[DK];
@@ -523,18 +525,18 @@ __global__ __launch_bounds__(kThreads2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   constexpr int kUK = L::kRowK / 8, kUV = L::kRowV / 8;  // 16-byte units per padded row
   constexpr int kNK = kKT * kUK / 64, kNV = kKT * kUV / 64;  // loads per tile
   static_assert(kKT * kUK % 64 == 0 && kKT * kUV % 64 == 0, "tiles must be whole loads");
-  constexpr int kJK = (kNK + kWaves2 - 1) / kWaves2, kJV = (kNV + kWaves2 - 1) / kWaves2;
+  constexpr int kJK = (kNK + W - 1) / W, kJV = (kNV + W - 1) / W;
   constexpr uint32_t kOob = 0x80000000u;  // past kBufRange
   uint32_t k_off[kJK], v_off[kJV];
 #pragma unroll
   for (int j = 0; j < kJK; ++j) {
-    const int u = 64 * (wave + kWaves2 * j) + lane, row = u / kUK, ch = u % kUK;
+    const int u = 64 * (wave + W * j) + lane, row = u / kUK, ch = u % kUK;
     const bool pad = ch == kUK - 1;
     k_off[j] = pad ? kOob : (static_cast<uint32_t>(row) * static_cast<uint32_t>(a.k_ss) + 8 * ch) * 2;
   }
 #pragma unroll
   for (int j = 0; j < kJV; ++j) {
-    const int u = 64 * (wave + kWaves2 * j) + lane, row = u / kUV, ch = u % kUV;
+    const int u = 64 * (wave + W * j) + lane, row = u / kUV, ch = u % kUV;
     const bool pad = ch >= D / 8;  // kRowV / 8 - D / 8 pad units per row
     v_off[j] = pad ? kOob : (static_cast<uint32_t>(row) * static_cast<uint32_t>(a.v_ss) + 8 * ch) * 2;
   }
@@ -564,7 +566,7 @@ __global__ __launch_bounds__(kThreads2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
     const Rsrc r = make_rsrc(k_cur, range_of(k_left));
 #pragma unroll
     for (int j = 0; j < kJK; ++j)
-      if (wave + kWaves2 * j < kNK) load_lds16(r, lds + slot * L::kSlot + 512 * (wave + kWaves2 * j), k_off[j]);
+      if (wave + W * j < kNK) load_lds16(r, lds + slot * L::kSlot + 512 * (wave + W * j), k_off[j]);
     k_cur += k_tile;
     k_left -= k_step;
   };
@@ -574,8 +576,8 @@ __global__ __launch_bounds__(kThreads2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
     const Rsrc r = make_rsrc(v_cur, range_of(v_left));
 #pragma unroll
     for (int j = 0; j < kJV; ++j)
-      if (wave + kWaves2 * j < kNV)
-        load_lds16(r, lds + slot * L::kSlot + L::kK + 512 * (wave + kWaves2 * j), v_off[j]);
+      if (wave + W * j < kNV)
+        load_lds16(r, lds + slot * L::kSlot + L::kK + 512 * (wave + W * j), v_off[j]);
     v_cur += v_tile;
     v_left -= v_step;
   };
@@ -601,7 +603,7 @@ __global__ __launch_bounds__(kThreads2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
       m_off[j] = ok ? (at + 32 * hw) * MT::kEsz + 16 * ch : kOob;
     }
   }
-  auto mask_block = [&](int slot) { return lds + SLOTS * L::kSlot + (slot * kWaves2 + wave) * (MT::kBytes / 2); };
+  auto mask_block = [&](int slot) { return lds + SLOTS * L::kSlot + (slot * W + wave) * (MT::kBytes / 2); };
   auto dma_m = [&](int kb, int slot) {
     if constexpr (MK != kNoMask) {
       const uint32_t done = static_cast<uint32_t>(kb) * MT::kEsz;  // < Skv esz <= m_bytes
@@ -1670,8 +1672,58 @@ size_t split_bytes(int64_t rows, int nsplit, int D) {
 
 int pack_heads(int B, int Hkv, int g, int Sq);
 
-int64_t blocks_for(int B, int Hkv, int g, int Sq, int pack) {
-  return static_cast<int64_t>(B) * Hkv * (g / pack) * ((static_cast<int64_t>(pack) * Sq + kQB - 1) / kQB);
+int64_t blocks_for(int B, int Hkv, int g, int Sq, int pack, int rows = kQB) {
+  return static_cast<int64_t>(B) * Hkv * (g / pack) * ((static_cast<int64_t>(pack) * Sq + rows - 1) / rows);
+}
+
+// The workgroup an LDS-kernel call runs: W wavefronts, each a row tile of
+// its own (W x 32 rows), or two to a tile in half steps (W / 2 x 32 rows).
+//  k256  8 wavefronts, 256 rows, one workgroup per compute unit;
+//  k128  4 wavefronts, 128 rows, two per unit: half the rows of k256 waste
+//        less of a last round and of causal attention's uneven blocks, and
+//        the two of a unit do not wait for each other at barriers;
+//  kHalf8 8 wavefronts, 128 rows in half steps, K / V two steps ahead;
+//  kHalf4 4 wavefronts, 64 rows in half steps, two per unit: the shortest
+//        chain per block, for grids that leave units idle otherwise.
+enum Shape { k256, k128, kHalf8, kHalf4 };
+int shape_rows(Shape s) { return s == k256 ? 256 : s == kHalf4 ? 64 : 128; }
+
+// Which of them, for `groups` (sequence, q heads sharing rows, key split)
+// triples of `rows` rows over `keys` keys each.  Measured, prepared calls, one
+// box, 32 / 8 heads of D 128 at batch 1 unless said (k256 / kHalf8 / k128 /
+// kHalf4, us):
+//  * one step of keys: k128 (64 x 64: 7.1 / 7.1 / 6.5 / 7.0), the fold of
+//    half steps is not paid back;
+//  * else at most 64 rows: kHalf8 (16 queries x 8000 keys, B 4: 34.8 in
+//    kHalf8, 38.7 in k128, 37.9 in kHalf4);
+//  * a 64-row grid of one block per unit (causal, whose long and short
+//    blocks share units: two): kHalf4 (512 x 512: 20.8 / 16.8 / 15.5 / 14.1;
+//    causal 1000: 31.2 / 24.6 / 24.0 / 21.2).  Beyond it k128 is level or
+//    better (1000 x 1000: 32.2 / 27.3 / 25.7 / 25.7; 2048 causal: 56.4 / 52.0
+//    / 49.1 / 50.3; B 4 x 64 x 2000 keys: 28.1 / 36.8 / 27.8 / 32.9);
+//  * D 128, nearly whole rounds of 256-row blocks without more padding, and
+//    for causal attention at least 14 blocks a head, whose uneven lengths
+//    then even out: k256 (4096: 255.4 / 321 / 258.3 / 316; causal 8192: 513 /
+//    643 / 527 / 638; B 4 x 200 x 8000 keys: 124.3 / 159 / 129.2 / 176);
+//  * else k128 (1536: 69.3 / 73.2 / 60.7 / 71.3; 2500: 142.6 / 141.7 / 121.8 /
+//    129.6; causal 3072: 89.7 / 106.0 / 84.9 / 102.2; D 64, 4 x 16 heads x
+//    4096: 352 / 477 / 338 / 397).
+// A mask's blocks beside K and V leave room for one workgroup of any shape
+// per unit, except boolean masks at D 64 (k128, kHalf4) and fp16 masks at D
+// 64 (kHalf4): kHalf8 then while its grid is one block per unit (1000 x
+// 1000 with a causal boolean mask: 44.9 / 34.0 / 39.4 / 52.4), else k256.
+Shape pick_shape(int64_t groups, int64_t rows, int keys, int D, bool causal, int mask_kind) {
+  const int64_t cus = device_cus() > 0 ? device_cus() : 256;
+  auto blocks = [&](int64_t r) { return groups * ((rows + r - 1) / r); };
+  const bool two_half = mask_kind == kNoMask || D == 64;        // two kHalf4 per unit
+  const bool two_full = two_half && mask_kind != kMaskF16;      // two k128 per unit
+  if (keys <= kKT && two_full) return k128;
+  if (rows <= 64) return kHalf8;
+  if (two_half && blocks(64) <= (causal ? 2 : 1) * cus) return kHalf4;
+  if (!two_full) return blocks(128) <= cus ? kHalf8 : k256;
+  const int64_t n256 = blocks(256), rounds = (n256 + cus - 1) / cus;
+  const bool whole = n256 * 100 >= rounds * cus * 85 && blocks(128) * 100 >= n256 * 195;
+  return D == 128 && whole && (!causal || rows > 13 * 256) ? k256 : k128;
 }
 
 // The grid of a call: short query runs pack all g q heads of a KV head into
@@ -1689,12 +1741,13 @@ struct GridPlan {
   size_t part_bytes = 0;
   bool short_decode = false;  // sdpa_decode_short_kernel
   int waves = kWaves2;         // its wavefronts per block
+  Shape shape = k256;
 };
 
-// masked: a staged or copied mask, can_pack: its rows of a KV head's q heads
-// fit one buffer descriptor (else heads stay apart).
+// mask_kind: a staged or copied mask's; can_pack: its rows of a KV head's q
+// heads fit one buffer descriptor (else heads stay apart).
 GridPlan plan_grid(int B, int Hq, int Hkv, int Sq, int Skv, int D, bool causal, size_t ws_bytes,
-                   bool masked = false, bool can_pack = true) {
+                   int mask_kind = kNoMask, bool can_pack = true) {
   GridPlan gp;
   const int g = can_pack ? Hq / Hkv : 1;
   const int Hb = Hq / g;  // the (KV head, pack group) pairs of a sequence
@@ -1702,7 +1755,7 @@ GridPlan plan_grid(int B, int Hq, int Hkv, int Sq, int Skv, int D, bool causal, 
   // Short decode: one row tile (the g q heads of a KV head times Sq <= 32
   // rows) whose keys fit one block (kWaves2 slices), or a split of them
   // over blocks that all run in one round of the device.
-  if (!causal && !masked && Sq > 0 && static_cast<int64_t>(g) * Sq <= 32) {
+  if (!causal && mask_kind == kNoMask && Sq > 0 && static_cast<int64_t>(g) * Sq <= 32) {
     const int kw = D == 64 ? ShortLds<64>::kKW : ShortLds<128>::kKW;
     const int64_t cus = device_cus() > 0 ? device_cus() : 256;
     int waves = kWaves2;
@@ -1738,10 +1791,14 @@ GridPlan plan_grid(int B, int Hq, int Hkv, int Sq, int Skv, int D, bool causal, 
       gp.nsplit = ns;
       gp.split_keys = keys;
       gp.part_bytes = pb;
+      gp.shape = pick_shape(static_cast<int64_t>(B) * Hb * (g / p0) * ns, static_cast<int64_t>(p0) * Sq, keys, D, causal,
+                            mask_kind);
       return gp;
     }
   }
   gp.pack = pack_heads(B, Hb, g, Sq);
+  gp.shape = pick_shape(static_cast<int64_t>(B) * Hb * (g / gp.pack), static_cast<int64_t>(gp.pack) * Sq, Skv, D, causal,
+                        mask_kind);
   return gp;
 }
 
@@ -1776,17 +1833,17 @@ void launch_short(const Fwd2Args& f2, int D, bool prescaled, int waves, hipStrea
     launch_short_w<kWaves2>(f2, D, prescaled, st);
 }
 
-template <int MK, int SLOTS, bool HALF = false>
+template <int MK, int SLOTS, bool HALF, int W>
 void launch_lds(const Fwd2Args& f2, int D, bool prescaled, hipStream_t st) {
   const dim3 grid(f2.n_items);
   if (D == 128 && prescaled)
-    sdpa_fwd_lds_kernel<128, true, MK, SLOTS, HALF><<<grid, kThreads2, 0, st>>>(f2);
+    sdpa_fwd_lds_kernel<128, true, MK, SLOTS, HALF, W><<<grid, W * 64, 0, st>>>(f2);
   else if (D == 128)
-    sdpa_fwd_lds_kernel<128, false, MK, SLOTS, HALF><<<grid, kThreads2, 0, st>>>(f2);
+    sdpa_fwd_lds_kernel<128, false, MK, SLOTS, HALF, W><<<grid, W * 64, 0, st>>>(f2);
   else if (prescaled)
-    sdpa_fwd_lds_kernel<64, true, MK, SLOTS, HALF><<<grid, kThreads2, 0, st>>>(f2);
+    sdpa_fwd_lds_kernel<64, true, MK, SLOTS, HALF, W><<<grid, W * 64, 0, st>>>(f2);
   else
-    sdpa_fwd_lds_kernel<64, false, MK, SLOTS, HALF><<<grid, kThreads2, 0, st>>>(f2);
+    sdpa_fwd_lds_kernel<64, false, MK, SLOTS, HALF, W><<<grid, W * 64, 0, st>>>(f2);
 }
 
 // A copy of a mask with 16-byte rows: [bm][hm][qm][pitch bytes], keys past
@@ -1905,8 +1962,8 @@ size_t copy_room(const MaskPlan& mp) {
 }
 
 // The grid of a staged or copied mask's call given ws_bytes beyond the copy.
-GridPlan masked_grid(const MaskPlan& mp, int B, int Hq, int Hkv, int Sq, int Skv, int D, size_t ws_bytes) {
-  return plan_grid(B, Hq, Hkv, Sq, Skv, D, false, ws_bytes, true, mask_extent(mp, Hq / Hkv) <= kBufRange);
+GridPlan masked_grid(const MaskPlan& mp, int kind, int B, int Hq, int Hkv, int Sq, int Skv, int D, size_t ws_bytes) {
+  return plan_grid(B, Hq, Hkv, Sq, Skv, D, false, ws_bytes, kind, mask_extent(mp, Hq / Hkv) <= kBufRange);
 }
 
 // Compute units of the current device, cached per device; 0 if the runtime
@@ -1959,7 +2016,7 @@ extern "C" size_t spyre_sdpa_fwd_call_workspace_bytes(const void* attn_mask, int
   if (!mask_strides || mask_kind < kNoMask || mask_kind > kMaskBool) return 0;
   const MaskPlan mp = plan_mask(attn_mask, mask_kind, mask_strides, B, Hq, Sq, Skv);
   if (mp.route == kRouteVt) return spyre_sdpa_fwd_workspace_bytes(B, Hkv, Skv, D);
-  const size_t part = masked_grid(mp, B, Hq, Hkv, Sq, Skv, D, SIZE_MAX).part_bytes;
+  const size_t part = masked_grid(mp, mask_kind, B, Hq, Hkv, Sq, Skv, D, SIZE_MAX).part_bytes;
   return part ? copy_room(mp) + part : mp.copy_bytes;
 }
 
@@ -2126,14 +2183,15 @@ extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const
     const size_t part_at = copy_room(mp);
     const size_t part_room = ws_room > part_at ? ws_room - part_at : 0;
     const GridPlan gpl = mask_kind == kNoMask ? plan_grid(B, Hq, Hkv, Sq, Skv, D, is_causal != 0, part_room)
-                                              : masked_grid(mp, B, Hq, Hkv, Sq, Skv, D, part_room);
+                                              : masked_grid(mp, mask_kind, B, Hq, Hkv, Sq, Skv, D, part_room);
     f2.pack = gpl.pack;
     f2.gp = fa.g / f2.pack;
-    f2.qblocks = static_cast<int>((static_cast<int64_t>(f2.pack) * Sq + kQB - 1) / kQB);
+    const int rows = shape_rows(gpl.shape);
+    f2.qblocks = static_cast<int>((static_cast<int64_t>(f2.pack) * Sq + rows - 1) / rows);
     f2.nsplit = gpl.nsplit;
     f2.split_keys = gpl.nsplit > 1 ? gpl.split_keys : Skv;
     f2.part = gpl.nsplit > 1 ? reinterpret_cast<float*>(static_cast<char*>(workspace) + part_at) : nullptr;
-    const int64_t items = blocks_for(B, Hkv, fa.g, Sq, f2.pack) * f2.nsplit;
+    const int64_t items = blocks_for(B, Hkv, fa.g, Sq, f2.pack, rows) * f2.nsplit;
     SPYRE_REQUIRE(items < (int64_t{1} << 31), SPYRE_EUNSUPPORTED, "too many query blocks");
     f2.n_items = static_cast<uint32_t>(items);
     f2.by_split = spyre_hip::make_fastdiv(static_cast<uint32_t>(f2.nsplit));
@@ -2150,23 +2208,24 @@ extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const
     f2.m_sh = mp.sh;
     f2.m_sq = mp.sq;
     f2.m_bytes = static_cast<uint32_t>(mask_extent(mp, f2.pack));
-    // Blocks of at most 128 rows: half steps (two wavefronts per row tile).
-    const bool half = static_cast<int64_t>(f2.pack) * Sq <= kQB / 2;
     if (gpl.short_decode) {
       // One row tile, its keys all in flight at once; a key split merges in
       // the same kernel.
       f2.ticket = spyre_hip::next_call_ticket();
       launch_short(f2, D, prescaled, gpl.waves, st);
-    } else if (mask_kind == kMaskF16) {
-      half ? launch_lds<kMaskF16, 2, true>(f2, D, prescaled, st) : launch_lds<kMaskF16, 2>(f2, D, prescaled, st);
-    } else if (mask_kind == kMaskBool) {
-      half ? launch_lds<kMaskBool, 2, true>(f2, D, prescaled, st) : launch_lds<kMaskBool, 2>(f2, D, prescaled, st);
-    } else if (half) {
-      launch_lds<kNoMask, 4, true>(f2, D, prescaled, st);
-    } else if (static_cast<int64_t>(f2.pack) * Sq < kQB) {
-      launch_lds<kNoMask, 4>(f2, D, prescaled, st);  // blocks with fewer rows than wavefronts can fill
     } else {
-      launch_lds<kNoMask, 2>(f2, D, prescaled, st);
+      auto go = [&](auto mk) {
+        constexpr int MK = decltype(mk)::value;
+        switch (gpl.shape) {
+          case k256: launch_lds<MK, 2, false, 8>(f2, D, prescaled, st); break;
+          case kHalf8: launch_lds<MK, MK == kNoMask ? 4 : 2, true, 8>(f2, D, prescaled, st); break;
+          case k128: launch_lds<MK, 2, false, 4>(f2, D, prescaled, st); break;
+          default: launch_lds<MK, 2, true, 4>(f2, D, prescaled, st); break;
+        }
+      };
+      if (mask_kind == kMaskF16) go(std::integral_constant<int, kMaskF16>{});
+      else if (mask_kind == kMaskBool) go(std::integral_constant<int, kMaskBool>{});
+      else go(std::integral_constant<int, kNoMask>{});
     }
     if (f2.nsplit > 1 && !gpl.short_decode) {
       const hipError_t e0 = hipGetLastError();
