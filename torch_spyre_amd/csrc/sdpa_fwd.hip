@@ -358,16 +358,24 @@ static_assert(kStick % kKT == 0, "the Vt padding must cover whole steps");
 constexpr int kPadH = 8;            // LDS row padding, halves (16 bytes)
 constexpr int kPrefetch = 4;        // LDS operand reads in flight ahead of the MFMA using them
 
+// K and V tiles in LDS: rows of D halves, unpadded (two workgroups of W = 4
+// per compute unit then have 80 KB each, masks included, and a step's tiles
+// are 32 loads at D 128 where padded rows took 37), the 16-byte units of a
+// row exchanged by an XOR of their index with a function of the row.  Against
+// padded rows: 4096 x 4096 249.9 -> 246.5 us, causal 137.9 -> 135.6, D 64 (4 x 16
+// heads x 2048) 88.6 -> 86.1, fp16 mask [4096, 4096] 292.9 -> 284.7.
 template <int D>
 struct Lds2 {
-  static constexpr int kRowK = D + kPadH;    // K tile row (one key), halves
-  // V tile row: a transposed read serves 32 lanes at once, 4 rows x 4
-  // 8-byte units in each of two column groups 32 bytes apart; a row step of
-  // 16 (D = 128: 160 halves) or 48 (D = 64: 96 halves) banks mod 64 puts all
-  // of them in distinct banks.
-  static constexpr int kRowV = D + 32;
-  static constexpr int kK = kKT * kRowK;
-  static constexpr int kSlot = kK + kKT * kRowV;  // one slot: a K tile and a V tile
+  static constexpr int kTile = kKT * D;    // halves
+  static constexpr int kSlot = 2 * kTile;  // one slot: a K tile and a V tile
+  static constexpr int kUnits = D / 8;     // 16-byte units per row
+  // K: the 16 lanes an operand read serves at once read the same unit of 16
+  // rows (key32_of of 16 consecutive rho); the XOR puts them in 16 distinct
+  // units of the 256 bytes that LDS's 64 banks hold.
+  __device__ static __forceinline__ int swz_k(int row) { return D == 128 ? row & 15 : (row >> 1) & 7; }
+  // V: a transposed read serves 32 lanes at once, 4 consecutive rows x 64
+  // bytes; the XOR moves whole 64-byte groups, to four distinct ones.
+  __device__ static __forceinline__ int swz_v(int row) { return D == 128 ? 4 * (row & 3) : 4 * ((row >> 1) & 1); }
 };
 
 // S^T row rho of a 32-key half maps to key key32_of(rho) of that half: MFMA
@@ -428,17 +436,17 @@ struct Fwd2Args {
 };
 
 // A wavefront's mask block for one step: its 32 rows x the step's 64 keys
-// (HALF: the 32 keys of its half), rows padded by 16 bytes, staged in LDS by
-// buffer loads like the K / V tiles (whole 1 KB loads; units past the block
-// arrive as zeros in a spare tail).
+// (HALF: the 32 keys of its half), staged in LDS by buffer loads like the K /
+// V tiles, the 16-byte units of a row exchanged like K's.
 template <int ESZ, int KEYS> struct MaskRows {
   static constexpr int kEsz = ESZ;
-  static constexpr int kDataU = KEYS * ESZ / 16, kRowU = kDataU + 1;  // 16-byte units of a row
-  static constexpr int kLoads = (32 * kRowU + 63) / 64, kBytes = kLoads * 1024;
+  static constexpr int kU = KEYS * ESZ / 16;  // 16-byte units of a row
+  static constexpr int kLoads = 32 * kU / 64, kBytes = 32 * kU * 16;
+  __device__ static __forceinline__ int swz(int row) { return (row / (16 / kU)) & (kU - 1); }
 };
 template <int MK, bool HALF> struct MaskTile : MaskRows<MK == kMaskF16 ? 2 : 1, HALF ? 32 : 64> {};
 template <bool HALF> struct MaskTile<kNoMask, HALF> {
-  static constexpr int kEsz = 1, kDataU = 0, kRowU = 1, kLoads = 0, kBytes = 0;
+  static constexpr int kEsz = 1, kU = 1, kLoads = 0, kBytes = 0;
 };
 
 // PRESCALED (|scale log2 e| <= 1, so q * that never overflows fp16): Q is
@@ -460,8 +468,10 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   using MT = MaskTile<MK, HALF>;
   constexpr int DK = D / 16;  // QK k-steps
   constexpr int DM = D / 32;  // O row tiles
-  // Two K / V slots, then (masked calls) two mask blocks per wavefront.
-  __shared__ __align__(16) _Float16 lds[SLOTS * L::kSlot + W * MT::kBytes];
+  // The K / V slots, then (masked calls) two mask blocks per wavefront, or
+  // one where two would not leave room for a second workgroup of W = 4.
+  constexpr int kMaskSlots = MK != kNoMask && W == 4 && SLOTS * L::kSlot * 2 + 2 * W * MT::kBytes > 80 * 1024 ? 1 : 2;
+  __shared__ __align__(16) _Float16 lds[SLOTS * L::kSlot + kMaskSlots * W * MT::kBytes / 2];
 
   // item = ((b * Hkv + kvh) * qblocks + (qblocks - 1 - qb)) * gp + gi: the
   // blocks of one (sequence, KV head) are consecutive, latest query block
@@ -518,27 +528,19 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
 
   // Tiles move from L2 straight into LDS (buffer loads with the LDS flag):
   // lane l of a load writes the 16 bytes at M0 + 16 l, so load i of a tile
-  // fills its 16-byte units 64 i .. 64 i + 63, padded rows included.  Lane
-  // l of load i fetches the unit's source; pad units and K / V rows past Skv
-  // get an offset past the buffer's range and are written as zeros.  Per-lane
+  // fills its 16-byte units 64 i .. 64 i + 63.  Lane l of load i fetches the
+  // unit's source (the row's unit that the XOR puts there); K / V rows past
+  // Skv lie past the buffer's range and are written as zeros.  Per-lane
   // offsets are fixed for the whole loop; the step only moves the base.
-  constexpr int kUK = L::kRowK / 8, kUV = L::kRowV / 8;  // 16-byte units per padded row
-  constexpr int kNK = kKT * kUK / 64, kNV = kKT * kUV / 64;  // loads per tile
-  static_assert(kKT * kUK % 64 == 0 && kKT * kUV % 64 == 0, "tiles must be whole loads");
-  constexpr int kJK = (kNK + W - 1) / W, kJV = (kNV + W - 1) / W;
+  constexpr int kU = L::kUnits, kJ = kU / W;  // loads per tile, and per wavefront
+  static_assert(kU % W == 0, "every wavefront loads as much");
   constexpr uint32_t kOob = 0x80000000u;  // past kBufRange
-  uint32_t k_off[kJK], v_off[kJV];
+  uint32_t k_off[kJ], v_off[kJ];
 #pragma unroll
-  for (int j = 0; j < kJK; ++j) {
-    const int u = 64 * (wave + W * j) + lane, row = u / kUK, ch = u % kUK;
-    const bool pad = ch == kUK - 1;
-    k_off[j] = pad ? kOob : (static_cast<uint32_t>(row) * static_cast<uint32_t>(a.k_ss) + 8 * ch) * 2;
-  }
-#pragma unroll
-  for (int j = 0; j < kJV; ++j) {
-    const int u = 64 * (wave + W * j) + lane, row = u / kUV, ch = u % kUV;
-    const bool pad = ch >= D / 8;  // kRowV / 8 - D / 8 pad units per row
-    v_off[j] = pad ? kOob : (static_cast<uint32_t>(row) * static_cast<uint32_t>(a.v_ss) + 8 * ch) * 2;
+  for (int j = 0; j < kJ; ++j) {
+    const int u = 64 * (wave + W * j) + lane, row = u / kU, ch = u % kU;
+    k_off[j] = (static_cast<uint32_t>(row) * static_cast<uint32_t>(a.k_ss) + 8 * (ch ^ L::swz_k(row))) * 2;
+    v_off[j] = (static_cast<uint32_t>(row) * static_cast<uint32_t>(a.v_ss) + 8 * (ch ^ L::swz_v(row))) * 2;
   }
   // K / V tiles load in sequence (K(0), K(1), ... and V(0), V(1), ...), so
   // each has a running cursor: the next tile's first row and the bytes from
@@ -565,8 +567,7 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   auto dma_k = [&](int slot) {
     const Rsrc r = make_rsrc(k_cur, range_of(k_left));
 #pragma unroll
-    for (int j = 0; j < kJK; ++j)
-      if (wave + W * j < kNK) load_lds16(r, lds + slot * L::kSlot + 512 * (wave + W * j), k_off[j]);
+    for (int j = 0; j < kJ; ++j) load_lds16(r, lds + slot * L::kSlot + 512 * (wave + W * j), k_off[j]);
     k_cur += k_tile;
     k_left -= k_step;
   };
@@ -575,9 +576,7 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   auto dma_v = [&](int slot) {
     const Rsrc r = make_rsrc(v_cur, range_of(v_left));
 #pragma unroll
-    for (int j = 0; j < kJV; ++j)
-      if (wave + W * j < kNV)
-        load_lds16(r, lds + slot * L::kSlot + L::kK + 512 * (wave + W * j), v_off[j]);
+    for (int j = 0; j < kJ; ++j) load_lds16(r, lds + slot * L::kSlot + L::kTile + 512 * (wave + W * j), v_off[j]);
     v_cur += v_tile;
     v_left -= v_step;
   };
@@ -592,18 +591,18 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
     mbase = static_cast<const char*>(a.mask) + (b * a.m_sb + (kvh * a.g + gi * pack) * a.m_sh) * MT::kEsz;
 #pragma unroll
     for (int j = 0; j < MT::kLoads; ++j) {
-      const int u = 64 * j + lane, row = u / MT::kRowU, ch = u % MT::kRowU;
+      const int u = 64 * j + lane, row = u / MT::kU, ch = (u % MT::kU) ^ MT::swz(row);
       // a valid row's offset lies below m_bytes < 2^31, so 32 bits of each product do
       uint32_t mq = q0 + row, at = mq * static_cast<uint32_t>(a.m_sq);
       if (pack > 1) {
         mq = fdiv(q0 + row, a.by_pack);
         at = mq * static_cast<uint32_t>(a.m_sq) + (q0 + row - mq * pack) * static_cast<uint32_t>(a.m_sh);
       }
-      const bool ok = row < kQW && ch < MT::kDataU && static_cast<int>(mq) < a.Sq;
+      const bool ok = static_cast<int>(mq) < a.Sq;
       m_off[j] = ok ? (at + 32 * hw) * MT::kEsz + 16 * ch : kOob;
     }
   }
-  auto mask_block = [&](int slot) { return lds + SLOTS * L::kSlot + (slot * W + wave) * (MT::kBytes / 2); };
+  auto mask_block = [&](int slot) { return lds + SLOTS * L::kSlot + ((kMaskSlots == 2 ? slot : 0) * W + wave) * (MT::kBytes / 2); };
   auto dma_m = [&](int kb, int slot) {
     if constexpr (MK != kNoMask) {
       const uint32_t done = static_cast<uint32_t>(kb) * MT::kEsz;  // < Skv esz <= m_bytes
@@ -636,16 +635,20 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
 #pragma unroll
   for (int dm = 0; dm < DM; ++dm) o[dm] = f32x16{};
 
-  // S^T half mt (keys 32mt .. 32mt + 31 of the step) from the K tile at kt.
-  auto qk = [&](const _Float16* kt, int mt) {
-    const _Float16* krow = kt + (mt * 32 + key32_of(col)) * L::kRowK + 8 * half;
-    f32x16 acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const f16x8*>(krow), qv[0],
+  auto lds_at = [&](uint32_t byte) { return reinterpret_cast<const char*>(lds) + byte; };
+  // This lane's K operands in a K tile: row key32_of(col) of a 32-key half,
+  // unit 2 ks + half of k-step ks, at byte k_lane ^ (32 ks) + 64 D mt.
+  const uint32_t k_lane = static_cast<uint32_t>(key32_of(col) * D * 2 + ((half ^ L::swz_k(key32_of(col))) * 16));
+  auto k_frag = [&](uint32_t kt, int mt, int ks) -> f16x8 {  // kt: the tile's byte + k_lane
+    return *reinterpret_cast<const f16x8*>(lds_at((kt ^ (32 * ks)) + mt * 32 * D * 2));
+  };
+  // S^T half mt (keys 32mt .. 32mt + 31 of the step) from K tile 0 of slot 0.
+  auto qk = [&](int mt) {
+    f32x16 acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(k_frag(k_lane, mt, 0), qv[0],
                                                         PRESCALED ? neg_m_tile : f32x16{}, 0, 0, 0);
 #pragma unroll
-    for (int ks = 1; ks < DK; ++ks) {
-      const f16x8 ka = *reinterpret_cast<const f16x8*>(krow + 16 * ks);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qv[ks], acc, 0, 0, 0);
-    }
+    for (int ks = 1; ks < DK; ++ks)
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(k_frag(k_lane, mt, ks), qv[ks], acc, 0, 0, 0);
     return acc;
   };
   // Lane (query column, half) holds S^T rows 8i + 4half + v of each 32-key
@@ -667,28 +670,44 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   // units (PRESCALED: log2 units, else divided by |scale|), a keep-mask
   // sends dropped scores to -inf.
   const float bias_mul = PRESCALED ? kLog2e : kLog2e / scale_abs;
+  // This lane's byte of the block: row col, its first key's unit (fp16: unit
+  // `half`; boolean: byte 8 half of unit 0).
+  uint32_t m_lane = 0;
+  if constexpr (MK == kMaskF16) m_lane = col * (16 * MT::kU) + ((half ^ MT::swz(col)) * 16);
+  if constexpr (MK == kMaskBool) m_lane = col * (16 * MT::kU) + MT::swz(col) * 16 + 8 * half;
   // Half mt of the mask block (HALF: its one half, mt 0) onto S half s.
   auto apply_mask_half = [&](int t, int mt, f32x16& s) {
     if constexpr (MK != kNoMask) {
-      const char* row = reinterpret_cast<const char*>(mask_block(t & 1)) + col * (16 * MT::kRowU);
+      const char* blk = reinterpret_cast<const char*>(mask_block(t & 1));
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int k4 = 32 * mt + 16 * (i >> 1) + 8 * half + 4 * (i & 1);
+        // keys 32 mt + 16 (i / 2) + 8 half + 4 (i % 2) .. + 3 of row col
         if constexpr (MK == kMaskF16) {
-          const f16x4 m4 = *reinterpret_cast<const f16x4*>(row + 2 * k4);
+          const uint32_t at = (m_lane ^ (64 * mt + 32 * (i >> 1))) + 8 * (i & 1);
+          const f16x4 m4 = *reinterpret_cast<const f16x4*>(blk + at);
 #pragma unroll
           for (int v = 0; v < 4; ++v) s[4 * i + v] = __builtin_fmaf(static_cast<float>(m4[v]), bias_mul, s[4 * i + v]);
         } else {
-          const uint32_t m4 = *reinterpret_cast<const uint32_t*>(row + k4);
+          const uint32_t at = (m_lane ^ (32 * mt + 16 * (i >> 1))) + 4 * (i & 1);
+          const uint32_t m4 = *reinterpret_cast<const uint32_t*>(blk + at);
 #pragma unroll
           for (int v = 0; v < 4; ++v) s[4 * i + v] = ((m4 >> (8 * v)) & 0xffu) != 0 ? s[4 * i + v] : -INFINITY;
         }
       }
     }
   };
+  // One mask block per wavefront: the next step's loads go out once this
+  // step's reads have returned.
+  auto next_mask = [&](int t) {
+    if constexpr (MK != kNoMask && kMaskSlots == 1) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (t + 1 < n_tiles) dma_m(kb0 + (t + 1) * kKT, 0);
+    }
+  };
   auto apply_mask = [&](int t, f32x16 (&s)[2]) {
     apply_mask_half(t, 0, s[0]);
     apply_mask_half(t, 1, s[1]);
+    next_mask(t);
   };
   // The running max (log2 domain) moves only when a score of the step
   // exceeds it by more than 2^8, so P <= 256 (fine in fp16) and most steps
@@ -791,24 +810,52 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   // Each fragment is read kPrefetch MFMAs before its use: with reads issued
   // only just ahead, every MFMA waited out an LDS read.
   constexpr int kNF = 2 * DK + 4 * DM;
-  // LDS element offsets of the Vt rows of the step's four 16-key columns,
-  // hidden from the compiler: otherwise it pairs reads whose addresses are
-  // 32 bytes apart and issues the earlier one late, beside the later one.
-  uint32_t vtr;  // this lane's V tile element for the transposed reads, in the step's slot
   // Within each 16 lanes, lane s reads V[key 8 half + s / 4][d 16 (lane / 16 % 2) + 4 (s % 4)
   // .. + 3]; ds_read_b64_tr_b16 hands lane j of the 16 the four keys of column d + j.
-  const uint32_t vtr_lane = static_cast<uint32_t>((8 * half + ((lane & 15) >> 2)) * L::kRowV +
-                                                  16 * ((lane >> 4) & 1) + 4 * (lane & 3));
-  auto tr4 = [&](uint32_t e) { return tr_read4(lds + e); };
-  auto frag = [&](const _Float16* k1, int i) -> f16x8 {
-    if (i < 2 * DK)  // the two halves' chains alternate: half i % 2, k-step i / 2
-      return *reinterpret_cast<const f16x8*>(k1 + ((i % 2) * 32 + key32_of(col)) * L::kRowK + 8 * half +
-                                             16 * (i / 2));
-    i -= 2 * DK;
-    // keys 16 (i / DM) + 8 half .. + 7 of feature 32 (i % DM) + col
-    const uint32_t e = vtr + (16 * (i / DM)) * L::kRowV + 32 * (i % DM);
-    const v4i16 lo = tr4(e), hi = tr4(e + 4 * L::kRowV);
+  const int v_row = 8 * half + ((lane & 15) >> 2);
+  const uint32_t v_lane = static_cast<uint32_t>(L::kTile * 2 + v_row * D * 2 + L::swz_v(v_row) * 16 +
+                                                32 * ((lane >> 4) & 1) + 8 * (lane & 3));
+  // Half steps: the step's LDS bytes of this lane's K and V operands, the XOR
+  // of a k-step or O row tile applied at each read (their registers have
+  // room for two workgroups anyway, their time is latency).  Full steps: every
+  // such byte in a register of its own for the whole loop, the slot (the
+  // step's parity) in the reads' immediate offset -- the XORs in an
+  // issue-bound loop cost 2-9 % (4096 causal 136.1 -> 145.1 us).  Hidden
+  // from the compiler either way: it would pair reads whose addresses are 32
+  // bytes apart and issue the earlier one late, beside the later one.
+  uint32_t k_cur_lds, v_cur_lds, k_at[DK], v_at[DM];
+  if constexpr (!HALF) {
+#pragma unroll
+    for (int ks = 0; ks < DK; ++ks) {
+      k_at[ks] = k_lane ^ (32 * ks);
+      asm volatile("" : "+v"(k_at[ks]));
+    }
+#pragma unroll
+    for (int dm = 0; dm < DM; ++dm) {
+      v_at[dm] = v_lane ^ (64 * dm);
+      asm volatile("" : "+v"(v_at[dm]));
+    }
+  }
+  auto step_lds = [&](int t) {
+    k_cur_lds = static_cast<uint32_t>(((t + 1) % SLOTS) * L::kSlot * 2) + k_lane;
+    v_cur_lds = static_cast<uint32_t>((t % SLOTS) * L::kSlot * 2) + v_lane;
+    asm volatile("" : "+v"(k_cur_lds), "+v"(v_cur_lds));
+  };
+  // V^T operand at LDS byte `at` (of c = 0): keys 16 c + 8 half .. + 7 of one
+  // feature per lane (rows + 4 have the XOR of rows + 0).
+  auto v_frag = [&](uint32_t at, int c) -> f16x8 {
+    const char* p = lds_at(at + 16 * c * D * 2);
+    const v4i16 lo = tr_read4(reinterpret_cast<const _Float16*>(p)),
+                hi = tr_read4(reinterpret_cast<const _Float16*>(p + 4 * D * 2));
     return __builtin_bit_cast(f16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  // Fragment i of a full step of parity par (K(t+1) in slot 1 - par, V(t) in
+  // slot par).
+  auto frag = [&](int par, int i) -> f16x8 {
+    if (i < 2 * DK)  // the two halves' chains alternate
+      return *reinterpret_cast<const f16x8*>(
+          lds_at(k_at[i / 2] + (1 - par) * L::kSlot * 2 + (i % 2) * 32 * D * 2));
+    return v_frag(v_at[(i - 2 * DK) % DM] + par * L::kSlot * 2, (i - 2 * DK) / DM);
   };
   // Keeps a region's operand reads interleaved one per MFMA (n of each).
   // Keeps a region's operand reads interleaved with its MFMAs i0 .. i1 - 1:
@@ -851,13 +898,9 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   // lives in slot 0 of cur / nxt; its fragments are K half hw (vi < DK) and
   // the V^T operands of keys 32 hw .. + 31 (vi - DK = j DM + dm).
   constexpr int kNFH = DK + 2 * DM;
-  auto frag_h = [&](const _Float16* k1, int vi) -> f16x8 {
-    if (vi < DK)
-      return *reinterpret_cast<const f16x8*>(k1 + (hw * 32 + key32_of(col)) * L::kRowK + 8 * half + 16 * vi);
-    const int i = vi - DK;
-    const uint32_t e = vtr + (16 * (2 * hw + i / DM)) * L::kRowV + 32 * (i % DM);
-    const v4i16 lo = tr4(e), hi = tr4(e + 4 * L::kRowV);
-    return __builtin_bit_cast(f16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  auto frag_h = [&](int vi) -> f16x8 {
+    if (vi < DK) return *reinterpret_cast<const f16x8*>(lds_at((k_cur_lds ^ (32 * vi)) + hw * 32 * D * 2));
+    return v_frag(v_cur_lds ^ (64 * ((vi - DK) % DM)), 2 * hw + (vi - DK) / DM);
   };
   auto interleave_h = [](int i0, int i1) {
     for (int i = i0; i < i1; ++i) {
@@ -870,11 +913,10 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
     }
   };
   auto step_h = [&](int t, f32x16& cur, f32x16& nxt) {
-    const _Float16* k1 = lds + ((t + 1) % SLOTS) * L::kSlot;
     if constexpr (SLOTS == 2) {
       if (t + 2 < n_tiles) dma_k(t & 1);
       if (t + 1 < n_tiles) dma_v((t + 1) & 1);
-      if (t + 1 < n_tiles) dma_m(kb0 + (t + 1) * kKT, (t + 1) & 1);
+      if (kMaskSlots == 2 && t + 1 < n_tiles) dma_m(kb0 + (t + 1) * kKT, (t + 1) & 1);
     } else if ((t & 1) == 0) {
       if (t + 3 < n_tiles) dma_k((t + 3) % 4);
       if (t + 4 < n_tiles) dma_k(t % 4);
@@ -882,16 +924,18 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
       if (t + 3 < n_tiles) dma_v((t + 3) % 4);
     }
     if (active(t)) {
-      vtr = static_cast<uint32_t>((t % SLOTS) * L::kSlot + L::kK) + vtr_lane;
-      asm volatile("" : "+v"(vtr));
+      step_lds(t);
       f16x8 fr[kNFH];
 #pragma unroll
-      for (int i = 0; i < kPrefetch; ++i) fr[i] = frag_h(k1, i);
+      for (int i = 0; i < kPrefetch; ++i) fr[i] = frag_h(i);
       auto mfma = [&](int i, const f16x8& b, f32x16& acc) {
         acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[i], b, acc, 0, 0, 0);
-        if (i + kPrefetch < kNFH) fr[i + kPrefetch] = frag_h(k1, i + kPrefetch);
+        if (i + kPrefetch < kNFH) fr[i + kPrefetch] = frag_h(i + kPrefetch);
       };
-      if constexpr (MK != kNoMask) apply_mask_half(t, 0, cur);
+      if constexpr (MK != kNoMask) {
+        apply_mask_half(t, 0, cur);
+        next_mask(t);
+      }
       if (edge(t)) {  // the key test on this half
         const int kl = key_last - (kb0 + t * kKT) - 32 * hw - 8 * half;
 #pragma unroll
@@ -952,14 +996,13 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   // scheduling region pairs one MFMA group with one VALU group.  At a
   // wavefront's last active step S(t+1) reads a stale K slot and is never
   // used.
-  auto step = [&](int t, f32x16 (&cur)[2], f32x16 (&nxt)[2]) {
-    const _Float16* k1 = lds + ((t + 1) % SLOTS) * L::kSlot;
+  auto step = [&](int t, int par, f32x16 (&cur)[2], f32x16 (&nxt)[2]) {
     if constexpr (SLOTS == 2) {
       // K(t+2) replaces K(t) (read during step t-1), V(t+1) replaces
       // V(t-1); both land during this step's math.
       if (t + 2 < n_tiles) dma_k(t & 1);
       if (t + 1 < n_tiles) dma_v((t + 1) & 1);
-      if (t + 1 < n_tiles) dma_m(kb0 + (t + 1) * kKT, (t + 1) & 1);
+      if (kMaskSlots == 2 && t + 1 < n_tiles) dma_m(kb0 + (t + 1) * kKT, (t + 1) & 1);
     } else if ((t & 1) == 0) {
       // Steps t, t + 1 read K(t+1), K(t+2), V(t), V(t+1) (slot = tile % 4);
       // K(t+3), K(t+4), V(t+2), V(t+3) fill the other four slot halves,
@@ -971,15 +1014,13 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
       if (t + 3 < n_tiles) dma_v((t + 3) % 4);
     }
     if (active(t)) {
-      vtr = static_cast<uint32_t>((t % SLOTS) * L::kSlot + L::kK) + vtr_lane;
-      asm volatile("" : "+v"(vtr));
       f16x8 fr[kNF];
 #pragma unroll
-      for (int i = 0; i < kPrefetch; ++i) fr[i] = frag(k1, i);
+      for (int i = 0; i < kPrefetch; ++i) fr[i] = frag(par, i);
       // MFMA i, then the read of fragment i + kPrefetch.
       auto mfma = [&](int i, const f16x8& b, f32x16& acc) {
         acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[i], b, acc, 0, 0, 0);
-        if (i + kPrefetch < kNF) fr[i + kPrefetch] = frag(k1, i + kPrefetch);
+        if (i + kPrefetch < kNF) fr[i + kPrefetch] = frag(par, i + kPrefetch);
       };
       if constexpr (MK == kNoMask) {
         if (edge(t)) mask_step(t, cur);
@@ -1098,10 +1139,10 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   __syncthreads();
   if (active(0)) {
     if constexpr (HALF) {
-      sa[0] = qk(lds, hw);
+      sa[0] = qk(hw);
     } else {
-      sa[0] = qk(lds, 0);
-      sa[1] = qk(lds, 1);
+      sa[0] = qk(0);
+      sa[1] = qk(1);
     }
   }
   __syncthreads();  // step 0 overwrites K(0)
@@ -1111,8 +1152,8 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
       step_h(t, sa[0], sb[0]);
       if (t + 1 < n_tiles) step_h(t + 1, sb[0], sa[0]);
     } else {
-      step(t, sa, sb);
-      if (t + 1 < n_tiles) step(t + 1, sb, sa);
+      step(t, 0, sa, sb);
+      if (t + 1 < n_tiles) step(t + 1, 1, sb, sa);
     }
   }
   if constexpr (HALF) {
@@ -1121,6 +1162,7 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
     dma_wait();
     __syncthreads();  // every wavefront is done with the tiles
     constexpr int kRec = DM * 16 + 2;
+    static_assert(W / 2 * 64 * kRec * 4 <= sizeof(lds), "the records fit where the tiles were");
     float* rec = reinterpret_cast<float*>(lds) + ((wave >> 1) * 64 + lane) * kRec;
     if (hw == 1) {
 #pragma unroll
@@ -1645,21 +1687,41 @@ __global__ __launch_bounds__(256) void sdpa_split_merge_rows_kernel(MergeArgs a)
 
 int device_cus();
 
-// Key split of a call without the causal flag: splits enough that the
-// grid gives every compute unit a block, each split at least 8 steps (512
-// keys; shorter splits lose more to the merge pass than they gain) -- or,
-// when the unsplit grid would use at most an eighth of the compute units,
-// at least four steps (256 keys): such calls are bound by the latency of
-// each block's chain of steps more than by the merge (2 x 8 heads x 256
-// queries x 256 keys: 18.7 us split into 64-key runs, 15.6 unsplit or in
-// 256-key runs; 64 queries x 1024 keys: 12.7 split in 256-key runs, 14.3
-// unsplit).  Returns nsplit; split_keys is a multiple of 64.
-int plan_split(int64_t blocks, int Skv, int* split_keys) {
+// Key split of a call without the causal flag, given its grid of 256-row
+// blocks: splits enough that the grid gives every compute unit a block, each
+// of at least `least` keys, once the keys are worth the partials' round trip
+// through memory and the merge pass -- more keys, the nearer the unsplit grid
+// of 64- or 128-row blocks comes to filling the device.  Measured (32 / 8
+// heads, D 128, batch 1, us; the boundary's two sides):
+//  * blocks of at most 64 rows (decode, short runs of queries), which half
+//    steps cover whatever the grid: while the grid leaves units idle, past
+//    512 keys in runs of 256 up to 1/8 of the units (2 x 16 heads of D 64 x 40
+//    queries x 1100 keys: 11.9, runs of 512 13.3), beyond from 1024 in runs of
+//    512 (16 x 32 / 8 heads x 8 x 2100: unsplit 40.3, split 34.4);
+//  * up to 1/32 of the units (40 queries): past 512 keys, runs of 256 (512
+//    keys unsplit 10.6, split 12.2; 800: 13.6 and 12.9; 1600 in runs of 256
+//    14.6, of 512 17.0);
+//  * up to 1/8 (256 queries): from 1024, runs of 512 (800 keys unsplit 16.5,
+//    split 20.8; 1100: 21.0 and 21.2; 3200 in runs of 256 33.5, of 512 32.6);
+//  * up to 1/3 (512 queries): from 2048, runs of 768 (1600 keys unsplit 28.2,
+//    split 33.5; 2200: 37.0 and 36.7); D 64 from 1536 (2 x 16 heads x 300 x
+//    2000: 26.1 and 22.6);
+//  * up to 1/2 (900 queries): from 3072 (2000 keys unsplit 39.6, split 48.9;
+//    8000: 136.2 and 126.6; D 64, 2 x 16 heads x 900 x 4000: 49.7 and 44.8);
+//  * above, never (1280 x 1280 unsplit 38.9, split 51.0).
+// Returns nsplit; split_keys is a multiple of 64.
+int plan_split(int64_t blocks, int64_t rows, int Skv, int D, int* split_keys) {
   *split_keys = Skv;
   const int64_t cus = device_cus() > 0 ? device_cus() : 256;
-  const int min_keys = blocks * 8 <= cus ? 4 * kKT : 512;
-  if (blocks >= cus || Skv < 2 * min_keys) return 1;
-  const int64_t ns = std::min<int64_t>((cus + blocks - 1) / blocks, Skv / min_keys);
+  const bool few = rows <= 64;
+  const bool eighth = 8 * blocks <= cus;
+  const int from = 32 * blocks <= cus || (few && eighth) ? 513
+                   : few || eighth                      ? 1024
+                   : 3 * blocks <= cus                  ? (D == 64 ? 1536 : 2048)
+                                                        : 3072;
+  const int least = 32 * blocks <= cus || (few && eighth) ? 4 * kKT : few || eighth ? 512 : 768;
+  if ((few ? blocks >= cus : 2 * blocks > cus) || Skv < from) return 1;
+  const int64_t ns = std::min<int64_t>((cus + blocks - 1) / blocks, Skv / least);
   if (ns <= 1) return 1;
   const int64_t keys = ((Skv + ns - 1) / ns + kKT - 1) / kKT * kKT;
   *split_keys = static_cast<int>(keys);
@@ -1678,52 +1740,58 @@ int64_t blocks_for(int B, int Hkv, int g, int Sq, int pack, int rows = kQB) {
 
 // The workgroup an LDS-kernel call runs: W wavefronts, each a row tile of
 // its own (W x 32 rows), or two to a tile in half steps (W / 2 x 32 rows).
-//  k256  8 wavefronts, 256 rows, one workgroup per compute unit;
-//  k128  4 wavefronts, 128 rows, two per unit: half the rows of k256 waste
-//        less of a last round and of causal attention's uneven blocks, and
-//        the two of a unit do not wait for each other at barriers;
-//  kHalf8 8 wavefronts, 128 rows in half steps, K / V two steps ahead;
-//  kHalf4 4 wavefronts, 64 rows in half steps, two per unit: the shortest
-//        chain per block, for grids that leave units idle otherwise.
+//  k256   8 wavefronts, 256 rows, one workgroup per compute unit;
+//  k128   4 wavefronts, 128 rows, two per unit: half the rows of k256 waste
+//         less of a last round and of causal attention's uneven blocks, and
+//         the two of a unit do not wait for each other at barriers;
+//  kHalf8 8 wavefronts, 128 rows in half steps, without a mask K / V two
+//         steps ahead;
+//  kHalf4 4 wavefronts, 64 rows in half steps, two per unit (D 64: three):
+//         the shortest chain per block, for grids that leave units idle
+//         otherwise.
 enum Shape { k256, k128, kHalf8, kHalf4 };
 int shape_rows(Shape s) { return s == k256 ? 256 : s == kHalf4 ? 64 : 128; }
 
-// Which of them, for `groups` (sequence, q heads sharing rows, key split)
-// triples of `rows` rows over `keys` keys each.  Measured, prepared calls, one
-// box, 32 / 8 heads of D 128 at batch 1 unless said (k256 / kHalf8 / k128 /
+// Which of them, for `pairs` (sequence, q heads sharing rows) pairs of `rows`
+// rows over nsplit runs of `keys` keys (g: q heads per KV head).  Measured, prepared calls, one box,
+// 32 / 8 heads of D 128 at batch 1 unless said (k256 / k128 / kHalf8 /
 // kHalf4, us):
-//  * one step of keys: k128 (64 x 64: 7.1 / 7.1 / 6.5 / 7.0), the fold of
+//  * one step of keys: k128 (64 x 64: 6.5 / 6.5 / 7.1 / 6.9), the fold of
 //    half steps is not paid back;
-//  * else at most 64 rows: kHalf8 (16 queries x 8000 keys, B 4: 34.8 in
-//    kHalf8, 38.7 in k128, 37.9 in kHalf4);
-//  * a 64-row grid of one block per unit (causal, whose long and short
-//    blocks share units: two): kHalf4 (512 x 512: 20.8 / 16.8 / 15.5 / 14.1;
-//    causal 1000: 31.2 / 24.6 / 24.0 / 21.2).  Beyond it k128 is level or
-//    better (1000 x 1000: 32.2 / 27.3 / 25.7 / 25.7; 2048 causal: 56.4 / 52.0
-//    / 49.1 / 50.3; B 4 x 64 x 2000 keys: 28.1 / 36.8 / 27.8 / 32.9);
-//  * D 128, nearly whole rounds of 256-row blocks without more padding, and
-//    for causal attention at least 14 blocks a head, whose uneven lengths
-//    then even out: k256 (4096: 255.4 / 321 / 258.3 / 316; causal 8192: 513 /
-//    643 / 527 / 638; B 4 x 200 x 8000 keys: 124.3 / 159 / 129.2 / 176);
-//  * else k128 (1536: 69.3 / 73.2 / 60.7 / 71.3; 2500: 142.6 / 141.7 / 121.8 /
-//    129.6; causal 3072: 89.7 / 106.0 / 84.9 / 102.2; D 64, 4 x 16 heads x
-//    4096: 352 / 477 / 338 / 397).
-// A mask's blocks beside K and V leave room for one workgroup of any shape
-// per unit, except boolean masks at D 64 (k128, kHalf4) and fp16 masks at D
-// 64 (kHalf4): kHalf8 then while its grid is one block per unit (1000 x
-// 1000 with a causal boolean mask: 44.9 / 34.0 / 39.4 / 52.4), else k256.
-Shape pick_shape(int64_t groups, int64_t rows, int keys, int D, bool causal, int mask_kind) {
+//  * else at most 64 rows: kHalf8 (16 queries x 2000 keys, boolean mask, B 4:
+//    17.8 / 18.4 / 16.4 / 17.7);
+//  * a 64-row grid within one round of the device (causal and masked blocks,
+//    of uneven cost, two rounds; three at D 64): kHalf4 (512 x 512: 20.5 /
+//    15.0 / 16.3 / 13.6; causal 1000: 30.3 / 23.3 / 24.0 / 21.4; causal boolean
+//    mask 1000: 43.8 / 34.8 / 32.1 / 31.2; D 64, 8 x 16 heads x 384, padding
+//    mask: 16.1 / 16.1 / 21.1 / 14.7).  Past it k128 (1000 x 1000: 32.0 / 25.6
+//    / 27.1 / 25.5; B 4 x 640, padding mask: 56.4 / 47.8 / 58.3 / 49.9; causal
+//    4096: 142.9 / 141.7 / 190.7 / 188.1; 3072: 170.2 / 151.7 / 184.8 / 183.9),
+//    but k256 at D 128 where its grid is whole rounds of even blocks (4096 x
+//    4096: 251.8 / 253.7; 8192: 942 / 960; 5000, 2.5 rounds: 408.0 / 383.6),
+//    or causal of two rounds, where each long block is followed by its
+//    complement, and heads that share K and V, which then stay in the L2
+//    (4096: 132.2 / 136.1, with inputs from HBM 136.6 / 136.9; 16 / 8 heads x
+//    8192: 245.8 / 252.1; 32 heads of their own K and V: 187.7 / 172.2; B 2,
+//    four rounds: 274.1 / 267.8);
+//  * key splits, whose blocks are even and end in a store of their partials:
+//    kHalf4 within one round (64 queries x 2000 keys: 25.4 / 20.1 / 20.4 /
+//    17.3; beyond it, B 4: 30.3 / 29.9 / 37.8 / 35.6); at D 128 k256 when its
+//    grid is whole rounds (B 4 x 128 x 8000: 95.6 / 100.2 / 122 / 120; 15
+//    sixteenths of a round, B 1: 39.7 / 37.4 / 48.0 / 46.9) or a block has at
+//    most 128 rows (B 4 x 32 x 8000: 41.4 / 45.0 / 44.3 / 43.3; D 64: kHalf8,
+//    4 x 16 heads x 64 x 8000: 47.0 / 48.1 / 42.3 / 43.8); else k128.
+Shape pick_shape(int64_t pairs, int64_t rows, int g, int keys, int nsplit, int D, bool causal, bool masked) {
   const int64_t cus = device_cus() > 0 ? device_cus() : 256;
-  auto blocks = [&](int64_t r) { return groups * ((rows + r - 1) / r); };
-  const bool two_half = mask_kind == kNoMask || D == 64;        // two kHalf4 per unit
-  const bool two_full = two_half && mask_kind != kMaskF16;      // two k128 per unit
-  if (keys <= kKT && two_full) return k128;
+  auto blocks = [&](int64_t r) { return pairs * nsplit * ((rows + r - 1) / r); };
+  if (keys <= kKT) return k128;
   if (rows <= 64) return kHalf8;
-  if (two_half && blocks(64) <= (causal ? 2 : 1) * cus) return kHalf4;
-  if (!two_full) return blocks(128) <= cus ? kHalf8 : k256;
-  const int64_t n256 = blocks(256), rounds = (n256 + cus - 1) / cus;
-  const bool whole = n256 * 100 >= rounds * cus * 85 && blocks(128) * 100 >= n256 * 195;
-  return D == 128 && whole && (!causal || rows > 13 * 256) ? k256 : k128;
+  if (blocks(64) <= (nsplit > 1 ? 1 : D == 64 ? 3 : causal || masked ? 2 : 1) * cus) return kHalf4;
+  const bool whole = D == 128 && blocks(256) % cus == 0;
+  const bool paired = g > 1 && blocks(256) == 2 * cus && rows >= 14 * 256;
+  if (nsplit == 1) return whole && (!causal || paired) ? k256 : k128;
+  if (rows <= 128) return D == 128 ? k256 : kHalf8;
+  return whole ? k256 : k128;
 }
 
 // The grid of a call: short query runs pack all g q heads of a KV head into
@@ -1744,10 +1812,10 @@ struct GridPlan {
   Shape shape = k256;
 };
 
-// mask_kind: a staged or copied mask's; can_pack: its rows of a KV head's q
-// heads fit one buffer descriptor (else heads stay apart).
+// masked: a staged or copied mask; can_pack: its rows of a KV head's q heads
+// fit one buffer descriptor (else heads stay apart).
 GridPlan plan_grid(int B, int Hq, int Hkv, int Sq, int Skv, int D, bool causal, size_t ws_bytes,
-                   int mask_kind = kNoMask, bool can_pack = true) {
+                   bool masked = false, bool can_pack = true) {
   GridPlan gp;
   const int g = can_pack ? Hq / Hkv : 1;
   const int Hb = Hq / g;  // the (KV head, pack group) pairs of a sequence
@@ -1755,7 +1823,7 @@ GridPlan plan_grid(int B, int Hq, int Hkv, int Sq, int Skv, int D, bool causal, 
   // Short decode: one row tile (the g q heads of a KV head times Sq <= 32
   // rows) whose keys fit one block (kWaves2 slices), or a split of them
   // over blocks that all run in one round of the device.
-  if (!causal && mask_kind == kNoMask && Sq > 0 && static_cast<int64_t>(g) * Sq <= 32) {
+  if (!causal && !masked && Sq > 0 && static_cast<int64_t>(g) * Sq <= 32) {
     const int kw = D == 64 ? ShortLds<64>::kKW : ShortLds<128>::kKW;
     const int64_t cus = device_cus() > 0 ? device_cus() : 256;
     int waves = kWaves2;
@@ -1784,21 +1852,21 @@ GridPlan plan_grid(int B, int Hq, int Hkv, int Sq, int Skv, int D, bool causal, 
   if (!causal && Sq > 0) {
     const int p0 = Sq < kQB ? g : 1;
     int keys = Skv;
-    const int ns = plan_split(blocks_for(B, Hb, g, Sq, p0), Skv, &keys);
+    const int ns = plan_split(blocks_for(B, Hb, g, Sq, p0), static_cast<int64_t>(p0) * Sq, Skv, D, &keys);
     const size_t pb = split_bytes(static_cast<int64_t>(B) * Hq * Sq, ns, D);
     if (ns > 1 && ws_bytes >= pb) {
       gp.pack = p0;
       gp.nsplit = ns;
       gp.split_keys = keys;
       gp.part_bytes = pb;
-      gp.shape = pick_shape(static_cast<int64_t>(B) * Hb * (g / p0) * ns, static_cast<int64_t>(p0) * Sq, keys, D, causal,
-                            mask_kind);
+      gp.shape = pick_shape(static_cast<int64_t>(B) * Hb * (g / p0), static_cast<int64_t>(p0) * Sq, g, keys, ns, D,
+                            causal, masked);
       return gp;
     }
   }
   gp.pack = pack_heads(B, Hb, g, Sq);
-  gp.shape = pick_shape(static_cast<int64_t>(B) * Hb * (g / gp.pack), static_cast<int64_t>(gp.pack) * Sq, Skv, D, causal,
-                        mask_kind);
+  gp.shape = pick_shape(static_cast<int64_t>(B) * Hb * (g / gp.pack), static_cast<int64_t>(gp.pack) * Sq, g, Skv, 1, D,
+                        causal, masked);
   return gp;
 }
 
@@ -1962,8 +2030,8 @@ size_t copy_room(const MaskPlan& mp) {
 }
 
 // The grid of a staged or copied mask's call given ws_bytes beyond the copy.
-GridPlan masked_grid(const MaskPlan& mp, int kind, int B, int Hq, int Hkv, int Sq, int Skv, int D, size_t ws_bytes) {
-  return plan_grid(B, Hq, Hkv, Sq, Skv, D, false, ws_bytes, kind, mask_extent(mp, Hq / Hkv) <= kBufRange);
+GridPlan masked_grid(const MaskPlan& mp, int B, int Hq, int Hkv, int Sq, int Skv, int D, size_t ws_bytes) {
+  return plan_grid(B, Hq, Hkv, Sq, Skv, D, false, ws_bytes, true, mask_extent(mp, Hq / Hkv) <= kBufRange);
 }
 
 // Compute units of the current device, cached per device; 0 if the runtime
@@ -2016,7 +2084,7 @@ extern "C" size_t spyre_sdpa_fwd_call_workspace_bytes(const void* attn_mask, int
   if (!mask_strides || mask_kind < kNoMask || mask_kind > kMaskBool) return 0;
   const MaskPlan mp = plan_mask(attn_mask, mask_kind, mask_strides, B, Hq, Sq, Skv);
   if (mp.route == kRouteVt) return spyre_sdpa_fwd_workspace_bytes(B, Hkv, Skv, D);
-  const size_t part = masked_grid(mp, mask_kind, B, Hq, Hkv, Sq, Skv, D, SIZE_MAX).part_bytes;
+  const size_t part = masked_grid(mp, B, Hq, Hkv, Sq, Skv, D, SIZE_MAX).part_bytes;
   return part ? copy_room(mp) + part : mp.copy_bytes;
 }
 
@@ -2183,7 +2251,7 @@ extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const
     const size_t part_at = copy_room(mp);
     const size_t part_room = ws_room > part_at ? ws_room - part_at : 0;
     const GridPlan gpl = mask_kind == kNoMask ? plan_grid(B, Hq, Hkv, Sq, Skv, D, is_causal != 0, part_room)
-                                              : masked_grid(mp, mask_kind, B, Hq, Hkv, Sq, Skv, D, part_room);
+                                              : masked_grid(mp, B, Hq, Hkv, Sq, Skv, D, part_room);
     f2.pack = gpl.pack;
     f2.gp = fa.g / f2.pack;
     const int rows = shape_rows(gpl.shape);
