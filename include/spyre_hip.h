@@ -250,7 +250,7 @@ int spyre_paged_decode_attn_noalloc_f16(const void* q, const void* k_cache, cons
 
 /* Workspace bytes that cover any spyre_sdpa_fwd_f16 call with an attention
  * mask: V re-laid out with its sticks along tokens, B * Hkv * D *
- * ceil(Skv / 64) * 64 fp16, which the fp32-mask kernel reads.  Calls without
+ * ceil(Skv / 64) * 64 fp16, which the per-wavefront kernel reads.  Calls without
  * a mask (plain or causal) need no workspace. */
 size_t spyre_sdpa_fwd_workspace_bytes(int B, int Hkv, int Skv, int D);
 
@@ -271,9 +271,11 @@ size_t spyre_sdpa_fwd_workspace_bytes(int B, int Hkv, int Skv, int D);
  * bytes) for fp16 / bool masks other than those with key stride 1, a 16-byte
  * aligned pointer, b / h / i strides and Skv of whole 16 bytes (staged in
  * LDS beside K and V as they lie) a copy with 16-byte rows of the mask's
- * non-broadcast extent (then staged the same way); for fp32 masks, spyre_sdpa_fwd_workspace_bytes.  A
+ * non-broadcast extent (then staged the same way); for fp32 masks, the larger
+ * of a key split's partials and spyre_sdpa_fwd_workspace_bytes (which fp32
+ * masks whose keys are not contiguous use).  A
  * call whose fp16 / bool mask needs a copy but whose workspace holds only
- * spyre_sdpa_fwd_workspace_bytes runs the fp32-mask kernel instead (same
+ * spyre_sdpa_fwd_workspace_bytes runs the per-wavefront kernel instead (same
  * results within the SDPA tolerance, slower).  No reference counterpart:
  * the reference's decomposition (torch_spyre/_inductor/decompositions.py:
  * 523-609) allocates its intermediates itself. */

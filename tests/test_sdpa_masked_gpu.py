@@ -18,6 +18,10 @@ from tests.test_sdpa_gpu import LSE_ATOL, assert_close, randn
 
 pytestmark = pytest.mark.gpu
 
+DTYPE = {"f16": torch.float16, "f32": torch.float32}
+# fp32 masks keep q unscaled: fp32 scores and row sums
+LSE_BAR = {"f32": 1e-4}
+
 
 def make_mask(kind, shape, B, Hq, Sq, Skv, seed):
     """tail: query i sees keys up to Skv - Sq + i; pad: each sequence's own
@@ -33,11 +37,11 @@ def make_mask(kind, shape, B, Hq, Sq, Skv, seed):
         keep = torch.rand(dims, generator=g) > 0.3
         keep[..., 0] = True
         if kind != "bool":
-            return (torch.randn(dims, generator=g) * 2).to(torch.float16).masked_fill(~keep, -float("inf"))
+            return (torch.randn(dims, generator=g) * 2).to(DTYPE[kind]).masked_fill(~keep, -float("inf"))
     if kind == "bool":
         return keep
-    low = torch.finfo(torch.float16).min if shape == "pad" else -float("inf")
-    return torch.zeros(keep.shape, dtype=torch.float16).masked_fill_(~keep, low)
+    low = torch.finfo(DTYPE[kind]).min if shape == "pad" else -float("inf")
+    return torch.zeros(keep.shape, dtype=DTYPE[kind]).masked_fill_(~keep, low)
 
 
 # Rows per block: 4 (decode), 60, 128 (a whole half-step block), 132 (just
@@ -50,7 +54,7 @@ CASES = [(3, 8, 2, 1, 64, 128), (2, 32, 8, 1, 1000, 128), (1, 8, 8, 1, 2048, 64)
 
 
 @pytest.mark.parametrize("shape", ["tail", "pad", "bhqk", "1h1k"])
-@pytest.mark.parametrize("kind", ["bool", "f16"])
+@pytest.mark.parametrize("kind", ["bool", "f16", "f32"])
 @pytest.mark.parametrize("case", CASES, ids=str)
 def test_masked_grids(cuda, case, kind, shape):
     import torch_spyre_amd as tsa
@@ -63,10 +67,10 @@ def test_masked_grids(cuda, case, kind, shape):
                                                 enable_gqa=True, return_lse=True)
     assert_close(out, OA.sdpa_cpu_fp32(q, k, v, attn_mask=mask))
     _, lse64 = OA.sdpa_decomposition_fp64(q, k, v, attn_mask=mask.numpy(), return_lse=True)
-    assert np.allclose(lse.cpu().numpy(), lse64, atol=LSE_ATOL, rtol=0)
+    assert np.allclose(lse.cpu().numpy(), lse64, atol=LSE_BAR.get(kind, LSE_ATOL), rtol=0)
 
 
-@pytest.mark.parametrize("kind", ["bool", "f16"])
+@pytest.mark.parametrize("kind", ["bool", "f16", "f32"])
 @pytest.mark.parametrize("Sq,Skv", [(1, 2048), (40, 1536)])
 def test_masked_rows_and_splits(cuda, kind, Sq, Skv):
     """Rows with every key masked give zeros and LSE -inf beside live rows of
@@ -80,7 +84,7 @@ def test_masked_rows_and_splits(cuda, kind, Sq, Skv):
     keep = torch.ones((1, Hq, Sq, Skv), dtype=torch.bool)
     keep[:, 0, :, :-7] = False
     keep[:, 1] = False
-    mask = keep if kind == "bool" else torch.zeros(keep.shape, dtype=torch.float16).masked_fill_(~keep, -float("inf"))
+    mask = keep if kind == "bool" else torch.zeros(keep.shape, dtype=DTYPE[kind]).masked_fill_(~keep, -float("inf"))
     out, lse = tsa.scaled_dot_product_attention(q.to(cuda), k.to(cuda), v.to(cuda), attn_mask=mask.to(cuda),
                                                 enable_gqa=True, return_lse=True)
     assert not out[:, 1].float().abs().sum() and bool(torch.isneginf(lse[:, 1]).all())
@@ -88,7 +92,7 @@ def test_masked_rows_and_splits(cuda, kind, Sq, Skv):
     ref = OA.sdpa_cpu_fp32(q, k, v, attn_mask=mask)
     assert_close(out[:, live], ref[:, live])
     _, lse64 = OA.sdpa_decomposition_fp64(q, k, v, attn_mask=mask.numpy(), return_lse=True)
-    assert np.allclose(lse[:, live].cpu().numpy(), lse64[:, live], atol=LSE_ATOL, rtol=0)
+    assert np.allclose(lse[:, live].cpu().numpy(), lse64[:, live], atol=LSE_BAR.get(kind, LSE_ATOL), rtol=0)
 
 
 def test_masked_call_with_less_workspace(cuda):
@@ -122,7 +126,7 @@ SHAPES = [(1, 8, 8, 64, 64, False), (1, 8, 8, 64, 65, False), (1, 8, 8, 65, 200,
 
 
 @pytest.mark.parametrize("D", [64, 128])
-@pytest.mark.parametrize("kind", [None, "bool", "f16"])
+@pytest.mark.parametrize("kind", [None, "bool", "f16", "f32"])
 @pytest.mark.parametrize("case", SHAPES, ids=str)
 def test_workgroup_shapes(cuda, case, kind, D):
     import torch_spyre_amd as tsa
@@ -141,5 +145,44 @@ def test_workgroup_shapes(cuda, case, kind, D):
     assert_close(out[:, heads], OA.sdpa_cpu_fp32(qs, ks, vs, attn_mask=mask, is_causal=causal))
     _, lse64 = OA.sdpa_decomposition_fp64(qs, ks, vs, attn_mask=None if mask is None else mask.numpy(),
                                           is_causal=causal, return_lse=True)
-    assert np.allclose(lse[:, heads].cpu().numpy(), lse64, atol=LSE_ATOL, rtol=0)
+    assert np.allclose(lse[:, heads].cpu().numpy(), lse64, atol=LSE_BAR.get(kind, LSE_ATOL), rtol=0)
     assert not torch.isnan(out).any()
+
+
+@pytest.mark.parametrize("layout", ["rows", "odd_rows", "offset", "transposed", "key_broadcast"])
+@pytest.mark.parametrize("case", [(2, 8, 2, 20, 130, 64), (1, 4, 4, 97, 333, 128)], ids=str)
+def test_f32_mask_layouts(cuda, case, layout):
+    """An fp32 bias as rows of whole 16-byte units (loaded as such), as rows of
+    an odd number of floats and from an odd offset (loaded 4 bytes a lane, the
+    last row ending with the allocation), and with key strides other than 1
+    (the per-wavefront kernel): one answer."""
+    import torch_spyre_amd as tsa
+
+    B, Hq, Hkv, Sq, Skv, D = case
+    q = randn((B, Hq, Sq, D), SEED + 340)
+    k, v = randn((B, Hkv, Skv, D), SEED + 341), randn((B, Hkv, Skv, D), SEED + 342)
+    bias = torch.randn((Hq, Sq, Skv), generator=torch.Generator().manual_seed(SEED + 343))
+    if layout == "key_broadcast":
+        bias = bias[..., :1].expand(Hq, Sq, Skv)
+    n = bias.numel()
+    if layout == "rows":
+        wide = torch.zeros((Hq, Sq, (Skv + 7) // 4 * 4), device=cuda)
+        dev = wide[..., :Skv]
+        dev.copy_(bias)
+    elif layout == "odd_rows":
+        wide = torch.full((Hq, Sq, Skv + 1 + Skv % 2), float("nan"), device=cuda)
+        dev = wide[..., :Skv]
+        dev.copy_(bias)
+    elif layout == "offset":
+        flat = torch.empty(n + 1, device=cuda)
+        dev = flat[1:].view(Hq, Sq, Skv)
+        dev.copy_(bias)
+    elif layout == "transposed":
+        dev = bias.transpose(1, 2).contiguous().to(cuda).transpose(1, 2)
+    else:
+        dev = bias[..., :1].contiguous().to(cuda).expand(Hq, Sq, Skv)
+    out, lse = tsa.scaled_dot_product_attention(q.to(cuda), k.to(cuda), v.to(cuda), attn_mask=dev[None],
+                                                enable_gqa=True, return_lse=True)
+    assert_close(out, OA.sdpa_cpu_fp32(q, k, v, attn_mask=bias[None]))
+    _, lse64 = OA.sdpa_decomposition_fp64(q, k, v, attn_mask=bias[None].numpy(), return_lse=True)
+    assert np.allclose(lse.cpu().numpy(), lse64, atol=1e-4, rtol=0)

@@ -11,11 +11,12 @@
 // the reference's torch.softmax would give NaN there).
 //
 // Kernels, on the caller's stream:
-//  * sdpa_fwd_lds_kernel serves calls without a mask (plain or causal) and
-//    fp16 / boolean masks whose rows are whole 16-byte units.  A workgroup
+//  * sdpa_fwd_lds_kernel serves calls without a mask (plain or causal),
+//    fp16 / boolean masks whose rows are whole 16-byte units (others are
+//    copied first) and fp32 biases with contiguous keys.  A workgroup
 //    of 4 or 8 wavefronts takes 32 queries of one (sequence, q head) per
 //    wavefront or pair of wavefronts (pick_shape).  Per 64-key step the K and
-//    V tiles (row-major, padded) move from L2 straight into LDS (buffer loads
+//    V tiles (row-major, swizzled) move from L2 straight into LDS (buffer loads
 //    with the LDS flag), once for all its wavefronts:
 //       S^T[key, q] = K[key, :] Q^T[:, q]     2 x D/16 MFMA 32x32x16
 //       online softmax in fp32 (exp2 domain), lazy rescaling of the max;
@@ -24,7 +25,7 @@
 //    LDS reads.  The loop is software-pipelined: step t's softmax overlaps
 //    S(t+1).  A mask is staged per wavefront beside the tiles, a step ahead;
 //    steps it blanks for the whole wavefront skip their softmax and P V.
-//  * Other masks (fp32 biases, rows that are not whole 16-byte units):
+//  * Other masks (fp32 biases whose keys are not contiguous, slices of 2 GiB):
 //    1. v_token_sticks_kernel: V [B, Hkv, Skv, D] (rows may be strided) ->
 //       Vt [B, Hkv, D, S64] in the workspace: V with its sticks along tokens
 //       (the transpose-restick of each head), zero-padded to S64 = ceil(Skv
@@ -86,6 +87,11 @@ __device__ __forceinline__ short __attribute__((ext_vector_type(4))) tr_read4(co
 
 __device__ __forceinline__ void load_lds16(Rsrc r, _Float16* dst, uint32_t voff) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, voff, 0, 0, 0);
+}
+
+// The same with 4 bytes per lane (lane l writes dst + 4 l).
+__device__ __forceinline__ void load_lds4(Rsrc r, _Float16* dst, uint32_t voff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 4, voff, 0, 0, 0);
 }
 
 // Range of the buffer descriptors whose bases move with the key step; the
@@ -405,9 +411,10 @@ struct Fwd2Args {
   const _Float16* q;
   const _Float16* k;
   const _Float16* v;
-  const void* mask;          // fp16 bias or uint8 keep-mask, keys contiguous
+  const void* mask;          // fp16 / fp32 bias or uint8 keep-mask, keys contiguous
   int64_t m_sb, m_sh, m_sq;  // elements
   uint32_t m_bytes;          // extent of one block's `pack` q heads of the mask
+  int m_wide;                // fp32: rows of whole 16-byte units, loaded as such
   int64_t q_sb, q_sh, q_ss;
   int64_t k_sb, k_sh, k_ss;
   int64_t v_sb, v_sh, v_ss;
@@ -444,7 +451,8 @@ template <int ESZ, int KEYS> struct MaskRows {
   static constexpr int kLoads = 32 * kU / 64, kBytes = 32 * kU * 16;
   __device__ static __forceinline__ int swz(int row) { return (row / (16 / kU)) & (kU - 1); }
 };
-template <int MK, bool HALF> struct MaskTile : MaskRows<MK == kMaskF16 ? 2 : 1, HALF ? 32 : 64> {};
+template <int MK, bool HALF>
+struct MaskTile : MaskRows<MK == kMaskF32 ? 4 : MK == kMaskF16 ? 2 : 1, HALF ? 32 : 64> {};
 template <bool HALF> struct MaskTile<kNoMask, HALF> {
   static constexpr int kEsz = 1, kU = 1, kLoads = 0, kBytes = 0;
 };
@@ -464,6 +472,15 @@ template <bool HALF> struct MaskTile<kNoMask, HALF> {
 template <int D, bool PRESCALED, int MK, int SLOTS, bool HALF, int W>
 __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   static_assert(SLOTS == 2 || (SLOTS == 4 && MK == kNoMask), "four slots leave no room for a mask");
+  // fp32 biases: half steps only (the 32-query block of a full step, 8 KB a
+  // wavefront, leaves no room beside K and V), scores scaled and biased in
+  // fp32 (log2 units), row sums of the fp32 probabilities and a running max
+  // that follows every new one (a row's largest probability is then exactly
+  // 1 in fp16), as the per-wavefront kernel has them: the same error, 2.6e-4
+  // of fp64 at S 777, D 64 (2.9e-4 with the lazy max).
+  constexpr bool F32M = MK == kMaskF32;
+  constexpr float kLazy = F32M ? 0.f : 8.f;  // half steps: how far a score may pass the running max
+  static_assert(!F32M || (HALF && !PRESCALED), "fp32 biases: half steps, q as it is");
   using L = Lds2<D>;
   using MT = MaskTile<MK, HALF>;
   constexpr int DK = D / 16;  // QK k-steps
@@ -585,30 +602,53 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   // arrive as zeros.  Offsets are from the first of the block's `pack` q
   // heads (a row is a (query, head) pair); the descriptor's range ends with
   // the last of them.
-  uint32_t m_off[MT::kLoads > 0 ? MT::kLoads : 1];
+  // fp32 rows need not be whole 16-byte units (nor start on one): those are
+  // loaded 4 bytes a lane, two rows of 32 keys per load, whose range check
+  // is exact to the key.
+  constexpr int kNarrow = F32M ? 16 : 0;  // such loads
+  uint32_t m_off[kNarrow > 0 ? kNarrow : MT::kLoads > 0 ? MT::kLoads : 1];
   const char* mbase = nullptr;
   if constexpr (MK != kNoMask) {
     mbase = static_cast<const char*>(a.mask) + (b * a.m_sb + (kvh * a.g + gi * pack) * a.m_sh) * MT::kEsz;
-#pragma unroll
-    for (int j = 0; j < MT::kLoads; ++j) {
-      const int u = 64 * j + lane, row = u / MT::kU, ch = (u % MT::kU) ^ MT::swz(row);
-      // a valid row's offset lies below m_bytes < 2^31, so 32 bits of each product do
-      uint32_t mq = q0 + row, at = mq * static_cast<uint32_t>(a.m_sq);
+    const uint32_t m_sq = static_cast<uint32_t>(a.m_sq), m_sh = static_cast<uint32_t>(a.m_sh);
+    // Byte offset of the wavefront's row `row`, key 32 hw; kOob past Sq.  A
+    // valid row's offset lies below m_bytes < 2^31, so 32 bits of each product do.
+    auto row_off = [&](int row) -> uint32_t {
+      uint32_t mq = q0 + row, at = mq * m_sq;
       if (pack > 1) {
         mq = fdiv(q0 + row, a.by_pack);
-        at = mq * static_cast<uint32_t>(a.m_sq) + (q0 + row - mq * pack) * static_cast<uint32_t>(a.m_sh);
+        at = mq * m_sq + (q0 + row - mq * pack) * m_sh;
       }
-      const bool ok = static_cast<int>(mq) < a.Sq;
-      m_off[j] = ok ? (at + 32 * hw) * MT::kEsz + 16 * ch : kOob;
+      return static_cast<int>(mq) < a.Sq ? (at + 32 * hw) * MT::kEsz : kOob;
+    };
+    if (F32M && !a.m_wide) {
+#pragma unroll
+      for (int j = 0; j < kNarrow; ++j) {
+        const int row = 2 * j + half;
+        m_off[j] = row_off(row) + (((col >> 2) ^ MT::swz(row)) * 4 + (col & 3)) * 4;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < MT::kLoads; ++j) {
+        const int u = 64 * j + lane, row = u / MT::kU, ch = (u % MT::kU) ^ MT::swz(row);
+        m_off[j] = row_off(row) + 16 * ch;
+      }
     }
   }
-  auto mask_block = [&](int slot) { return lds + SLOTS * L::kSlot + ((kMaskSlots == 2 ? slot : 0) * W + wave) * (MT::kBytes / 2); };
+  auto mask_block = [&](int slot) {
+    return lds + SLOTS * L::kSlot + ((kMaskSlots == 2 ? slot : 0) * W + wave) * (MT::kBytes / 2);
+  };
   auto dma_m = [&](int kb, int slot) {
     if constexpr (MK != kNoMask) {
       const uint32_t done = static_cast<uint32_t>(kb) * MT::kEsz;  // < Skv esz <= m_bytes
       const Rsrc r = make_rsrc(reinterpret_cast<const _Float16*>(mbase + done), a.m_bytes - done);
+      if (F32M && !a.m_wide) {
 #pragma unroll
-      for (int j = 0; j < MT::kLoads; ++j) load_lds16(r, mask_block(slot) + 512 * j, m_off[j]);
+        for (int j = 0; j < kNarrow; ++j) load_lds4(r, mask_block(slot) + 128 * j, m_off[j]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < MT::kLoads; ++j) load_lds16(r, mask_block(slot) + 512 * j, m_off[j]);
+      }
     }
   };
   // The loads must have landed before the barrier that publishes them.
@@ -671,9 +711,10 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   // sends dropped scores to -inf.
   const float bias_mul = PRESCALED ? kLog2e : kLog2e / scale_abs;
   // This lane's byte of the block: row col, its first key's unit (fp16: unit
-  // `half`; boolean: byte 8 half of unit 0).
+  // `half`; fp32: unit 2 half; boolean: byte 8 half of unit 0).
   uint32_t m_lane = 0;
   if constexpr (MK == kMaskF16) m_lane = col * (16 * MT::kU) + ((half ^ MT::swz(col)) * 16);
+  if constexpr (F32M) m_lane = col * (16 * MT::kU) + (((2 * half) ^ MT::swz(col)) * 16);
   if constexpr (MK == kMaskBool) m_lane = col * (16 * MT::kU) + MT::swz(col) * 16 + 8 * half;
   // Half mt of the mask block (HALF: its one half, mt 0) onto S half s.
   auto apply_mask_half = [&](int t, int mt, f32x16& s) {
@@ -682,7 +723,12 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         // keys 32 mt + 16 (i / 2) + 8 half + 4 (i % 2) .. + 3 of row col
-        if constexpr (MK == kMaskF16) {
+        if constexpr (F32M) {
+          const uint32_t at = m_lane ^ (64 * (i >> 1) + 16 * (i & 1));
+          const f32x4 m4 = *reinterpret_cast<const f32x4*>(blk + at);
+#pragma unroll
+          for (int v = 0; v < 4; ++v) s[4 * i + v] = __builtin_fmaf(s[4 * i + v], scale_abs, m4[v] * kLog2e);
+        } else if constexpr (MK == kMaskF16) {
           const uint32_t at = (m_lane ^ (64 * mt + 32 * (i >> 1))) + 8 * (i & 1);
           const f16x4 m4 = *reinterpret_cast<const f16x4*>(blk + at);
 #pragma unroll
@@ -749,17 +795,18 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
     }
   };
   // P (fp16) of half mt; the row sum adds the same fp16 values the PV
-  // product uses.
+  // product uses (fp32 biases: the fp32 values).
   auto softmax_half = [&](const f32x16& s, float neg_m, f16x8 (&pb)[2]) {
     float psum = 0.f;
 #pragma unroll
     for (int rr = 0; rr < 16; ++rr) {
-      const float p = fast_exp2(PRESCALED ? s[rr] : __builtin_fmaf(s[rr], scale_abs, neg_m));  // masked: 0
-      const int i = rr >> 2;
+      const float p = fast_exp2(PRESCALED ? s[rr] : F32M ? s[rr] + neg_m : __builtin_fmaf(s[rr], scale_abs, neg_m));
+      const int i = rr >> 2;  // masked: 0
       pb[i >> 1][(i & 1) * 4 + (rr & 3)] = static_cast<_Float16>(p);
+      if constexpr (F32M) psum += p;
     }
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < 2 && !F32M; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         psum = __builtin_amdgcn_fdot2(f16x2{pb[j][2 * e], pb[j][2 * e + 1]}, f16x2{1, 1}, psum, false);
@@ -949,10 +996,10 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
       float mx = -INFINITY;
 #pragma unroll
       for (int rr = 0; rr < 16; ++rr) mx = fmaxf(mx, cur[rr]);
-      mx = PRESCALED ? max_xor32(mx) + m_use : max_xor32(mx) * scale_abs;
+      mx = PRESCALED ? max_xor32(mx) + m_use : max_xor32(mx) * (F32M ? 1.f : scale_abs);
       // A step the mask blanks for every real row adds nothing (see step).
       const bool live = MK == kNoMask || __builtin_amdgcn_ballot_w64(q_ok && mx > -INFINITY && mx >= m_run - 32.f) != 0;
-      if (live && __builtin_amdgcn_ballot_w64(mx > m_run + 8.f) != 0) {
+      if (live && __builtin_amdgcn_ballot_w64(mx > m_run + kLazy) != 0) {
         const float m_new = fmaxf(m_run, mx);
         const float alpha = m_new == -INFINITY ? 1.f : fast_exp2(m_run - m_new);
         l_run *= alpha;
@@ -1781,12 +1828,13 @@ int shape_rows(Shape s) { return s == k256 ? 256 : s == kHalf4 ? 64 : 128; }
 //    sixteenths of a round, B 1: 39.7 / 37.4 / 48.0 / 46.9) or a block has at
 //    most 128 rows (B 4 x 32 x 8000: 41.4 / 45.0 / 44.3 / 43.3; D 64: kHalf8,
 //    4 x 16 heads x 64 x 8000: 47.0 / 48.1 / 42.3 / 43.8); else k128.
-Shape pick_shape(int64_t pairs, int64_t rows, int g, int keys, int nsplit, int D, bool causal, bool masked) {
+Shape pick_shape(int64_t pairs, int64_t rows, int g, int keys, int nsplit, int D, bool causal, int mask_kind) {
   const int64_t cus = device_cus() > 0 ? device_cus() : 256;
   auto blocks = [&](int64_t r) { return pairs * nsplit * ((rows + r - 1) / r); };
+  if (mask_kind == kMaskF32) return rows <= 64 ? kHalf8 : kHalf4;  // the kernel's two
   if (keys <= kKT) return k128;
   if (rows <= 64) return kHalf8;
-  if (blocks(64) <= (nsplit > 1 ? 1 : D == 64 ? 3 : causal || masked ? 2 : 1) * cus) return kHalf4;
+  if (blocks(64) <= (nsplit > 1 ? 1 : D == 64 ? 3 : causal || mask_kind != kNoMask ? 2 : 1) * cus) return kHalf4;
   const bool whole = D == 128 && blocks(256) % cus == 0;
   const bool paired = g > 1 && blocks(256) == 2 * cus && rows >= 14 * 256;
   if (nsplit == 1) return whole && (!causal || paired) ? k256 : k128;
@@ -1812,10 +1860,11 @@ struct GridPlan {
   Shape shape = k256;
 };
 
-// masked: a staged or copied mask; can_pack: its rows of a KV head's q heads
+// mask_kind: a staged or copied mask's; can_pack: its rows of a KV head's q heads
 // fit one buffer descriptor (else heads stay apart).
 GridPlan plan_grid(int B, int Hq, int Hkv, int Sq, int Skv, int D, bool causal, size_t ws_bytes,
-                   bool masked = false, bool can_pack = true) {
+                   int mask_kind = kNoMask, bool can_pack = true) {
+  const bool masked = mask_kind != kNoMask;
   GridPlan gp;
   const int g = can_pack ? Hq / Hkv : 1;
   const int Hb = Hq / g;  // the (KV head, pack group) pairs of a sequence
@@ -1860,13 +1909,13 @@ GridPlan plan_grid(int B, int Hq, int Hkv, int Sq, int Skv, int D, bool causal, 
       gp.split_keys = keys;
       gp.part_bytes = pb;
       gp.shape = pick_shape(static_cast<int64_t>(B) * Hb * (g / p0), static_cast<int64_t>(p0) * Sq, g, keys, ns, D,
-                            causal, masked);
+                            causal, mask_kind);
       return gp;
     }
   }
   gp.pack = pack_heads(B, Hb, g, Sq);
   gp.shape = pick_shape(static_cast<int64_t>(B) * Hb * (g / gp.pack), static_cast<int64_t>(gp.pack) * Sq, g, Skv, 1, D,
-                        causal, masked);
+                        causal, mask_kind);
   return gp;
 }
 
@@ -1912,6 +1961,15 @@ void launch_lds(const Fwd2Args& f2, int D, bool prescaled, hipStream_t st) {
     sdpa_fwd_lds_kernel<64, true, MK, SLOTS, HALF, W><<<grid, W * 64, 0, st>>>(f2);
   else
     sdpa_fwd_lds_kernel<64, false, MK, SLOTS, HALF, W><<<grid, W * 64, 0, st>>>(f2);
+}
+
+template <int W>
+void launch_f32(const Fwd2Args& f2, int D, hipStream_t st) {
+  const dim3 grid(f2.n_items);
+  if (D == 128)
+    sdpa_fwd_lds_kernel<128, false, kMaskF32, 2, true, W><<<grid, W * 64, 0, st>>>(f2);
+  else
+    sdpa_fwd_lds_kernel<64, false, kMaskF32, 2, true, W><<<grid, W * 64, 0, st>>>(f2);
 }
 
 // A copy of a mask with 16-byte rows: [bm][hm][qm][pitch bytes], keys past
@@ -1964,9 +2022,13 @@ bool aligned16(const void* p);
 //                stages it as it lies;
 //  kRouteCopied  other fp16 / bool masks: copied with 16-byte rows into the
 //                workspace first (mask_pad_kernel), then staged;
-//  kRouteVt      fp32 masks (or a copy whose slice would pass 2 GiB): the
+//  kRouteF32     fp32 with key stride 1: the main kernel in half steps
+//                (position bias [1, 16, 777, 777], B 2, D 64: 59.3 us by
+//                kRouteVt, 22.9 here; [1, 32, 2048, 2048], 32 / 8 heads, D 128:
+//                489 and 192; one query x 2000 keys: 213 and 14.7);
+//  kRouteVt      other fp32 masks (or a slice, or a copy's, past 2 GiB): the
 //                per-wavefront kernel, V through the workspace.
-enum MaskRoute { kRouteNone, kRouteStaged, kRouteCopied, kRouteVt };
+enum MaskRoute { kRouteNone, kRouteStaged, kRouteCopied, kRouteF32, kRouteVt };
 
 struct MaskPlan {
   MaskRoute route = kRouteNone;
@@ -1975,13 +2037,20 @@ struct MaskPlan {
   int64_t span = 0;                      // bytes of one (sequence, head) slice as staged
   int64_t bm = 1, hm = 1, qm = 1, pitch = 0;  // kRouteCopied: extents kept, row pitch (bytes)
   size_t copy_bytes = 0;
+  bool wide = false;                     // kRouteF32: slices of whole 16-byte units
 };
 
 MaskPlan plan_mask(const void* mask, int kind, const int64_t* ms, int B, int Hq, int Sq, int Skv) {
   MaskPlan p;
   if (kind == kNoMask) return p;
   if (kind == kMaskF32) {
-    p.route = kRouteVt;
+    p.esz = 4;
+    p.sb = ms[0];
+    p.sh = ms[1];
+    p.sq = ms[2];
+    p.span = Sq > 0 && Skv > 0 ? ((static_cast<int64_t>(Sq) - 1) * ms[2] + Skv) * 4 : 0;
+    p.route = ms[3] == 1 && p.span <= kBufRange ? kRouteF32 : kRouteVt;
+    p.wide = aligned16(mask) && ms[0] % 4 == 0 && ms[1] % 4 == 0 && ms[2] % 4 == 0 && Skv % 4 == 0;
     return p;
   }
   const int64_t esz = p.esz = kind == kMaskF16 ? 2 : 1;
@@ -2030,8 +2099,8 @@ size_t copy_room(const MaskPlan& mp) {
 }
 
 // The grid of a staged or copied mask's call given ws_bytes beyond the copy.
-GridPlan masked_grid(const MaskPlan& mp, int B, int Hq, int Hkv, int Sq, int Skv, int D, size_t ws_bytes) {
-  return plan_grid(B, Hq, Hkv, Sq, Skv, D, false, ws_bytes, true, mask_extent(mp, Hq / Hkv) <= kBufRange);
+GridPlan masked_grid(const MaskPlan& mp, int kind, int B, int Hq, int Hkv, int Sq, int Skv, int D, size_t ws_bytes) {
+  return plan_grid(B, Hq, Hkv, Sq, Skv, D, false, ws_bytes, kind, mask_extent(mp, Hq / Hkv) <= kBufRange);
 }
 
 // Compute units of the current device, cached per device; 0 if the runtime
@@ -2084,7 +2153,8 @@ extern "C" size_t spyre_sdpa_fwd_call_workspace_bytes(const void* attn_mask, int
   if (!mask_strides || mask_kind < kNoMask || mask_kind > kMaskBool) return 0;
   const MaskPlan mp = plan_mask(attn_mask, mask_kind, mask_strides, B, Hq, Sq, Skv);
   if (mp.route == kRouteVt) return spyre_sdpa_fwd_workspace_bytes(B, Hkv, Skv, D);
-  const size_t part = masked_grid(mp, B, Hq, Hkv, Sq, Skv, D, SIZE_MAX).part_bytes;
+  const size_t part = masked_grid(mp, mask_kind, B, Hq, Hkv, Sq, Skv, D, SIZE_MAX).part_bytes;
+  if (mp.route == kRouteF32) return std::max(part, spyre_sdpa_fwd_workspace_bytes(B, Hkv, Skv, D));
   return part ? copy_room(mp) + part : mp.copy_bytes;
 }
 
@@ -2140,7 +2210,8 @@ extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const
   MaskPlan mp = plan_mask(attn_mask, mask_kind, mask_strides, B, Hq, Sq, Skv);
   if (mp.route == kRouteCopied && (!workspace || workspace_bytes < mp.copy_bytes || !aligned16(workspace)))
     mp.route = kRouteVt;
-  const size_t need = mp.route == kRouteVt       ? spyre_sdpa_fwd_workspace_bytes(B, Hkv, Skv, D)
+  // (fp32 masks ask for V's relayout whichever kernel runs.)
+  const size_t need = mp.route >= kRouteF32      ? spyre_sdpa_fwd_workspace_bytes(B, Hkv, Skv, D)
                       : mp.route == kRouteCopied ? mp.copy_bytes
                                                  : 0;
   SPYRE_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && aligned16(workspace)),
@@ -2251,7 +2322,7 @@ extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const
     const size_t part_at = copy_room(mp);
     const size_t part_room = ws_room > part_at ? ws_room - part_at : 0;
     const GridPlan gpl = mask_kind == kNoMask ? plan_grid(B, Hq, Hkv, Sq, Skv, D, is_causal != 0, part_room)
-                                              : masked_grid(mp, B, Hq, Hkv, Sq, Skv, D, part_room);
+                                              : masked_grid(mp, mask_kind, B, Hq, Hkv, Sq, Skv, D, part_room);
     f2.pack = gpl.pack;
     f2.gp = fa.g / f2.pack;
     const int rows = shape_rows(gpl.shape);
@@ -2276,6 +2347,7 @@ extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const
     f2.m_sh = mp.sh;
     f2.m_sq = mp.sq;
     f2.m_bytes = static_cast<uint32_t>(mask_extent(mp, f2.pack));
+    f2.m_wide = mp.wide ? 1 : 0;
     if (gpl.short_decode) {
       // One row tile, its keys all in flight at once; a key split merges in
       // the same kernel.
@@ -2291,7 +2363,9 @@ extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const
           default: launch_lds<MK, 2, true, 4>(f2, D, prescaled, st); break;
         }
       };
-      if (mask_kind == kMaskF16) go(std::integral_constant<int, kMaskF16>{});
+      if (mask_kind == kMaskF32) {
+        gpl.shape == kHalf8 ? launch_f32<8>(f2, D, st) : launch_f32<4>(f2, D, st);
+      } else if (mask_kind == kMaskF16) go(std::integral_constant<int, kMaskF16>{});
       else if (mask_kind == kMaskBool) go(std::integral_constant<int, kMaskBool>{});
       else go(std::integral_constant<int, kNoMask>{});
     }

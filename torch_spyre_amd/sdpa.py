@@ -91,8 +91,8 @@ def _geometry_plan(q, k, v, mask, kind: int, is_causal: bool):
     mstrides = _lib.i64_array(mask.stride()) if mask is not None else None
     # The call's workspace: a key split's partials when the blocks would not
     # fill the device (none for causal calls), a copy with 16-byte rows of
-    # fp16 / bool masks the kernel cannot stage as they lie, V's relayout for
-    # fp32 masks.
+    # fp16 / bool masks the kernel cannot stage as they lie, room for V's
+    # relayout for fp32 masks.
     need = 0
     if kind != MASK_NONE or not is_causal:
         need = int(_lib.lib().spyre_sdpa_fwd_call_workspace_bytes(
