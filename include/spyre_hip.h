@@ -141,6 +141,16 @@ int spyre_kv_append_f16(const void* k_new, const void* v_new, void* k_cache, voi
                         const int32_t* positions, int B, int Hkv, int D, int page_size,
                         int64_t num_pages, void* stream);
 
+/* Dense K / V [B, Hkv, S, D] into the paged cache's page layouts: sequence
+ * b's page p becomes page b * P + p of k_pages [B P, Hkv, D/64, 64, 64] and
+ * v_pages [B P, Hkv, D, 64], P = max(1, ceil(S / 64)); tokens past S are
+ * zeros.  16-bit elements with feature stride 1, the other strides ({b, h,
+ * s}, elements) multiples of 8, 16-byte aligned pointers; D a multiple of
+ * 64.  No reference counterpart. */
+int spyre_dense_to_pages_f16(const void* k, const int64_t* k_strides, const void* v,
+                             const int64_t* v_strides, void* k_pages, void* v_pages, int B, int Hkv,
+                             int S, int D, void* stream);
+
 /* Workspace bytes needed by spyre_paged_decode_attn_f16: fp32 chunk
  * partials, B * Hkv * ceil(max_context_len / (8 * split_tokens)) * g * (D + 2)
  * floats, then a 4-byte arrival flag per (sequence, KV head, chunk).  The

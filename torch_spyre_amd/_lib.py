@@ -72,6 +72,8 @@ SIGNATURES = {
                                    POINTER(c_int64), POINTER(c_int64), c_int, POINTER(StrideInfo)]),
     "spyre_dma_copy": (c_int, [c_void_p, c_size_t, c_void_p, c_size_t, c_int, POINTER(StrideInfo),
                                c_int, c_void_p]),
+    "spyre_dense_to_pages_f16": (c_int, [c_void_p, POINTER(c_int64), c_void_p, POINTER(c_int64), c_void_p, c_void_p,
+                                         c_int, c_int, c_int, c_int, c_void_p]),
     "spyre_kv_append_f16": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64,
                                     c_void_p, c_int, c_int, c_int, c_int, c_int64, c_void_p]),
     "spyre_paged_decode_attn_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int]),

@@ -24,7 +24,7 @@ from typing import Optional
 import torch
 
 from . import _lib
-from .layout import DataFormats, SpyreTensorLayout
+from .layout import DataFormats, SpyreTensorLayout, get_device_dtype
 from .relayout import _require_cuda, _require_on, _stream_ptr, h2d_buffer
 
 PAGE = 64
@@ -303,14 +303,43 @@ def paged_decode_merge(context_lens: torch.Tensor, workspace: torch.Tensor, out:
     return out
 
 
+def _pages_kernel_takes(k: torch.Tensor, v: torch.Tensor) -> bool:
+    plain = (torch.Tensor, torch.nn.Parameter)
+    return (type(k) in plain and type(v) in plain and k.is_cuda and k.device == v.device and k.dtype == v.dtype
+            and k.dtype in (torch.float16, torch.bfloat16) and get_device_dtype(k.dtype) == DataFormats.SEN169_FP16
+            and k.shape == v.shape and k.shape[1] > 0 and k.shape[3] > 0 and k.shape[3] % 64 == 0)
+
+
+def _pages_operand(t: torch.Tensor) -> torch.Tensor:
+    """t with rows the pages kernel reads as 16-byte vectors: feature stride
+    1, other strides multiples of 8, 16-byte aligned; else a copy."""
+    st = t.stride()
+    ready = st[3] == 1 and all(x % 8 == 0 for x in st[:3]) and t.data_ptr() % 16 == 0
+    return t if ready else t.clone(memory_format=torch.contiguous_format)
+
+
 def dense_to_pages(k: torch.Tensor, v: torch.Tensor) -> tuple[PagedKVCache, torch.Tensor]:
     """Dense K/V [B, Hkv, S, D] -> paged cache (sequence b's page p is page
-    b*P + p) and its block table.  Each tensor is moved in one relayout pass:
-    the strided view [B, P, Hkv, 64, D] of the dense tensor is laid out with
-    the page layouts (K keeps its sticks on D, V is transpose-resticked onto
-    tokens).  Tokens past S are zero."""
+    b*P + p) and its block table; tokens past S are zero.  16-bit tensors
+    with D a multiple of 64 are moved by one kernel, K and V together
+    (spyre_dense_to_pages_f16); anything else is padded and moved in one
+    relayout pass per tensor: the strided view [B, P, Hkv, 64, D] of the dense
+    tensor laid out with the page layouts (K keeps its sticks on D, V is
+    transpose-resticked onto tokens)."""
     B, Hkv, S, D = k.shape
     P = max(1, (S + PAGE - 1) // PAGE)
+    if _pages_kernel_takes(k, v):
+        kr, vr = _pages_operand(k), _pages_operand(v)
+        cache = PagedKVCache.__new__(PagedKVCache)
+        cache.num_pages, cache.Hkv, cache.D = B * P, Hkv, D
+        cache.k_layout = k_page_layout(B * P, Hkv, D)
+        cache.v_layout = v_page_layout(B * P, Hkv, D)
+        cache.k = torch.empty((B * P, Hkv, D // 64, PAGE, 64), dtype=k.dtype, device=k.device)
+        cache.v = torch.empty((B * P, Hkv, D, PAGE), dtype=k.dtype, device=k.device)
+        _lib.check("spyre_dense_to_pages_f16", _lib.lib().spyre_dense_to_pages_f16(
+            kr.data_ptr(), _lib.i64_array(kr.stride()[:3]), vr.data_ptr(), _lib.i64_array(vr.stride()[:3]),
+            cache.k.data_ptr(), cache.v.data_ptr(), B, Hkv, S, D, _stream_ptr(k.device)))
+        return cache, torch.arange(B * P, dtype=torch.int32, device=k.device).view(B, P)
     S2 = P * PAGE
     if S2 != S:
         k = torch.nn.functional.pad(k, (0, 0, 0, S2 - S))
