@@ -276,7 +276,9 @@ size_t spyre_sdpa_fwd_workspace_bytes(int B, int Hkv, int Skv, int D);
  * grid fills at least half the device: when a sequence spans several
  * chunks, their fp32 partials B * Hkv * chunks * g * (D + 2) * 4 bytes and a
  * 4-byte arrival flag per (sequence, KV head, chunk), also without
- * initialisation (the chunks merge in the one kernel).  With a mask: a key
+ * initialisation (the chunks merge in the one kernel).  With a mask:
+ * decode partials as above, where the mask's keys are contiguous (read as it
+ * lies; the call still asks for the room named below); else a key
  * split's partials as above, and before them (its size rounded up to 256
  * bytes) for fp16 / bool masks other than those with key stride 1, a 16-byte
  * aligned pointer, b / h / i strides and Skv of whole 16 bytes (staged in

@@ -186,3 +186,77 @@ def test_f32_mask_layouts(cuda, case, layout):
     assert_close(out, OA.sdpa_cpu_fp32(q, k, v, attn_mask=bias[None]))
     _, lse64 = OA.sdpa_decomposition_fp64(q, k, v, attn_mask=bias[None].numpy(), return_lse=True)
     assert np.allclose(lse.cpu().numpy(), lse64, atol=1e-4, rtol=0)
+
+
+# Decode that reads its mask as it lies.  Short-decode kernel: one block with
+# ragged and empty slices (1, 31, 33, 300 keys), splits of eight- and of
+# four-wavefront blocks, several queries per head.  Split-KV decode kernels:
+# one run and several, a ragged last run read as a window, one chunk and
+# chunks merged in the kernel and by the merge pass, four-wavefront items.
+DECODE = [(2, 8, 2, 1, 1, 128), (3, 4, 4, 1, 31, 64), (1, 8, 2, 3, 33, 128), (1, 8, 8, 4, 300, 64),
+          (1, 32, 8, 1, 1500, 128), (2, 16, 2, 2, 2100, 64), (40, 32, 8, 1, 64, 128), (40, 8, 8, 1, 200, 64),
+          (16, 32, 8, 1, 2047, 128), (4, 64, 8, 1, 9000, 128), (24, 32, 8, 1, 5000, 128), (8, 32, 8, 1, 1111, 64)]
+
+
+@pytest.mark.parametrize("shape", ["tail", "pad", "bhqk", "1h1k", "holes"])
+@pytest.mark.parametrize("kind", ["bool", "f16", "f32"])
+@pytest.mark.parametrize("case", DECODE, ids=str)
+def test_masked_decode(cuda, case, kind, shape):
+    """holes: whole 64-key runs masked (skipped) in the middle and at both
+    ends of a sequence, and one sequence masked altogether (zeros, LSE -inf)."""
+    import torch_spyre_amd as tsa
+
+    B, Hq, Hkv, Sq, Skv, D = case
+    q = randn((B, Hq, Sq, D), SEED + 350)
+    k, v = randn((B, Hkv, Skv, D), SEED + 351), randn((B, Hkv, Skv, D), SEED + 352)
+    dead = []
+    if shape == "holes":
+        keep = torch.rand((B, 1, 1, (Skv + 63) // 64), generator=torch.Generator().manual_seed(SEED + 353)) > 0.5
+        keep = keep.repeat_interleave(64, dim=3)[..., :Skv].clone()
+        keep[:, :, :, Skv // 2] = True
+        keep[B - 1] = False
+        dead = [B - 1]
+        mask = keep if kind == "bool" else torch.zeros(keep.shape, dtype=DTYPE[kind]).masked_fill_(~keep, -float("inf"))
+    else:
+        mask = make_mask(kind, shape, B, Hq, Sq, Skv, SEED + 354 + Skv)
+    out, lse = tsa.scaled_dot_product_attention(q.to(cuda), k.to(cuda), v.to(cuda), attn_mask=mask.to(cuda),
+                                                enable_gqa=True, return_lse=True)
+    live = [b for b in range(B) if b not in dead]
+    for b in dead:
+        assert not out[b].float().abs().sum() and bool(torch.isneginf(lse[b]).all())
+    if not live:
+        return
+    m = mask[live] if mask.dim() == 4 and mask.shape[0] == B else mask
+    ref = OA.sdpa_cpu_fp32(q[live], k[live], v[live], attn_mask=m)
+    assert_close(out[live], ref)
+    some = live[:3]  # fp64 on a few sequences
+    m = mask[some] if mask.dim() == 4 and mask.shape[0] == B else mask
+    _, lse64 = OA.sdpa_decomposition_fp64(q[some], k[some], v[some], attn_mask=m.numpy(), return_lse=True)
+    assert np.allclose(lse[some].cpu().numpy(), lse64, atol=1e-4, rtol=0)
+
+
+@pytest.mark.parametrize("case", [(1, 8, 2, 1, 300, 128), (16, 32, 8, 1, 1000, 128)], ids=str)
+def test_masked_decode_reads_inside_the_mask(cuda, case):
+    """The mask ends with its allocation's last bytes, at an odd address, and
+    K / V rows past a padded sequence's end hold NaN: neither is read past."""
+    import torch_spyre_amd as tsa
+
+    B, Hq, Hkv, Sq, Skv, D = case
+    q = randn((B, Hq, Sq, D), SEED + 360)
+    k, v = randn((B, Hkv, Skv, D), SEED + 361), randn((B, Hkv, Skv, D), SEED + 362)
+    lens = torch.linspace(70, Skv, B).long() if B > 1 else torch.tensor([Skv])
+    keep = (torch.arange(Skv)[None] < lens[:, None])[:, None, None]
+    flat = torch.empty(B * Skv + 3, dtype=torch.bool, device=cuda)
+    mask = flat[3:].view(keep.shape)
+    mask.copy_(keep.to(cuda))
+    kn, vn = k.clone(), v.clone()
+    for b in range(B):  # whole 64-key runs past the end
+        first = (int(lens[b]) + 127) // 64 * 64
+        kn[b, :, first:], vn[b, :, first:] = float("nan"), float("nan")
+    if B == 1:
+        kn, vn = k, v
+    last = Skv % 64  # a ragged last run is read as the 64 keys ending with the last one
+    if B > 1 and last:
+        kn[:, :, Skv - 64 - 64:], vn[:, :, Skv - 64 - 64:] = k[:, :, Skv - 64 - 64:], v[:, :, Skv - 64 - 64:]
+    out = tsa.scaled_dot_product_attention(q.to(cuda), kn.to(cuda), vn.to(cuda), attn_mask=mask, enable_gqa=True)
+    assert_close(out, OA.sdpa_cpu_fp32(q, k, v, attn_mask=keep))

@@ -55,6 +55,8 @@
 
 namespace {
 
+using namespace spyre_hip;
+
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -104,6 +106,10 @@ struct SplitArgs {
   // (run_item, merge_in_kernel), their flags after the partials in ws.
   // 0: the merge pass combines them.
   uint32_t ticket;
+  // Dense K / V with a mask (DecodeMask kinds): element (b, h, t) at b m_sb +
+  // h m_sh + t, any alignment.
+  const void* mask;
+  int64_t m_sb, m_sh;
 };
 
 // Pages of a context and the number of chunks (of at most chunk_pages
@@ -326,6 +332,26 @@ __device__ __forceinline__ void load_v(f16x8 (&va)[D / 16][2], Rsrc vr, const Lo
   }
 }
 
+// Mask elements of the dense kernels (DecodeMask kinds) and the 16-byte
+// piece one lane of the live-run scan reads.
+template <int MK> struct DenseMask { using T = uint8_t; };
+template <> struct DenseMask<kDecodeMaskF16> { using T = _Float16; };
+template <> struct DenseMask<kDecodeMaskF32> { using T = float; };
+
+template <int MK>
+__device__ __forceinline__ bool mask_keeps(typename DenseMask<MK>::T x) {
+  if constexpr (MK == kDecodeMaskBool)
+    return x != 0;
+  else
+    return static_cast<float>(x) > -INFINITY;
+}
+
+// N consecutive mask elements at any alignment.
+template <int MK, int N>
+__device__ __forceinline__ void load_mask(const typename DenseMask<MK>::T* p, typename DenseMask<MK>::T (&x)[N]) {
+  __builtin_memcpy(x, p, sizeof(x));
+}
+
 // Pages [p0, p0 + n_it) of sequence b, KV head kvh (context ctx tokens),
 // streamed by one wavefront: the pages rotate through the operand registers
 // (the next page's K loads are issued as soon as this page's QK MFMAs have
@@ -336,7 +362,11 @@ __device__ __forceinline__ void load_v(f16x8 (&va)[D / 16][2], Rsrc vr, const Lo
 // DENSE: "pages" are 64-token runs of dense K / V (SplitArgs' dense
 // strides); lane (col, grp) then holds O^T[d][col] in o[db][v] for d the
 // feature of PV row i = 4 grp + v of MFMA db (load_v_dense).
-template <int D, bool DENSE = false>
+// MK (dense, ctx >= 64): the mask's kind.  The wavefront first scans its own
+// share of the mask (one load for up to 16 runs of a boolean row that every
+// head shares) and streams only the runs that keep a token: a padded
+// sequence's K and V past its end are not read.
+template <int D, bool DENSE = false, int MK = kDecodeNoMask>
 __device__ __forceinline__ void stream_pages(const SplitArgs& a, int b, int kvh, int p0, int n_it,
                                              int ctx, int lane, f32x4 (&o)[D / 16], float& m_out,
                                              float& l_out) {
@@ -426,6 +456,48 @@ __device__ __forceinline__ void stream_pages(const SplitArgs& a, int b, int kvh,
   // them; rotating measured slower there).
   const int rot = DENSE && n_it > 1 ? static_cast<int>((static_cast<uint32_t>(b) * a.Hkv + kvh + p0 / n_it) % n_it) : 0;
   auto run_of = [&](int it) { return it + rot < n_it ? it + rot : it + rot - n_it; };
+  // The runs streamed, in order: next_run(i) is the i-th (called for i = 0,
+  // 1, ... once each).  With a mask, those that keep a token of some head.
+  using MT = typename DenseMask<MK>::T;
+  const MT* mrow = nullptr;  // this lane's mask row (head col; padded heads read head 0's)
+  int n_run = n_it;
+  uint64_t live_hi = 0, live_lo = 0;  // runs from rot on, and before it
+  if constexpr (MK != kDecodeNoMask) {
+    const MT* m0 = static_cast<const MT*>(a.mask) + b * a.m_sb + static_cast<int64_t>(kvh) * a.g * a.m_sh;
+    mrow = m0 + (col < a.g ? col : 0) * a.m_sh;
+    uint64_t live = ~uint64_t{0};
+    if (n_it <= 64) {
+      constexpr int kPiece = 16 / sizeof(MT), kPerRun = kPage / kPiece;  // tokens a lane reads; lanes per run
+      live = 0;
+      const int end = min(ctx, (p0 + n_it) * kPage);
+      for (int c = 0; c < n_it * kPerRun; c += 64) {
+        const int t = p0 * kPage + (c + lane) * kPiece;
+        bool keep = false;
+        for (int r = 0; r < (a.m_sh == 0 ? 1 : a.g); ++r)
+          if (t < end) {  // the context's last pieces end with it (and may overlap: a run more, never one less)
+            MT x[kPiece];
+            load_mask<MK>(m0 + r * a.m_sh + min(t, ctx - kPiece), x);
+#pragma unroll
+            for (int e = 0; e < kPiece; ++e) keep = keep || mask_keeps<MK>(x[e]);
+          }
+        const uint64_t any = __builtin_amdgcn_ballot_w64(keep);
+        for (int k = 0; k < 64 / kPerRun && c / kPerRun + k < n_it; ++k)
+          if ((any >> (k * kPerRun)) & ((uint64_t{1} << kPerRun) - 1)) live |= uint64_t{1} << (c / kPerRun + k);
+      }
+      n_run = __builtin_popcountll(live);
+      if (n_run == 0) return;
+    }
+    live_lo = live & ((uint64_t{1} << rot) - 1);
+    live_hi = live ^ live_lo;
+  }
+  const bool listed = MK != kDecodeNoMask && n_it <= 64;
+  auto next_run = [&](int i) {
+    if (!listed) return run_of(i);
+    uint64_t& m = live_hi ? live_hi : live_lo;
+    const int r = __builtin_ctzll(m);
+    m &= m - 1;
+    return r;
+  };
   const LoadOffsets lo = DENSE ? LoadOffsets::dense<D>(lane, k_row, v_row) : LoadOffsets(lane);
   // Loads of a whole run (a page, or a 64-token window of dense K / V).
   auto issue_k = [&](f16x8 (&ka)[4][DS], Rsrc kr) {
@@ -440,9 +512,10 @@ __device__ __forceinline__ void stream_pages(const SplitArgs& a, int b, int kvh,
   };
   f16x8 ka[4][DS];
   VT va[VR][2];
+  int run = next_run(0);
   {
     Rsrc kr, vr;
-    locate(run_of(0), kr, vr);
+    locate(run, kr, vr);
     if (DENSE && ctx < kPage) {
       if constexpr (DENSE) {  // the one short run
         load_k_dense<D, false>(ka, kr, lo, k_row);
@@ -460,7 +533,15 @@ __device__ __forceinline__ void stream_pages(const SplitArgs& a, int b, int kvh,
   // 48.9 us for B 32 x 16 heads x 2048 tokens.)
   auto step = [&](int it) {
     int lo_tok, valid;  // this run's own window tokens: [lo_tok, valid)
-    window(run_of(it), lo_tok, valid);
+    window(run, lo_tok, valid);
+    // The mask of this lane's tokens, in flight during the QK products.
+    constexpr int kMW = 8 * sizeof(MT) / 4;  // 32-bit words of 8 elements
+    uint32_t mk[2][kMW];
+    if constexpr (MK != kDecodeNoMask) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        __builtin_memcpy(mk[j], mrow + ((p0 + run) * kPage - lo_tok + 32 * j + 8 * grp), sizeof(mk[j]));
+    }
 #pragma unroll
     for (int jh = 0; jh < 4; ++jh)
 #pragma unroll
@@ -476,14 +557,15 @@ __device__ __forceinline__ void stream_pages(const SplitArgs& a, int b, int kvh,
     // The K registers are consumed: start the next run's K loads into them
     // now, so they are in flight during this run's softmax and PV.
     const int nx = it + 1;
-    const bool more = nx < n_it;
+    const bool more = nx < n_run;
     Rsrc kr, vr;
     if (more) {
+      run = next_run(nx);
       if (!DENSE && (nx & 63) == 0) {  // the page ids of the next 64 runs
         const int q = nx + lane;
         ids = q < n_it ? trow[q] : 0;
       }
-      locate(run_of(nx), kr, vr);
+      locate(run, kr, vr);
       issue_k(ka, kr);
     }
 
@@ -498,6 +580,15 @@ __device__ __forceinline__ void stream_pages(const SplitArgs& a, int b, int kvh,
         for (int v = 0; v < 4; ++v) {
           const int t = 32 * (jh >> 1) + 8 * grp + 4 * (jh & 1) + v;
           float x = sc[jh][v] * a.scale_log2;
+          const int e = 4 * (jh & 1) + v;
+          if constexpr (MK == kDecodeMaskBool)
+            x = ((mk[jh >> 1][e / 4] >> (8 * (e % 4))) & 0xffu) != 0 ? x : -INFINITY;
+          if constexpr (MK == kDecodeMaskF16) {
+            typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+            x = __builtin_fmaf(static_cast<float>(__builtin_bit_cast(f16x2, mk[jh >> 1][e / 2])[e % 2]), kLog2e, x);
+          }
+          if constexpr (MK == kDecodeMaskF32)
+            x = __builtin_fmaf(__builtin_bit_cast(float, mk[jh >> 1][e]), kLog2e, x);
           if constexpr (decltype(edge)::value) x = t >= lo_tok && t < valid ? x : -INFINITY;
           sc[jh][v] = x;
           mx = fmaxf(mx, x);
@@ -510,14 +601,16 @@ __device__ __forceinline__ void stream_pages(const SplitArgs& a, int b, int kvh,
     mx = fmaxf(mx, wave_xor(mx, 16));
     mx = fmaxf(mx, wave_xor(mx, 32));
     const float m_new = fmaxf(m_run, mx);
-    const float alpha = fast_exp2(m_run - m_new);
+    // (a row without a kept token so far: -inf, weights 0)
+    const float m_use = MK != kDecodeNoMask && m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = fast_exp2(m_run - m_use);
     float psum = 0.f;
     f16x8 pb[2];
 #pragma unroll
     for (int jh = 0; jh < 4; ++jh)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const float pv = fast_exp2(sc[jh][v] - m_new);
+        const float pv = fast_exp2(sc[jh][v] - m_use);
         psum += pv;
         pb[jh >> 1][(jh & 1) * 4 + v] = static_cast<_Float16>(pv);
       }
@@ -558,7 +651,7 @@ __device__ __forceinline__ void stream_pages(const SplitArgs& a, int b, int kvh,
     if (more) issue_v(va, vr);
   };
 
-  for (int it = 0; it < n_it; ++it) step(it);
+  for (int it = 0; it < n_run; ++it) step(it);
   if (poisoned) l_run = NAN;  // propagates to the merged output: NaN, not a fault
   l_run += wave_xor(l_run, 16);
   l_run += wave_xor(l_run, 32);
@@ -595,13 +688,14 @@ __device__ __forceinline__ f32x4 merge_row4(int nch, LoadML load_ml, LoadO load_
 #pragma unroll
     for (int u = 0; u < G; ++u)
       if (c + u < nch) mc = fmaxf(mc, ml[u][0]);
-    const float r = fast_exp2(M - mc);  // first round: exp2(-inf) = 0
+    const float mu = mc == -INFINITY ? 0.f : mc;  // a masked row that has kept nothing yet: weights 0
+    const float r = fast_exp2(M - mu);  // first round: exp2(-inf) = 0
     L *= r;
     acc *= r;
 #pragma unroll
     for (int u = 0; u < G; ++u) {
       // Explicit fused multiply-adds: every kernel that merges rounds alike.
-      const float w = fast_exp2(ml[u][0] - mc);
+      const float w = fast_exp2(ml[u][0] - mu);
       if (c + u < nch) {
         L = __builtin_fmaf(ml[u][1], w, L);
 #pragma unroll
@@ -665,12 +759,12 @@ __device__ void merge_in_kernel(const SplitArgs& a, int b, int c, int kvh, int n
         },
         Mr, Lr);
     const int64_t row = static_cast<int64_t>(b) * a.Hq + kvh * a.g + col;
-    const float inv = bad ? NAN : 1.f / Lr;  // the merge pass's product, then NaN for a bad context
+    const float inv = bad ? NAN : Lr == 0.f ? 0.f : 1.f / Lr;  // as the merge pass; every token masked: zeros
     f16x4 rv;
 #pragma unroll
     for (int e = 0; e < 4; ++e) rv[e] = to_f16(ac[e] * inv);
     *reinterpret_cast<f16x4*>(a.out + row * D + d) = rv;
-    if (a.lse && d == 0) a.lse[row] = (Mr + log2f(Lr)) * kLn2;
+    if (a.lse && d == 0) a.lse[row] = Lr == 0.f ? -INFINITY : (Mr + log2f(Lr)) * kLn2;
   }
   for (int s2 = static_cast<int>(threadIdx.x); s2 < nch; s2 += W * 64)
     __builtin_amdgcn_raw_buffer_store_b32(0u, wr, fl_off + s2 * 4, 0, kAuxDevice);
@@ -682,7 +776,7 @@ __device__ void merge_in_kernel(const SplitArgs& a, int b, int c, int kvh, int n
 // sequence has one chunk and out is given, else the chunk's partial (O per
 // q head and feature; m, l) into the workspace for the merge pass -- or,
 // with a ticket, for the merge in the same kernel (merge_in_kernel).
-template <int D, bool DENSE = false, int W = kWaves>
+template <int D, bool DENSE = false, int W = kWaves, int MK = kDecodeNoMask>
 __device__ __forceinline__ void run_item(const SplitArgs& a, int b, int c, int kvh, int wave,
                                          int lane) {
   constexpr int DB = D / 16;
@@ -698,7 +792,7 @@ __device__ __forceinline__ void run_item(const SplitArgs& a, int b, int c, int k
   const int w1 = cp0 + static_cast<int>(static_cast<int64_t>(wave + 1) * nc / W);
   f32x4 o[DB];
   float m, l;
-  stream_pages<D, DENSE>(a, b, kvh, w0, w1 - w0, ctx, lane, o, m, l);
+  stream_pages<D, DENSE, MK>(a, b, kvh, w0, w1 - w0, ctx, lane, o, m, l);
   // Every wavefront's partial goes to LDS once; then each thread folds
   // output elements over the W partials, in wavefront order.  Lane
   // (col, grp) holds O^T[d = 16 db + 4 grp + v][col] in o[db][v]; a row of
@@ -781,9 +875,10 @@ __device__ __forceinline__ void run_item(const SplitArgs& a, int b, int c, int k
     if (single) {
       const int64_t row = static_cast<int64_t>(b) * a.Hq + kvh * a.g + col;
       // Empty context: zeros, as torch's CPU SDPA returns.
-      const float inv = ctx == 0 ? 0.f : (bad ? NAN : 1.f / L);
+      const bool none = ctx == 0 || (MK != kDecodeNoMask && L == 0.f);  // or every token masked
+      const float inv = none ? 0.f : (bad ? NAN : 1.f / L);
       a.out[row * D + d] = to_f16(O * inv);
-      if (a.lse && d == 0) a.lse[row] = ctx == 0 ? -INFINITY : (M + log2f(L)) * kLn2;
+      if (a.lse && d == 0) a.lse[row] = none ? -INFINITY : (M + log2f(L)) * kLn2;
     } else {
       a.ws[(slot * a.g + col) * D + d] = O;
       if (d == 0) {
@@ -864,12 +959,12 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void decode_split_list_ker
 // max_chunks chunks of its max_ctx tokens (grid = B Hkv max_chunks).  W
 // wavefronts per item and workgroup: 8, or 4 where the eight-wavefront
 // grid would take more than one round of the device (dense_decode_plan).
-template <int D, int W = kWaves>
+template <int D, int W = kWaves, int MK = kDecodeNoMask>
 __global__ __launch_bounds__(W * 64, kWavesPerSimd) void decode_dense_kernel(SplitArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
   const int item = blockIdx.x;
   const int c = item % a.max_chunks, r = item / a.max_chunks;
-  run_item<D, true, W>(a, r / a.Hkv, c, r % a.Hkv, wave, lane);
+  run_item<D, true, W, MK>(a, r / a.Hkv, c, r % a.Hkv, wave, lane);
 }
 
 // Workgroup slots of the four-wavefront dense kernel on the current device
@@ -992,13 +1087,13 @@ __global__ __launch_bounds__(kCols * D / 4) void decode_merge_rows_kernel(MergeA
   const f32x4 acc = merge_row4(
       ns, [&](int s) { return *reinterpret_cast<const f32x2*>(wm + s * sm); },
       [&](int s) { return *reinterpret_cast<const f32x4*>(wo + s * so); }, M, L);
-  const float inv = 1.f / L;
+  const float inv = L == 0.f ? 0.f : 1.f / L;  // every token masked: zeros
   const bool bad = ctx_raw > a.max_ctx;  // caller broke the max_context_len contract
   f16x4 rv;
 #pragma unroll
   for (int e = 0; e < 4; ++e) rv[e] = to_f16(bad ? NAN : acc[e] * inv);
   *reinterpret_cast<f16x4*>(o) = rv;
-  if (a.lse && d == 0) a.lse[row] = (M + log2f(L)) * kLn2;
+  if (a.lse && d == 0) a.lse[row] = L == 0.f ? -INFINITY : (M + log2f(L)) * kLn2;
 }
 
 // Chunks of the longest context: a chunk is kWaves wavefronts' shares of at
@@ -1294,8 +1389,11 @@ DenseDecodePlan dense_decode_plan(int B, int Hq, int Hkv, int Skv, int D) {
 }
 
 int dense_decode_launch(const DenseDecodePlan& plan, const void* q, const int64_t* q_strides, const void* k,
-                        const int64_t* k_strides, const void* v, const int64_t* v_strides, void* out, float* lse,
-                        void* workspace, int B, int Hq, int Hkv, int Skv, int D, float scale, void* stream) {
+                        const int64_t* k_strides, const void* v, const int64_t* v_strides, const void* mask,
+                        int mask_kind, const int64_t* mask_strides, void* out, float* lse, void* workspace, int B,
+                        int Hq, int Hkv, int Skv, int D, float scale, void* stream) {
+  SPYRE_REQUIRE(mask_kind == kDecodeNoMask || (mask && mask_strides && mask_strides[3] == 1 && Skv >= kPage),
+                SPYRE_EUNSUPPORTED, "dense decode: mask not covered");
   SPYRE_REQUIRE(plan.ok && (D == 64 || D == 128), SPYRE_EUNSUPPORTED, "dense decode: call not covered");
   SPYRE_REQUIRE(plan.chunks == 1 || workspace, SPYRE_EINVAL, "dense decode: no workspace");
   for (int i = 0; i < 3; ++i)
@@ -1329,19 +1427,33 @@ int dense_decode_launch(const DenseDecodePlan& plan, const void* q, const int64_
   sa.v_sb = v_strides[0];
   sa.v_sh = v_strides[1];
   sa.v_ss = v_strides[2];
+  sa.mask = mask;
+  if (mask_kind != kDecodeNoMask) {
+    sa.m_sb = mask_strides[0];
+    sa.m_sh = mask_strides[1];
+  }
   const bool fused = plan.fused;  // the chunks merge inside the kernel
   sa.ticket = fused ? next_call_ticket() : 0;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int64_t items = static_cast<int64_t>(B) * Hkv * plan.chunks;
   const dim3 grid(static_cast<unsigned>(items));
-  if (D == 128 && plan.waves == 4)
-    decode_dense_kernel<128, 4><<<grid, 4 * 64, 0, st>>>(sa);
-  else if (D == 128)
-    decode_dense_kernel<128><<<grid, kThreads, 0, st>>>(sa);
-  else if (plan.waves == 4)
-    decode_dense_kernel<64, 4><<<grid, 4 * 64, 0, st>>>(sa);
-  else
-    decode_dense_kernel<64><<<grid, kThreads, 0, st>>>(sa);
+  auto go = [&](auto mk) {
+    constexpr int MK = decltype(mk)::value;
+    if (D == 128 && plan.waves == 4)
+      decode_dense_kernel<128, 4, MK><<<grid, 4 * 64, 0, st>>>(sa);
+    else if (D == 128)
+      decode_dense_kernel<128, kWaves, MK><<<grid, kThreads, 0, st>>>(sa);
+    else if (plan.waves == 4)
+      decode_dense_kernel<64, 4, MK><<<grid, 4 * 64, 0, st>>>(sa);
+    else
+      decode_dense_kernel<64, kWaves, MK><<<grid, kThreads, 0, st>>>(sa);
+  };
+  switch (mask_kind) {
+    case kDecodeMaskF16: go(std::integral_constant<int, kDecodeMaskF16>{}); break;
+    case kDecodeMaskF32: go(std::integral_constant<int, kDecodeMaskF32>{}); break;
+    case kDecodeMaskBool: go(std::integral_constant<int, kDecodeMaskBool>{}); break;
+    default: go(std::integral_constant<int, kDecodeNoMask>{}); break;
+  }
   hipError_t e = hipGetLastError();
   SPYRE_REQUIRE(e == hipSuccess, SPYRE_EHIP, "dense decode launch failed: %s", hipGetErrorString(e));
   if (plan.chunks == 1 || fused) return SPYRE_OK;  // every sequence's output written

@@ -8,6 +8,9 @@
 
 namespace spyre_hip {
 
+// Mask kinds, numbered as SPYRE_MASK_*.
+enum DecodeMask { kDecodeNoMask = 0, kDecodeMaskF16 = 1, kDecodeMaskF32 = 2, kDecodeMaskBool = 3 };
+
 struct DenseDecodePlan {
   bool ok = false;      // the call is covered (sizes only; strides are the caller's check)
   int chunk_pages = 0;  // 64-token runs per chunk (a workgroup's share of a sequence)
@@ -29,11 +32,13 @@ uint32_t next_call_ticket();
 
 // Launches the plan: q strides {b, h} and K / V strides {b, h, s} in
 // elements (feature stride 1, 16-byte aligned rows, token strides below
-// 2^23); out [B, Hq, D] contiguous fp16; lse optional [B, Hq] fp32; the
+// 2^23); a mask (kind DecodeMask, strides {b, h, i, t} in elements with t
+// stride 1, any alignment) needs at least 64 keys; out [B, Hq, D] contiguous fp16; lse optional [B, Hq] fp32; the
 // workspace (16-byte aligned) holds plan.ws_bytes and needs no
 // initialisation: the flags a call sets are cleared by the same call.
 int dense_decode_launch(const DenseDecodePlan& plan, const void* q, const int64_t* q_strides, const void* k,
-                        const int64_t* k_strides, const void* v, const int64_t* v_strides, void* out, float* lse,
-                        void* workspace, int B, int Hq, int Hkv, int Skv, int D, float scale, void* stream);
+                        const int64_t* k_strides, const void* v, const int64_t* v_strides, const void* mask,
+                        int mask_kind, const int64_t* mask_strides, void* out, float* lse, void* workspace, int B,
+                        int Hq, int Hkv, int Skv, int D, float scale, void* stream);
 
 }  // namespace spyre_hip

@@ -25,6 +25,9 @@
 //    LDS reads.  The loop is software-pipelined: step t's softmax overlaps
 //    S(t+1).  A mask is staged per wavefront beside the tiles, a step ahead;
 //    steps it blanks for the whole wavefront skip their softmax and P V.
+//  * Decode: sdpa_decode_short_kernel (a row tile's keys all in flight at
+//    once) and the split-KV kernels of decode_attn.hip (dense_route), with
+//    or without a mask.
 //  * Other masks (fp32 biases whose keys are not contiguous, slices of 2 GiB):
 //    1. v_token_sticks_kernel: V [B, Hkv, Skv, D] (rows may be strided) ->
 //       Vt [B, Hkv, D, S64] in the workspace: V with its sticks along tokens
@@ -1270,7 +1273,7 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
 
 // ---- 4. short decode: a block's keys all in flight at once ----------------
 //
-// Calls without a mask or causal flag whose block holds one row tile (the g
+// Calls without the causal flag whose block holds one row tile (the g
 // q heads of a KV head times Sq <= 32 rows) and at most kWaves2 * KW keys
 // (KW = 64 keys at D = 64, 32 at D = 128): wavefront w loads keys
 // kb + w KW .. + KW - 1 of K and V into its own LDS slice, all loads issued
@@ -1294,8 +1297,12 @@ struct ShortLds {
   static_assert(64 * kFoldF * 4 <= kSliceB, "a wavefront's fold records fit its own slice");
 };
 
-template <int D, bool PRESCALED, int W>
+// A mask with contiguous keys is read as it lies, 4 elements of the lane's
+// row at a time, while the slices load (masked calls keep q unscaled and sum
+// the fp32 probabilities).
+template <int D, bool PRESCALED, int W, int MK = kNoMask>
 __global__ __launch_bounds__(W * 64) void sdpa_decode_short_kernel(Fwd2Args a) {
+  static_assert(MK == kNoMask || !PRESCALED, "masked: scores scaled in fp32");
   using L = ShortLds<D>;
   constexpr int DK = D / 16, DM = D / 32;
   constexpr int KW = L::kKW, MT = KW / 32;  // 32-key S^T tiles per wavefront
@@ -1354,6 +1361,31 @@ __global__ __launch_bounds__(W * 64) void sdpa_decode_short_kernel(Fwd2Args a) {
                  row < rows_here ? (static_cast<uint32_t>(row) * static_cast<uint32_t>(a.v_ss) + 8 * ch) * 2 : kOob);
     }
   }
+  // Mask elements of this lane's row, keys kw + 32 mt + 16 (i / 2) + 8 half +
+  // 4 (i % 2) .. + 3 in mw[mt][i]; a ragged slice's keys past its last one
+  // repeat that one (the key test below drops them).
+  using ME = typename MaskElem<MK>::T;
+  constexpr int kMW = sizeof(ME);  // 32-bit words of 4 elements
+  uint32_t mw[MT][4][kMW];
+  if constexpr (MK != kNoMask) {
+    if (rows_here > 0) {
+      const ME* mrow = static_cast<const ME*>(a.mask) + b * a.m_sb + (q_ok ? h * a.m_sh + qi * a.m_sq : kvh * a.g * a.m_sh) + kw;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int k4 = 32 * mt + 16 * (i >> 1) + 8 * half + 4 * (i & 1);
+          if (rows_here >= KW) {
+            __builtin_memcpy(mw[mt][i], mrow + k4, sizeof(mw[mt][i]));
+          } else {
+            ME x[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = mrow[min(k4 + e, rows_here - 1)];
+            __builtin_memcpy(mw[mt][i], x, sizeof(x));
+          }
+        }
+    }
+  }
 #pragma unroll
   for (int ks = 0; ks < DK; ++ks) {
     if constexpr (PRESCALED) {
@@ -1391,7 +1423,12 @@ __global__ __launch_bounds__(W * 64) void sdpa_decode_short_kernel(Fwd2Args a) {
 #pragma unroll
       for (int rr = 0; rr < 16; ++rr) {
         const int kr = mt * 32 + key32_of(8 * (rr >> 2) + (rr & 3));
-        const float x = PRESCALED ? s[mt][rr] : s[mt][rr] * scale_abs;
+        float x = PRESCALED ? s[mt][rr] : s[mt][rr] * scale_abs;
+        if constexpr (MK == kMaskBool) x = ((mw[mt][rr >> 2][0] >> (8 * (rr & 3))) & 0xffu) != 0 ? x : -INFINITY;
+        if constexpr (MK == kMaskF16)
+          x = __builtin_fmaf(static_cast<float>(__builtin_bit_cast(f16x2, mw[mt][rr >> 2][(rr & 3) / 2])[rr & 1]), kLog2e, x);
+        if constexpr (MK == kMaskF32)
+          x = __builtin_fmaf(__builtin_bit_cast(float, mw[mt][rr >> 2][rr & 3]), kLog2e, x);
         s[mt][rr] = kr <= kl ? x : -INFINITY;
       }
     float mx = -INFINITY;
@@ -1399,7 +1436,8 @@ __global__ __launch_bounds__(W * 64) void sdpa_decode_short_kernel(Fwd2Args a) {
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int rr = 0; rr < 16; ++rr) mx = fmaxf(mx, s[mt][rr]);
-    m = max_xor32(mx);  // the row's max over both lane halves (finite: key kw is visible)
+    m = max_xor32(mx);  // the row's max over both lane halves (finite without a mask: key kw is visible)
+    const float mu = MK != kNoMask && m == -INFINITY ? 0.f : m;  // a row with every key masked: weights 0
     // P (fp16) and its row sum over the same fp16 values; pb[mt][j] is the
     // PV operand of keys 32mt + 16j + 8half .. + 7.
     f16x8 pb[MT][2];
@@ -1408,9 +1446,13 @@ __global__ __launch_bounds__(W * 64) void sdpa_decode_short_kernel(Fwd2Args a) {
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) pb[mt][j][e] = static_cast<_Float16>(fast_exp2(s[mt][8 * j + e] - m));
+        for (int e = 0; e < 8; ++e) {
+          const float p = fast_exp2(s[mt][8 * j + e] - mu);
+          pb[mt][j][e] = static_cast<_Float16>(p);
+          if constexpr (MK != kNoMask) l += p;
+        }
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
+        for (int e = 0; e < 4 && MK == kNoMask; ++e)
           l = __builtin_amdgcn_fdot2(f16x2{pb[mt][j][2 * e], pb[mt][j][2 * e + 1]}, f16x2{1, 1}, l, false);
       }
     // O^T += V^T P^T: V^T operands by transposing reads of the V slice (rows
@@ -1846,12 +1888,10 @@ Shape pick_shape(int64_t pairs, int64_t rows, int g, int keys, int nsplit, int D
 // one block's rows and split the keys until the grid fills the device, if
 // the workspace (ws_bytes) holds the split's partials; otherwise the heads
 // are packed only as far as the unsplit grid still fills the device
-// (pack_heads).  Masked calls take the same grid, less the short-decode
-// kernel; one block per q head and 256 queries, unsplit, left most units or
+// (pack_heads).  Masked calls take the same grid; one block per q head and 256 queries, unsplit, left most units or
 // wavefronts idle for short query runs: 128 queries x 4096 keys with the
 // chunk's causal boolean mask (B 4, 32 / 8 heads) 94.0 us, packed and split
-// 54.3; one query x 2048 keys with a padding mask (B 16) 98.6 and 33.6; 512
-// queries x 512 keys (B 2) the same grid and time.
+// 54.3.
 struct GridPlan {
   int pack = 1, nsplit = 1, split_keys = 0;
   size_t part_bytes = 0;
@@ -1859,6 +1899,40 @@ struct GridPlan {
   int waves = kWaves2;         // its wavefronts per block
   Shape shape = k256;
 };
+
+// Short decode: one row tile (the g q heads of a KV head times Sq <= 32
+// rows) whose keys fit one block (kWaves2 slices), or a split of them
+// over blocks that all run in one round of the device.  Masks are read as they
+// lie (contiguous keys: the caller's check).
+bool short_grid(int B, int Hq, int Hkv, int Sq, int Skv, int D, size_t ws_bytes, GridPlan& gp) {
+  const int g = Hq / Hkv;
+  if (Sq <= 0 || static_cast<int64_t>(g) * Sq > 32) return false;
+  const int kw = D == 64 ? ShortLds<64>::kKW : ShortLds<128>::kKW;
+  const int64_t cus = device_cus() > 0 ? device_cus() : 256;
+  int waves = kWaves2;
+  int ns = std::max(1, (Skv + waves * kw - 1) / (waves * kw));
+  // A split over at most half the units at eight wavefronts: four-wavefront
+  // blocks of half the keys, twice as many, one per unit (batch-1 GQA, 4096
+  // keys at D 128: 256 blocks of 128 keys instead of 128 of 256).
+  if (ns > 1 && static_cast<int64_t>(B) * Hkv * 2 * ns <= cus) {
+    waves = 4;
+    ns = (Skv + waves * kw - 1) / (waves * kw);
+  }
+  // the partials, then one arrival flag per (sequence, KV head, split)
+  const size_t pb = ns > 1 ? split_bytes(static_cast<int64_t>(B) * Hq * Sq, ns, D) +
+                                 static_cast<size_t>(B) * Hkv * ns * sizeof(uint32_t)
+                           : 0;
+  if (static_cast<int64_t>(B) * Hkv * ns <= cus && (ns == 1 || ws_bytes >= pb)) {
+    gp.pack = g;
+    gp.nsplit = ns;
+    gp.split_keys = ns > 1 ? waves * kw : Skv;
+    gp.part_bytes = pb;
+    gp.short_decode = true;
+    gp.waves = waves;
+    return true;
+  }
+  return false;
+}
 
 // mask_kind: a staged or copied mask's; can_pack: its rows of a KV head's q heads
 // fit one buffer descriptor (else heads stay apart).
@@ -1869,35 +1943,7 @@ GridPlan plan_grid(int B, int Hq, int Hkv, int Sq, int Skv, int D, bool causal, 
   const int g = can_pack ? Hq / Hkv : 1;
   const int Hb = Hq / g;  // the (KV head, pack group) pairs of a sequence
   gp.split_keys = Skv;
-  // Short decode: one row tile (the g q heads of a KV head times Sq <= 32
-  // rows) whose keys fit one block (kWaves2 slices), or a split of them
-  // over blocks that all run in one round of the device.
-  if (!causal && !masked && Sq > 0 && static_cast<int64_t>(g) * Sq <= 32) {
-    const int kw = D == 64 ? ShortLds<64>::kKW : ShortLds<128>::kKW;
-    const int64_t cus = device_cus() > 0 ? device_cus() : 256;
-    int waves = kWaves2;
-    int ns = std::max(1, (Skv + waves * kw - 1) / (waves * kw));
-    // A split over at most half the units at eight wavefronts: four-wavefront
-    // blocks of half the keys, twice as many, one per unit (batch-1 GQA, 4096
-    // keys at D 128: 256 blocks of 128 keys instead of 128 of 256).
-    if (ns > 1 && static_cast<int64_t>(B) * Hkv * 2 * ns <= cus) {
-      waves = 4;
-      ns = (Skv + waves * kw - 1) / (waves * kw);
-    }
-    // the partials, then one arrival flag per (sequence, KV head, split)
-    const size_t pb = ns > 1 ? split_bytes(static_cast<int64_t>(B) * Hq * Sq, ns, D) +
-                                   static_cast<size_t>(B) * Hkv * ns * sizeof(uint32_t)
-                             : 0;
-    if (static_cast<int64_t>(B) * Hkv * ns <= cus && (ns == 1 || ws_bytes >= pb)) {
-      gp.pack = g;
-      gp.nsplit = ns;
-      gp.split_keys = ns > 1 ? waves * kw : Skv;
-      gp.part_bytes = pb;
-      gp.short_decode = true;
-      gp.waves = waves;
-      return gp;
-    }
-  }
+  if (!causal && !masked && short_grid(B, Hq, Hkv, Sq, Skv, D, ws_bytes, gp)) return gp;
   if (!causal && Sq > 0) {
     const int p0 = Sq < kQB ? g : 1;
     int keys = Skv;
@@ -1924,16 +1970,38 @@ GridPlan plan_grid(int B, int Hq, int Hkv, int Sq, int Skv, int D, bool causal, 
 // fills at least half the device: they stream K / V through the split-KV
 // decode kernels (decode_attn.hip), whose operands come straight from
 // memory into registers -- no LDS tiles, no barrier per step.
-spyre_hip::DenseDecodePlan dense_route(int B, int Hq, int Hkv, int Sq, int Skv, int D, bool causal, int mask_kind) {
-  if (mask_kind != kNoMask || causal || Sq != 1) return {};
-  if (plan_grid(B, Hq, Hkv, Sq, Skv, D, false, SIZE_MAX).short_decode) return {};
+// Masks with contiguous keys are read as they lie (16 sequences of up to
+// 2048 padded keys, 32 / 8 heads of D 128: 32.4 us in half steps of the LDS
+// kernel, 23.2 here, the padding's K and V not read); a mask row shorter than
+// the run its loads cover (64 keys) stays with the LDS kernel.
+spyre_hip::DenseDecodePlan dense_route(int B, int Hq, int Hkv, int Sq, int Skv, int D, bool causal, int mask_kind,
+                                       const int64_t* mask_strides) {
+  if (causal || Sq != 1) return {};
+  if (mask_kind != kNoMask && (mask_strides[3] != 1 || Skv < kKT)) return {};
+  GridPlan gp;
+  if (short_grid(B, Hq, Hkv, Sq, Skv, D, SIZE_MAX, gp)) return {};
   return spyre_hip::dense_decode_plan(B, Hq, Hkv, Skv, D);
 }
 
-template <int W>
-void launch_short_w(const Fwd2Args& f2, int D, bool prescaled, hipStream_t st) {
+template <int W, int MK>
+void launch_short_masked(const Fwd2Args& f2, int D, hipStream_t st) {
   const dim3 grid(f2.n_items);
-  if (D == 128 && prescaled)
+  if (D == 128)
+    sdpa_decode_short_kernel<128, false, W, MK><<<grid, W * 64, 0, st>>>(f2);
+  else
+    sdpa_decode_short_kernel<64, false, W, MK><<<grid, W * 64, 0, st>>>(f2);
+}
+
+template <int W>
+void launch_short_w(const Fwd2Args& f2, int D, bool prescaled, int mask_kind, hipStream_t st) {
+  const dim3 grid(f2.n_items);
+  if (mask_kind == kMaskF16)
+    launch_short_masked<W, kMaskF16>(f2, D, st);
+  else if (mask_kind == kMaskF32)
+    launch_short_masked<W, kMaskF32>(f2, D, st);
+  else if (mask_kind == kMaskBool)
+    launch_short_masked<W, kMaskBool>(f2, D, st);
+  else if (D == 128 && prescaled)
     sdpa_decode_short_kernel<128, true, W><<<grid, W * 64, 0, st>>>(f2);
   else if (D == 128)
     sdpa_decode_short_kernel<128, false, W><<<grid, W * 64, 0, st>>>(f2);
@@ -1943,11 +2011,11 @@ void launch_short_w(const Fwd2Args& f2, int D, bool prescaled, hipStream_t st) {
     sdpa_decode_short_kernel<64, false, W><<<grid, W * 64, 0, st>>>(f2);
 }
 
-void launch_short(const Fwd2Args& f2, int D, bool prescaled, int waves, hipStream_t st) {
+void launch_short(const Fwd2Args& f2, int D, bool prescaled, int waves, int mask_kind, hipStream_t st) {
   if (waves == 4)
-    launch_short_w<4>(f2, D, prescaled, st);
+    launch_short_w<4>(f2, D, prescaled, mask_kind, st);
   else
-    launch_short_w<kWaves2>(f2, D, prescaled, st);
+    launch_short_w<kWaves2>(f2, D, prescaled, mask_kind, st);
 }
 
 template <int MK, int SLOTS, bool HALF, int W>
@@ -2015,6 +2083,7 @@ __global__ __launch_bounds__(256) void mask_pad_kernel(MaskPadArgs a) {
 }
 
 bool aligned16(const void* p);
+int64_t s64_of(int Skv);
 
 // How a call's mask reaches the kernels:
 //  kRouteNone    no mask;
@@ -2025,7 +2094,7 @@ bool aligned16(const void* p);
 //  kRouteF32     fp32 with key stride 1: the main kernel in half steps
 //                (position bias [1, 16, 777, 777], B 2, D 64: 59.3 us by
 //                kRouteVt, 22.9 here; [1, 32, 2048, 2048], 32 / 8 heads, D 128:
-//                489 and 192; one query x 2000 keys: 213 and 14.7);
+//                489 and 192);
 //  kRouteVt      other fp32 masks (or a slice, or a copy's, past 2 GiB): the
 //                per-wavefront kernel, V through the workspace.
 enum MaskRoute { kRouteNone, kRouteStaged, kRouteCopied, kRouteF32, kRouteVt };
@@ -2098,6 +2167,14 @@ size_t copy_room(const MaskPlan& mp) {
   return mp.route == kRouteCopied ? (mp.copy_bytes + 255) / 256 * 256 : 0;
 }
 
+// The least workspace a masked call accepts (spyre_sdpa_fwd_min_workspace_bytes)
+// or, for a copied mask, its copy.
+size_t min_room(const MaskPlan& mp, int B, int Hkv, int Skv, int D) {
+  return mp.route == kRouteCopied ? mp.copy_bytes
+         : mp.route >= kRouteF32  ? static_cast<size_t>(B) * Hkv * D * s64_of(Skv) * sizeof(_Float16)
+                                  : 0;
+}
+
 // The grid of a staged or copied mask's call given ws_bytes beyond the copy.
 GridPlan masked_grid(const MaskPlan& mp, int kind, int B, int Hq, int Hkv, int Sq, int Skv, int D, size_t ws_bytes) {
   return plan_grid(B, Hq, Hkv, Sq, Skv, D, false, ws_bytes, kind, mask_extent(mp, Hq / Hkv) <= kBufRange);
@@ -2147,15 +2224,22 @@ extern "C" size_t spyre_sdpa_fwd_call_workspace_bytes(const void* attn_mask, int
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || Sq < 0 || Skv < 0 || (D != 64 && D != 128)) return 0;
   if (mask_kind == kNoMask) {  // a key split's partials (calls without the causal flag)
     const size_t split = plan_grid(B, Hq, Hkv, Sq, Skv, D, false, SIZE_MAX).part_bytes;
-    const spyre_hip::DenseDecodePlan dp = dense_route(B, Hq, Hkv, Sq, Skv, D, false, mask_kind);
+    const spyre_hip::DenseDecodePlan dp = dense_route(B, Hq, Hkv, Sq, Skv, D, false, mask_kind, nullptr);
     return dp.ok ? std::max(split, dp.ws_bytes) : split;  // the split for calls the decode route refuses
   }
   if (!mask_strides || mask_kind < kNoMask || mask_kind > kMaskBool) return 0;
   const MaskPlan mp = plan_mask(attn_mask, mask_kind, mask_strides, B, Hq, Sq, Skv);
-  if (mp.route == kRouteVt) return spyre_sdpa_fwd_workspace_bytes(B, Hkv, Skv, D);
+  // Decode that reads the mask as it lies takes its partials alone, but the
+  // call also holds what the kernels that stage or copy the mask would need.
+  GridPlan gs;
+  if (mask_strides[3] == 1 && short_grid(B, Hq, Hkv, Sq, Skv, D, SIZE_MAX, gs))
+    return std::max(gs.part_bytes, min_room(mp, B, Hkv, Skv, D));
+  const spyre_hip::DenseDecodePlan dp = dense_route(B, Hq, Hkv, Sq, Skv, D, false, mask_kind, mask_strides);
+  const size_t decode = dp.ok ? dp.ws_bytes : 0;
+  if (mp.route == kRouteVt) return std::max(decode, spyre_sdpa_fwd_workspace_bytes(B, Hkv, Skv, D));
   const size_t part = masked_grid(mp, mask_kind, B, Hq, Hkv, Sq, Skv, D, SIZE_MAX).part_bytes;
-  if (mp.route == kRouteF32) return std::max(part, spyre_sdpa_fwd_workspace_bytes(B, Hkv, Skv, D));
-  return part ? copy_room(mp) + part : mp.copy_bytes;
+  if (mp.route == kRouteF32) return std::max({decode, part, spyre_sdpa_fwd_workspace_bytes(B, Hkv, Skv, D)});
+  return std::max(decode, part ? copy_room(mp) + part : mp.copy_bytes);
 }
 
 extern "C" size_t spyre_sdpa_fwd_min_workspace_bytes(const void* attn_mask, int mask_kind,
@@ -2216,9 +2300,20 @@ extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const
                                                  : 0;
   SPYRE_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && aligned16(workspace)),
                 SPYRE_ENOSPC, "workspace %zu < %zu bytes (or misaligned)", workspace_bytes, need);
-  const bool lds_path = mp.route != kRouteVt;
   if (Sq == 0) return SPYRE_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
+  const size_t ws_room = workspace && aligned16(workspace) ? workspace_bytes : 0;
+  // Decode that reads its mask as it lies: no copy, no relayout of V.
+  const bool direct = mask_kind == kNoMask || mask_strides[3] == 1;
+  const spyre_hip::DenseDecodePlan dp =
+      direct ? dense_route(B, Hq, Hkv, Sq, Skv, D, is_causal != 0, mask_kind, mask_strides) : spyre_hip::DenseDecodePlan{};
+  const bool dense = dp.ok && k_strides[2] < (int64_t{1} << 23) && v_strides[2] < (int64_t{1} << 23) &&
+                     (k_strides[2] == 0 || k_strides[2] >= D) && (v_strides[2] == 0 || v_strides[2] >= D) &&
+                     (dp.ws_bytes == 0 || ws_room >= dp.ws_bytes);
+  GridPlan gs;
+  const bool as_it_lies = mask_kind != kNoMask && direct && (dense || short_grid(B, Hq, Hkv, Sq, Skv, D, ws_room, gs));
+  if (as_it_lies) mp.route = kRouteNone;
+  const bool lds_path = mp.route != kRouteVt;
   const int s64 = static_cast<int>(s64_of(Skv));
   const void* mask_ptr = attn_mask;
   if (mp.route == kRouteCopied) {
@@ -2284,12 +2379,9 @@ extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const
   fa.causal = is_causal ? 1 : 0;
   fa.scale_log2 = scale * kLog2e;
   if (lds_path) {
-    const spyre_hip::DenseDecodePlan dp = dense_route(B, Hq, Hkv, Sq, Skv, D, is_causal != 0, mask_kind);
-    if (dp.ok && k_strides[2] < (int64_t{1} << 23) && v_strides[2] < (int64_t{1} << 23) &&
-        (k_strides[2] == 0 || k_strides[2] >= D) && (v_strides[2] == 0 || v_strides[2] >= D) &&
-        (dp.ws_bytes == 0 || (workspace && aligned16(workspace) && workspace_bytes >= dp.ws_bytes)))
-      return spyre_hip::dense_decode_launch(dp, q, q_strides, k, k_strides, v, v_strides, out, lse, workspace, B,
-                                            Hq, Hkv, Skv, D, scale, stream);
+    if (dense)
+      return spyre_hip::dense_decode_launch(dp, q, q_strides, k, k_strides, v, v_strides, attn_mask, mask_kind,
+                                            mask_strides, out, lse, workspace, B, Hq, Hkv, Skv, D, scale, stream);
     // K/V tiles (and mask blocks) shared through LDS.
     Fwd2Args f2{};
     f2.q = fa.q;
@@ -2318,11 +2410,11 @@ extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const
     // instead of g mostly idle ones).
     // And (plan_grid) a key split when the blocks would not fill the device
     // and the workspace holds its partials (after a mask's copy).
-    const size_t ws_room = workspace && aligned16(workspace) ? workspace_bytes : 0;
     const size_t part_at = copy_room(mp);
     const size_t part_room = ws_room > part_at ? ws_room - part_at : 0;
-    const GridPlan gpl = mask_kind == kNoMask ? plan_grid(B, Hq, Hkv, Sq, Skv, D, is_causal != 0, part_room)
-                                              : masked_grid(mp, mask_kind, B, Hq, Hkv, Sq, Skv, D, part_room);
+    const GridPlan gpl = as_it_lies               ? gs
+                         : mask_kind == kNoMask ? plan_grid(B, Hq, Hkv, Sq, Skv, D, is_causal != 0, part_room)
+                                                : masked_grid(mp, mask_kind, B, Hq, Hkv, Sq, Skv, D, part_room);
     f2.pack = gpl.pack;
     f2.gp = fa.g / f2.pack;
     const int rows = shape_rows(gpl.shape);
@@ -2343,16 +2435,16 @@ extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const
     // |scale log2 e| <= 1: q times it stays within fp16, so Q is prescaled.
     const bool prescaled = fabsf(f2.scale_log2) <= 1.f;
     f2.mask = mask_ptr;
-    f2.m_sb = mp.sb;
-    f2.m_sh = mp.sh;
-    f2.m_sq = mp.sq;
+    f2.m_sb = as_it_lies ? mask_strides[0] : mp.sb;
+    f2.m_sh = as_it_lies ? mask_strides[1] : mp.sh;
+    f2.m_sq = as_it_lies ? mask_strides[2] : mp.sq;
     f2.m_bytes = static_cast<uint32_t>(mask_extent(mp, f2.pack));
     f2.m_wide = mp.wide ? 1 : 0;
     if (gpl.short_decode) {
       // One row tile, its keys all in flight at once; a key split merges in
       // the same kernel.
       f2.ticket = spyre_hip::next_call_ticket();
-      launch_short(f2, D, prescaled, gpl.waves, st);
+      launch_short(f2, D, prescaled, gpl.waves, mask_kind, st);
     } else {
       auto go = [&](auto mk) {
         constexpr int MK = decltype(mk)::value;
