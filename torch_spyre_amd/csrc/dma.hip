@@ -14,10 +14,11 @@
 //               one such workgroup per CU, the chip reads in one phase and
 //               writes in the next, which HBM serves better than the mixed
 //               read/write stream of small per-lane copies.
-//  * vec:       one loop is unit-stride on both sides.  Each lane moves four
-//               items of up to 16 bytes (loads issued before stores); eight
-//               lanes cover one 128-byte stick, so every wavefront touches
-//               whole cache lines on both sides.
+//  * vec:       one loop is unit-stride on both sides.  Each lane moves one or
+//               four items of up to 16 bytes (loads issued before stores) at
+//               any alignment and length of run; eight lanes cover one
+//               128-byte stick.  The vec nests of one description (a tensor's
+//               whole sticks and the remainder of its rows) run in one launch.
 //  * transpose: one loop is unit-stride in src and another in dst (the stick
 //               moves to another dim, e.g. transpose-restick).  A wavefront
 //               owns four 64x64 tiles of 2-byte elements (8x8 blocks of
@@ -82,6 +83,7 @@ struct Nest {
   FastDiv inner;              // inner loop length in items
   FastDiv outer[kMaxLoops];   // outer loop lengths
   int64_t inner_ss, inner_sd; // inner strides (bytes per item)
+  int64_t last;               // vec: where a run's last item starts (bytes)
   int64_t ss[kMaxLoops], sd[kMaxLoops];  // outer strides (bytes)
   int64_t off_s, off_d;       // bytes
   uint32_t total;             // items
@@ -95,11 +97,30 @@ template <> struct VecT<4> { using T = uint32_t; };
 template <> struct VecT<2> { using T = uint16_t; };
 template <> struct VecT<1> { using T = uint8_t; };
 
+// The same at any address: the vector loads and stores of this device take
+// them.  A run of any length of at least VB bytes is items of VB bytes, the
+// last of which starts VB before the run's end: where VB does not divide the
+// run it moves some bytes a second time, to where they already are.  (fp16
+// [2, 777, 5001], whose rows start on odd elements: 2-byte items took 19.1 us
+// to sticks and 18.9 back, these 8.0 and 8.2.)
+template <int VB>
+struct AnyT {
+  typedef typename VecT<VB>::T T __attribute__((aligned(1)));
+};
+
+// VB: bytes of a vec item; 0: one element, the inner loop strided.
+template <int VB>
 __device__ __forceinline__ void item_offsets(const Nest& n, uint32_t i, int64_t& so, int64_t& sd) {
   uint32_t q = fdiv(i, n.inner);
   const uint32_t r = i - q * n.inner.d;
-  so = n.off_s + static_cast<int64_t>(r) * n.inner_ss;
-  sd = n.off_d + static_cast<int64_t>(r) * n.inner_sd;
+  if (VB) {
+    const int64_t b = min(static_cast<int64_t>(r) * VB, n.last);
+    so = n.off_s + b;
+    sd = n.off_d + b;
+  } else {
+    so = n.off_s + static_cast<int64_t>(r) * n.inner_ss;
+    sd = n.off_d + static_cast<int64_t>(r) * n.inner_sd;
+  }
   for (int k = 0; k < n.nouter; ++k) {
     const uint32_t q2 = fdiv(q, n.outer[k]);
     const int64_t c = q - q2 * n.outer[k].d;
@@ -114,15 +135,15 @@ __device__ __forceinline__ void item_offsets(const Nest& n, uint32_t i, int64_t&
 template <int VB, int ITEMS, bool GUARDED>
 __device__ __forceinline__ void vec_items(const char* __restrict__ src, char* __restrict__ dst,
                                           const Nest& n, uint32_t base) {
-  using T = typename VecT<VB>::T;
-  T v[ITEMS];
+  using T = typename AnyT<VB>::T;
+  typename VecT<VB>::T v[ITEMS];
   int64_t doff[ITEMS];
 #pragma unroll
   for (int it = 0; it < ITEMS; ++it) {
     const uint32_t i = base + it * kThreads;
     if (!GUARDED || i < n.total) {
       int64_t so;
-      item_offsets(n, i, so, doff[it]);
+      item_offsets<VB>(n, i, so, doff[it]);
       v[it] = __builtin_nontemporal_load(reinterpret_cast<const T*>(src + so));
     }
   }
@@ -133,18 +154,124 @@ __device__ __forceinline__ void vec_items(const char* __restrict__ src, char* __
       __builtin_nontemporal_store(v[it], reinterpret_cast<T*>(dst + doff[it]));
 }
 
-// Each lane moves ITEMS items of VB bytes; all loads are issued before the
-// stores so several cache lines per lane are in flight.  Only the last
-// block predicates its items.
+// Block `block` of a nest of VB-byte items; only the last one predicates
+// its items.
 template <int VB, int ITEMS>
-__global__ __launch_bounds__(kThreads) void dma_vec_kernel(const char* __restrict__ src,
-                                                           char* __restrict__ dst, Nest n) {
-  const uint32_t first = blockIdx.x * (kThreads * ITEMS);
+__device__ __forceinline__ void vec_block(const char* __restrict__ src, char* __restrict__ dst, const Nest& n,
+                                          uint32_t block) {
+  const uint32_t first = block * (kThreads * ITEMS);
   const uint32_t base = first + threadIdx.x;
   if (first + kThreads * ITEMS <= n.total)
     vec_items<VB, ITEMS, false>(src, dst, n, base);
   else
     vec_items<VB, ITEMS, true>(src, dst, n, base);
+}
+
+template <int VB, int ITEMS>
+__global__ __launch_bounds__(kThreads) void dma_vec_kernel(const char* __restrict__ src,
+                                                           char* __restrict__ dst, Nest n) {
+  vec_block<VB, ITEMS>(src, dst, n, blockIdx.x);
+}
+
+// A vec nest of at most three outer loops whose byte offsets fit 32 bits: the
+// usual one.  Every argument is read in one batch at entry and the index is
+// taken apart by straight-line 32-bit code; dma_vec_kernel reads each outer
+// loop's arguments when it comes to it, a memory round trip apiece before
+// the first load.
+struct SmallNest {
+  uint32_t total, vb, last;        // items; bytes per item; where a run's last item starts
+  FastDiv inner, o0, o1;           // items per run; lengths of the first two outer loops (the third is the rest)
+  uint32_t ss[3], sd[3], off_s, off_d;  // bytes
+};
+
+#define SPYRE_PIN_SMALL(x)                                                                                       \
+  "+s"(x.total), "+s"(x.vb), "+s"(x.last), "+s"(x.inner.d), "+s"(x.inner.mul), "+s"(x.inner.shift), "+s"(x.o0.d), "+s"(x.o0.mul), \
+      "+s"(x.o0.shift), "+s"(x.o1.d), "+s"(x.o1.mul), "+s"(x.o1.shift), "+s"(x.ss[0]), "+s"(x.ss[1]), "+s"(x.ss[2]), \
+      "+s"(x.sd[0]), "+s"(x.sd[1]), "+s"(x.sd[2]), "+s"(x.off_s), "+s"(x.off_d)
+
+__device__ __forceinline__ void small_offsets(const SmallNest& n, uint32_t vb, uint32_t i, uint32_t& so, uint32_t& sd) {
+  const uint32_t q0 = fdiv(i, n.inner), q1 = fdiv(q0, n.o0), q2 = fdiv(q1, n.o1);
+  const uint32_t r = min((i - q0 * n.inner.d) * vb, n.last), c0 = q0 - q1 * n.o0.d, c1 = q1 - q2 * n.o1.d;
+  so = n.off_s + r + c0 * n.ss[0] + c1 * n.ss[1] + q2 * n.ss[2];
+  sd = n.off_d + r + c0 * n.sd[0] + c1 * n.sd[1] + q2 * n.sd[2];
+}
+
+template <int VB, int ITEMS>
+__device__ __forceinline__ void small_block(const char* src, char* dst, const SmallNest& n, uint32_t block) {
+  using T = typename AnyT<VB>::T;
+  typename VecT<VB>::T v[ITEMS];
+  uint32_t doff[ITEMS];
+  const uint32_t base = block * (kThreads * ITEMS) + threadIdx.x;
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it) {
+    const uint32_t i = base + it * kThreads;
+    uint32_t so;
+    small_offsets(n, VB, i, so, doff[it]);
+    if (i < n.total) v[it] = __builtin_nontemporal_load(reinterpret_cast<const T*>(src + so));
+  }
+  __builtin_amdgcn_sched_barrier(0);  // keep every load ahead of the stores
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it)
+    if (base + it * kThreads < n.total) __builtin_nontemporal_store(v[it], reinterpret_cast<T*>(dst + doff[it]));
+}
+
+// One such nest (blocks below `blocks`) and, in the same launch, another: a
+// tensor's whole sticks and the remainder of its rows.  A remainder is a few
+// thousand items; as a launch of its own it took 5.6-6.1 us beside a main
+// nest of 14.  fp32 [3, 1021, 2500] to its device layout: 20.2 us in two
+// launches, 17.2 in one of the general kernel, 13.1 here; fp16 [1000, 1000]
+// 9.8 and 4.8.  ITEMS: 4, or 1 for nests that would not fill the device with
+// four to a lane.
+template <int VB, int ITEMS>
+__global__ __launch_bounds__(kThreads) void dma_vec_pair_kernel(const char* __restrict__ src_arg,
+                                                                char* __restrict__ dst_arg, SmallNest a_arg,
+                                                                SmallNest b_arg, uint32_t blocks_arg) {
+  const char* src = src_arg;
+  char* dst = dst_arg;
+  SmallNest a = a_arg;
+  uint32_t blocks = blocks_arg;
+  asm volatile("" : "+s"(src), "+s"(dst), "+s"(blocks), SPYRE_PIN_SMALL(a));
+  if (blockIdx.x < blocks) {
+    small_block<VB, ITEMS>(src, dst, a, blockIdx.x);
+    return;
+  }
+  SmallNest b = b_arg;
+  asm volatile("" : SPYRE_PIN_SMALL(b));
+  const uint32_t block = blockIdx.x - blocks;
+  switch (b.vb) {
+    case 16: small_block<16, 1>(src, dst, b, block); break;
+    case 8: small_block<8, 1>(src, dst, b, block); break;
+    case 4: small_block<4, 1>(src, dst, b, block); break;
+    case 2: small_block<2, 1>(src, dst, b, block); break;
+    default: small_block<1, 1>(src, dst, b, block); break;
+  }
+}
+#undef SPYRE_PIN_SMALL
+
+// Several vec nests in one launch: blocks first[k] .. first[k + 1] - 1 run
+// nest k.
+constexpr int kMulti = 8;
+struct MultiNest {
+  Nest n[kMulti];
+  uint32_t first[kMulti];
+  uint32_t vb[kMulti];
+  int count;
+};
+
+__global__ __launch_bounds__(kThreads) void dma_vec_multi_kernel(const char* __restrict__ src,
+                                                                 char* __restrict__ dst, MultiNest m) {
+  int k = 0;
+  for (int i = 1; i < m.count; ++i)
+    if (blockIdx.x >= m.first[i]) k = i;
+  k = __builtin_amdgcn_readfirstlane(k);
+  const uint32_t block = blockIdx.x - m.first[k];
+  switch (m.vb[k]) {
+    case 16: vec_block<16, kItems>(src, dst, m.n[k], block); break;
+    case 8: vec_block<8, kItems>(src, dst, m.n[k], block); break;
+    case 4: vec_block<4, kItems>(src, dst, m.n[k], block); break;
+    case 2: vec_block<2, kItems>(src, dst, m.n[k], block); break;
+    default: vec_block<1, kItems>(src, dst, m.n[k], block); break;
+  }
 }
 
 // Stick-tile nest: a 128-byte stick (8 x 16 B) moved whole; loop A (nA
@@ -861,7 +988,7 @@ __global__ __launch_bounds__(kThreads) void dma_scalar_kernel(const char* __rest
   const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
   if (i >= n.total) return;
   int64_t so, sd;
-  item_offsets(n, i, so, sd);
+  item_offsets<0>(n, i, so, sd);
   *reinterpret_cast<T*>(dst + sd) = *reinterpret_cast<const T*>(src + so);
 }
 
@@ -940,8 +1067,7 @@ int check_launch(const char* what) {
 // and whose outer loops are `outer`; splits the launch along the outermost
 // loop when the item count exceeds 2^31.
 template <typename Launch>
-int launch_nest(const Loop& inner, std::vector<Loop> outer, int64_t off_s, int64_t off_d,
-                int64_t item_bytes, Launch&& launch) {
+int launch_nest(const Loop& inner, std::vector<Loop> outer, int64_t off_s, int64_t off_d, Launch&& launch) {
   int64_t per = inner.size;
   for (const Loop& o : outer) per *= o.size;
   if (per == 0) return SPYRE_OK;
@@ -956,7 +1082,7 @@ int launch_nest(const Loop& inner, std::vector<Loop> outer, int64_t off_s, int64
     for (int64_t c = 0; c < top.size; c += step) {
       std::vector<Loop> o2 = outer;
       o2.push_back({std::min(step, top.size - c), top.ss, top.sd});
-      const int rc = launch_nest(inner, o2, off_s + c * top.ss, off_d + c * top.sd, item_bytes, launch);
+      const int rc = launch_nest(inner, o2, off_s + c * top.ss, off_d + c * top.sd, launch);
       if (rc != SPYRE_OK) return rc;
     }
     return SPYRE_OK;
@@ -974,11 +1100,131 @@ int launch_nest(const Loop& inner, std::vector<Loop> outer, int64_t off_s, int64
   n.off_s = off_s;
   n.off_d = off_d;
   n.total = static_cast<uint32_t>(per);
-  (void)item_bytes;
   return launch(n);
 }
 
-int run_info(const char* src, char* dst, int esz, const spyre_stride_info& info, hipStream_t st) {
+// Whole sticks of up to this many bytes go with the description's other nests
+// in one launch instead of through a tile kernel of their own.  Measured, two
+// launches against one: fp32 [512, 4100] 9.1 / 6.8 us, [2048, 4100] 14.4 /
+// 13.7, [3, 1024, 4100] (48 MiB) 22.9 / 20.6; [4000, 4100] (63 MiB) 28.1 / 33.8.
+constexpr int64_t kHeldBytes = int64_t{48} << 20;
+
+// A vec nest held back to share a launch with others.
+struct VecNest {
+  Nest n;
+  int vb;
+};
+
+int launch_vec(const char* src, char* dst, const VecNest& v, hipStream_t st) {
+  const dim3 grid((v.n.total + kThreads * kItems - 1) / (kThreads * kItems));
+  switch (v.vb) {
+    case 16: dma_vec_kernel<16, kItems><<<grid, kThreads, 0, st>>>(src, dst, v.n); break;
+    case 8: dma_vec_kernel<8, kItems><<<grid, kThreads, 0, st>>>(src, dst, v.n); break;
+    case 4: dma_vec_kernel<4, kItems><<<grid, kThreads, 0, st>>>(src, dst, v.n); break;
+    case 2: dma_vec_kernel<2, kItems><<<grid, kThreads, 0, st>>>(src, dst, v.n); break;
+    default: dma_vec_kernel<1, kItems><<<grid, kThreads, 0, st>>>(src, dst, v.n); break;
+  }
+  return check_launch("dma_vec_kernel");
+}
+
+// n as a SmallNest, if it is one: offsets and strides non-negative, the far
+// end of either side within 32 bits.
+bool small_nest(const VecNest& v, SmallNest& s) {
+  const Nest& n = v.n;
+  if (n.nouter > 3) return false;
+  const int64_t run = static_cast<int64_t>(n.inner.d) * v.vb;
+  int64_t end_s = n.off_s + run, end_d = n.off_d + run;
+  if (n.off_s < 0 || n.off_d < 0) return false;
+  for (int k = 0; k < n.nouter; ++k) {
+    if (n.ss[k] < 0 || n.sd[k] < 0) return false;
+    end_s += (static_cast<int64_t>(n.outer[k].d) - 1) * n.ss[k];
+    end_d += (static_cast<int64_t>(n.outer[k].d) - 1) * n.sd[k];
+  }
+  // strides wrap like the offsets they sum to; a length-1 loop's may be anything
+  if (end_s >= (int64_t{1} << 32) || end_d >= (int64_t{1} << 32)) return false;
+  const FastDiv one = make_fastdiv(1);
+  s = SmallNest{n.total, static_cast<uint32_t>(v.vb), static_cast<uint32_t>(n.last), n.inner, n.nouter > 0 ? n.outer[0] : one,
+                n.nouter > 1 ? n.outer[1] : one, {}, {}, static_cast<uint32_t>(n.off_s), static_cast<uint32_t>(n.off_d)};
+  for (int k = 0; k < n.nouter; ++k) {
+    s.ss[k] = static_cast<uint32_t>(n.ss[k]);
+    s.sd[k] = static_cast<uint32_t>(n.sd[k]);
+  }
+  return true;
+}
+
+// One or two nests by dma_vec_pair_kernel; false: not that kind.
+bool launch_pair(const char* src, char* dst, const std::vector<VecNest>& vs, hipStream_t st) {
+  SmallNest a, b{};
+  if (vs.empty() || vs.size() > 2) return false;
+  const bool swap = vs.size() == 2 && vs[1].n.total > vs[0].n.total;  // the larger one first
+  const VecNest& va = vs[swap ? 1 : 0];
+  if (!small_nest(va, a) || (vs.size() == 2 && !small_nest(vs[swap ? 0 : 1], b))) return false;
+  const int64_t cus = dma_device_cus() > 0 ? dma_device_cus() : 256;
+  const bool wide = a.total > 2 * cus * kThreads;
+  const uint32_t per = kThreads * (wide ? kItems : 1);
+  const uint32_t blocks = (a.total + per - 1) / per;
+  const dim3 grid(blocks + (b.total + kThreads - 1) / kThreads);
+  auto go = [&](auto vb_c) {
+    constexpr int VB = decltype(vb_c)::value;
+    if (wide)
+      dma_vec_pair_kernel<VB, kItems><<<grid, kThreads, 0, st>>>(src, dst, a, b, blocks);
+    else
+      dma_vec_pair_kernel<VB, 1><<<grid, kThreads, 0, st>>>(src, dst, a, b, blocks);
+  };
+  switch (va.vb) {
+    case 16: go(std::integral_constant<int, 16>{}); break;
+    case 8: go(std::integral_constant<int, 8>{}); break;
+    case 4: go(std::integral_constant<int, 4>{}); break;
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    default: go(std::integral_constant<int, 1>{}); break;
+  }
+  return true;
+}
+
+int launch_vecs(const char* src, char* dst, const std::vector<VecNest>& vs, hipStream_t st) {
+  if (launch_pair(src, dst, vs, st)) return check_launch("dma_vec_pair_kernel");
+  for (size_t i = 0; i < vs.size(); i += kMulti) {
+    const size_t count = std::min<size_t>(kMulti, vs.size() - i);
+    int rc;
+    if (count == 1) {
+      rc = launch_vec(src, dst, vs[i], st);
+    } else {
+      MultiNest m{};
+      m.count = static_cast<int>(count);
+      uint32_t blocks = 0;  // at most kMulti x 2^30 items / 1024
+      for (size_t k = 0; k < count; ++k) {
+        m.n[k] = vs[i + k].n;
+        m.vb[k] = static_cast<uint32_t>(vs[i + k].vb);
+        m.first[k] = blocks;
+        blocks += (vs[i + k].n.total + kThreads * kItems - 1) / (kThreads * kItems);
+      }
+      dma_vec_multi_kernel<<<dim3(blocks), kThreads, 0, st>>>(src, dst, m);
+      rc = check_launch("dma_vec_multi_kernel");
+    }
+    if (rc != SPYRE_OK) return rc;
+  }
+  return SPYRE_OK;
+}
+
+// Runs of `row` bytes by the vec kernel: items of 16 bytes, or as many as a
+// shorter run holds, wherever they start.
+int run_vec(const char* src, char* dst, int64_t row, const std::vector<Loop>& outer, int64_t off_s, int64_t off_d,
+            hipStream_t st, std::vector<VecNest>* held) {
+  std::vector<VecNest> vs;
+  int b = 16;
+  while (b > row) b /= 2;
+  const int rc = launch_nest({(row + b - 1) / b, b, b}, outer, off_s, off_d, [&](Nest& n) {
+    n.last = row - b;
+    (held ? *held : vs).push_back({n, b});
+    return static_cast<int>(SPYRE_OK);
+  });
+  return rc != SPYRE_OK || held ? rc : launch_vecs(src, dst, vs, st);
+}
+
+// Moves one nest; held non-null: a nest the vec kernel serves is appended
+// there instead of launched.
+int run_info(const char* src, char* dst, int esz, const spyre_stride_info& info, hipStream_t st,
+             std::vector<VecNest>* held) {
   for (int q = 0; q < info.rank; ++q)
     if (info.size[q] == 0) return SPYRE_OK;
   std::vector<Loop> loops = normalise(info, esz);
@@ -1026,9 +1272,11 @@ int run_info(const char* src, char* dst, int esz, const spyre_stride_info& info,
       tail.stride_src[0] = tail.stride_dst[0] = 1;
       tail.offset_src = info.offset_src + done / esz;
       tail.offset_dst = info.offset_dst + done / esz;
-      return run_info(src, dst, esz, tail, st);
+      return run_info(src, dst, esz, tail, st, held);
     }
-    if (vb == 16 && row == 128) {
+    int64_t bytes = row;
+    for (const Loop& o : outer) bytes *= o.size;
+    if (vb == 16 && row == 128 && !(held && bytes <= kHeldBytes)) {
       // stick tile: loop A continues the stick in dst, loop B in src.
       int ai = -1, bi = -1;
       for (size_t k = 0; k < outer.size(); ++k) {
@@ -1195,18 +1443,7 @@ int run_info(const char* src, char* dst, int esz, const spyre_stride_info& info,
         }
       }
     }
-    const Loop inner{row / vb, vb, vb};
-    return launch_nest(inner, outer, off_s, off_d, vb, [&](const Nest& n) {
-      const dim3 grid((n.total + kThreads * kItems - 1) / (kThreads * kItems));
-      switch (vb) {
-        case 16: dma_vec_kernel<16, kItems><<<grid, kThreads, 0, st>>>(src, dst, n); break;
-        case 8: dma_vec_kernel<8, kItems><<<grid, kThreads, 0, st>>>(src, dst, n); break;
-        case 4: dma_vec_kernel<4, kItems><<<grid, kThreads, 0, st>>>(src, dst, n); break;
-        case 2: dma_vec_kernel<2, kItems><<<grid, kThreads, 0, st>>>(src, dst, n); break;
-        default: dma_vec_kernel<1, kItems><<<grid, kThreads, 0, st>>>(src, dst, n); break;
-      }
-      return check_launch("dma_vec_kernel");
-    });
+    return run_vec(src, dst, row, outer, off_s, off_d, st, held);
   }
 
   // transpose: loop A unit-stride in src, loop B unit-stride in dst.
@@ -1349,10 +1586,14 @@ int run_info(const char* src, char* dst, int esz, const spyre_stride_info& info,
     }
   }
 
+  // Elements apart on both sides, beside other nests (the remainder of rows
+  // one element longer than whole sticks): runs of one element in their launch.
+  if (held && loops.size() <= 3) return run_vec(src, dst, esz, loops, off_s, off_d, st, held);
+
   // scalar fallback: innermost-by-dst loop first.
   const Loop inner{loops[0].size, loops[0].ss, loops[0].sd};
   std::vector<Loop> outer(loops.begin() + 1, loops.end());
-  return launch_nest(inner, outer, off_s, off_d, esz, [&](const Nest& n) {
+  return launch_nest(inner, outer, off_s, off_d, [&](const Nest& n) {
     const dim3 grid((n.total + kThreads - 1) / kThreads);
     switch (esz) {
       case 1: dma_scalar_kernel<1><<<grid, kThreads, 0, st>>>(src, dst, n); break;
@@ -1365,6 +1606,99 @@ int run_info(const char* src, char* dst, int esz, const spyre_stride_info& info,
 }
 
 }  // namespace
+
+// Whether two nests write no dst element in common, as far as their strides
+// show it (false: they may); planner descriptions' do.  Two views of it:
+//  * loops the nests share (same length and stride) step over everything
+//    below them, and what is below (each nest's other loops, from its offset)
+//    is two intervals apart: a row's whole sticks and its remainder in host
+//    order;
+//  * with all dst strides as the places of one number system (each place
+//    worth more than everything below it), each nest is a box of digits, and
+//    some place's digits are apart: the same two in stick order.
+static bool writes_apart(const spyre_stride_info& x, const spyre_stride_info& y) {
+  struct L {
+    int64_t size, sd;
+  };
+  struct List {  // at most both nests' loops
+    L v[2 * SPYRE_MAX_RANK];
+    int n = 0;
+    L* begin() { return v; }
+    L* end() { return v + n; }
+    void push(L l) { v[n++] = l; }
+  };
+  List lx, ly, common;
+  auto loops = [](const spyre_stride_info& s, List& l) {
+    for (int q = 0; q < s.rank; ++q) {
+      if (s.size[q] == 0 || (s.size[q] > 1 && (s.stride_dst[q] <= 0 || s.stride_dst[q] >= (int64_t{1} << 40)))) return false;
+      if (s.size[q] > 1) l.push({s.size[q], s.stride_dst[q]});
+    }
+    return true;
+  };
+  if (!loops(x, lx) || !loops(y, ly)) return false;
+  const int64_t base = std::min(x.offset_dst, y.offset_dst);
+  {
+    int64_t x1 = x.offset_dst - base, y1 = y.offset_dst - base;
+    const int64_t x0 = x1, y0 = y1;
+    bool taken[SPYRE_MAX_RANK] = {};
+    for (const L& l : lx) {
+      int k = 0;
+      while (k < ly.n && (taken[k] || ly.v[k].size != l.size || ly.v[k].sd != l.sd)) ++k;
+      if (k < ly.n) {
+        common.push(l);
+        taken[k] = true;
+      } else {
+        x1 += (l.size - 1) * l.sd;
+      }
+    }
+    for (int k = 0; k < ly.n; ++k)
+      if (!taken[k]) y1 += (ly.v[k].size - 1) * ly.v[k].sd;
+    bool apart = x1 < y0 || y1 < x0;
+    int64_t below = std::max(x1, y1);
+    std::sort(common.begin(), common.end(), [](const L& p, const L& q) { return p.sd < q.sd; });
+    for (const L& l : common) {
+      apart = apart && l.sd > below;
+      below += (l.size - 1) * l.sd;
+    }
+    if (apart) return true;
+  }
+  int64_t places[2 * SPYRE_MAX_RANK];
+  int np = 0;
+  for (const L& l : lx) places[np++] = l.sd;
+  for (const L& l : ly) places[np++] = l.sd;
+  std::sort(places, places + np);
+  np = static_cast<int>(std::unique(places, places + np) - places);
+  auto digits = [&](int64_t rest, List& l, L* d) {  // per place: {lowest, highest}
+    for (int p = np; p-- > 0;) {
+      d[p] = {rest / places[p], rest / places[p]};
+      rest %= places[p];
+    }
+    for (const L& o : l) {
+      L& v = d[std::lower_bound(places, places + np, o.sd) - places];
+      if (v.size != v.sd) return false;  // two loops of one stride
+      v.sd += o.size - 1;
+    }
+    return rest == 0;
+  };
+  L dx[2 * SPYRE_MAX_RANK], dy[2 * SPYRE_MAX_RANK];
+  if (!digits(x.offset_dst - base, lx, dx) || !digits(y.offset_dst - base, ly, dy)) return false;
+  int64_t below = 0;  // the most that the places below add up to
+  bool apart = false;
+  for (int p = 0; p < np; ++p) {
+    const int64_t most = std::max(dx[p].sd, dy[p].sd);
+    if (places[p] <= below || most >= (int64_t{1} << 22)) return false;
+    below += most * places[p];
+    apart = apart || dx[p].sd < dy[p].size || dy[p].sd < dx[p].size;
+  }
+  return apart;
+}
+
+static bool disjoint_writes(const spyre_stride_info* infos, int n) {
+  for (int i = 0; i < n; ++i)
+    for (int j = 0; j < i; ++j)
+      if (!writes_apart(infos[i], infos[j])) return false;
+  return true;
+}
 
 // Largest element index a loop nest touches on one side (strides >= 0).
 static bool nest_extent(const spyre_stride_info& s, bool src_side, int64_t& hi) {
@@ -1409,10 +1743,17 @@ extern "C" int spyre_dma_copy(const void* src, size_t src_bytes, void* dst, size
                   static_cast<long long>((hd + 1) * elem_bytes), dst_bytes);
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
+  // Nests that write apart from each other, between buffers that are apart,
+  // may run in any order, so their vec parts share launches; others run one
+  // after the other.
+  std::vector<VecNest> held;
+  const uintptr_t s0 = reinterpret_cast<uintptr_t>(src), d0 = reinterpret_cast<uintptr_t>(dst);
+  const bool share = n_infos > 1 && (s0 + src_bytes <= d0 || d0 + dst_bytes <= s0) && disjoint_writes(infos, n_infos);
+  if (share) held.reserve(static_cast<size_t>(n_infos) + 1);
   for (int i = 0; i < n_infos; ++i) {
     const int rc = run_info(static_cast<const char*>(src), static_cast<char*>(dst), elem_bytes,
-                            infos[i], st);
+                            infos[i], st, share ? &held : nullptr);
     if (rc != SPYRE_OK) return rc;
   }
-  return SPYRE_OK;
+  return launch_vecs(static_cast<const char*>(src), static_cast<char*>(dst), held, st);
 }
