@@ -188,6 +188,23 @@ int spyre_paged_decode_attn_f16(const void* q, const void* k_cache, const void* 
                                 int D, int page_size, int64_t num_pages, int max_context_len,
                                 int split_tokens, float scale, void* stream);
 
+/* spyre_paged_decode_attn_f16 with a workspace of its own for every call in
+ * flight: calls of few (sequence, KV head) pairs then spread each chunk over
+ * several workgroups, whose partials and arrival flags use the workspace
+ * whatever the context length.  Same arguments, number of kernels and results, bit for
+ * bit.  The spread form needs spyre_paged_decode_attn_call_workspace_bytes
+ * bytes, 16-byte aligned (asked of the current device; never less than
+ * spyre_paged_decode_attn_workspace_bytes); with less the call is
+ * spyre_paged_decode_attn_f16's.  No reference counterpart, as above. */
+size_t spyre_paged_decode_attn_call_workspace_bytes(int B, int Hq, int Hkv, int D, int max_context_len,
+                                                    int split_tokens);
+int spyre_paged_decode_attn_call_f16(const void* q, const void* k_cache, const void* v_cache,
+                                     const int32_t* block_table, int64_t bt_stride,
+                                     const int32_t* context_lens, void* out, float* lse,
+                                     void* workspace, size_t workspace_bytes, int B, int Hq, int Hkv,
+                                     int D, int page_size, int64_t num_pages, int max_context_len,
+                                     int split_tokens, float scale, void* stream);
+
 /* Kernels one spyre_paged_decode_attn_f16 call of these sizes launches on
  * the current device: 1 when every context fits one chunk or the chunks
  * merge inside the split kernel (its work list, B * Hkv * chunks items, fits

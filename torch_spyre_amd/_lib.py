@@ -82,6 +82,11 @@ SIGNATURES = {
                                             c_void_p, c_void_p, c_void_p, c_size_t, c_int, c_int,
                                             c_int, c_int, c_int, c_int64, c_int, c_int, c_float,
                                             c_void_p]),
+    "spyre_paged_decode_attn_call_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int]),
+    "spyre_paged_decode_attn_call_f16": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p,
+                                                 c_void_p, c_void_p, c_void_p, c_size_t, c_int, c_int,
+                                                 c_int, c_int, c_int, c_int64, c_int, c_int, c_float,
+                                                 c_void_p]),
     "spyre_paged_decode_attn_split_f16": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p,
                                                   c_void_p, c_size_t, c_int, c_int, c_int, c_int, c_int,
                                                   c_int64, c_int, c_int, c_float, c_void_p]),

@@ -152,7 +152,14 @@ class _DecodeArgs:
                              f"{block_table.shape[1]} pages")
         self.scale = 1.0 / math.sqrt(D) if scale is None else float(scale)
         need = workspace_bytes(B, Hq, Hkv, D, max_context_len, split_tokens)
+        # A workspace of this object's own: small grids may spread over it.  A
+        # caller's may be shared by calls in flight, as one-chunk calls allow.
+        L = _lib.lib()
+        self.call_fn = L.spyre_paged_decode_attn_call_f16 if workspace is None else L.spyre_paged_decode_attn_f16
         if workspace is None:
+            with torch.cuda.device(q.device):
+                need = max(need, L.spyre_paged_decode_attn_call_workspace_bytes(B, Hq, Hkv, D, max_context_len,
+                                                                                split_tokens))
             workspace = torch.empty(max(need, 4), dtype=torch.uint8, device=q.device)
         elif workspace.numel() * workspace.element_size() < need:
             raise ValueError(f"workspace holds {workspace.numel() * workspace.element_size()} bytes, need {need}")
@@ -195,7 +202,7 @@ def paged_decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
     if out.shape != q.shape or out.dtype != q.dtype or not out.is_contiguous():
         raise ValueError("out must be contiguous and shaped like q")
     lse = torch.empty((a.B, a.Hq), dtype=torch.float32, device=q.device) if return_lse else None
-    rc = _lib.lib().spyre_paged_decode_attn_f16(
+    rc = a.call_fn(
         q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_table.data_ptr(),
         block_table.stride(0), context_lens.data_ptr(), out.data_ptr(),
         lse.data_ptr() if lse is not None else None, a.ws.data_ptr(), a.ws_bytes, a.B, a.Hq, a.Hkv,
@@ -209,8 +216,9 @@ class PagedDecode:
 
     Checks shapes, dtypes and the workspace once; each launch then only
     passes the stored device pointers to the library (the tensors must stay
-    alive and keep their storage).  ``__call__`` is the single-call entry
-    (one kernel when max_context_len fits one chunk); ``split()`` and
+    alive and keep their storage; the launches of one object follow one
+    another, as they share its workspace).  ``__call__`` is the single-call
+    entry (one kernel when max_context_len fits one chunk); ``split()`` and
     ``merge()`` launch the two passes separately (the split pass then
     writes every chunk's partial to the workspace).  Each launch goes to the
     stream current at that moment, so the calls can be captured into a HIP
@@ -236,7 +244,7 @@ class PagedDecode:
         if a.ws.data_ptr() % 16 and a.max_ctx > CHUNK_WAVES * a.split:
             self.passes = 2  # a workspace aligned to less than 16 bytes takes the merge pass
         L = _lib.lib()
-        self._call_fn = L.spyre_paged_decode_attn_f16
+        self._call_fn = a.call_fn
         self._split_fn = L.spyre_paged_decode_attn_split_f16
         self._merge_fn = L.spyre_paged_decode_attn_merge_f16
         lse_ptr = lse.data_ptr() if lse is not None else None

@@ -121,6 +121,17 @@ __host__ __device__ __forceinline__ int chunks_of(int ctx, int chunk_pages) {
   return p == 0 ? 1 : p / chunk_pages + (p % chunk_pages != 0);
 }
 
+// Pages [w0, w1) of wavefront w of W of chunk c of nch: chunks are equal
+// shares of a sequence's pages, wavefronts equal shares of a chunk's.
+template <int W>
+__device__ __forceinline__ void wave_pages(int n_pages, int nch, int c, int w, int& w0, int& w1) {
+  const int cp0 = static_cast<int>(static_cast<int64_t>(c) * n_pages / nch);
+  const int cp1 = static_cast<int>(static_cast<int64_t>(c + 1) * n_pages / nch);
+  const int nc = cp1 - cp0;
+  w0 = cp0 + static_cast<int>(static_cast<int64_t>(w) * nc / W);
+  w1 = cp0 + static_cast<int>(static_cast<int64_t>(w + 1) * nc / W);
+}
+
 // Work-list mode handles batches up to this many sequences (their split
 // counts are prefix-summed in LDS); larger batches use grid mode.
 #ifndef SPYRE_DECODE_LIST_MAX
@@ -784,12 +795,8 @@ __device__ __forceinline__ void run_item(const SplitArgs& a, int b, int c, int k
   const int ctx = min(max(ctx_raw, 0), a.max_ctx);
   const int n_pages = pages_of(ctx);
   const int nch = chunks_of(ctx, a.chunk_pages);
-  // Chunk c holds pages [cp0, cp1); wavefront w an equal share of them.
-  const int cp0 = static_cast<int>(static_cast<int64_t>(c) * n_pages / nch);
-  const int cp1 = static_cast<int>(static_cast<int64_t>(c + 1) * n_pages / nch);
-  const int nc = cp1 - cp0;
-  const int w0 = cp0 + static_cast<int>(static_cast<int64_t>(wave) * nc / W);
-  const int w1 = cp0 + static_cast<int>(static_cast<int64_t>(wave + 1) * nc / W);
+  int w0, w1;
+  wave_pages<W>(n_pages, nch, c, wave, w0, w1);
   f32x4 o[DB];
   float m, l;
   stream_pages<D, DENSE, MK>(a, b, kvh, w0, w1 - w0, ctx, lane, o, m, l);
@@ -953,6 +960,153 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void decode_split_list_ker
     if (__builtin_amdgcn_readfirstlane(s_pre[mid]) <= bs) lo = mid; else hi = mid;
   }
   run_item<D>(a, lo, bs - __builtin_amdgcn_readfirstlane(s_pre[lo]), kvh, wave, lane);
+}
+
+// A chunk's kWaves wavefronts spread over kWaves / S workgroups of S, for
+// grids that leave most compute units idle (spread_waves).  One compute unit
+// draws about 46 GB/s from memory however many of its wavefronts ask: a chunk
+// of 4096 tokens of one KV head took 59 us in one workgroup and takes 21 in
+// eight (B 1 x 32 / 8 heads: 700 tokens 14.4 -> 9.2 us, 4096 59.1 -> 20.7,
+// 32768 63.5 -> 32.5; B 8 x 2048 32.0 -> 16.6, B 16 x 4096 60.5 -> 44.9).
+// Every wavefront streams the pages it would stream there, its partial goes
+// to the workspace, and whichever workgroup sees all of a (sequence, KV
+// head)'s arrival flags (as merge_in_kernel: possibly more than one, all
+// writing the same bits) folds the wavefronts of each chunk and merges the
+// chunks with run_item's and merge_row4's arithmetic in their order: the
+// results are bit for bit those of decode_split_list_kernel.  Workspace: O
+// [B, Hkv, max_chunks, kWaves, g, D], (m, l) alike, a flag per workgroup.
+constexpr int kSpreadChunks = 16;  // chunks at most (one group of merge_row4)
+constexpr int kSpreadWaves = 4;    // wavefronts launched per workgroup: S stream, all merge
+static_assert(kSpreadChunks <= kMergeChunk, "the chunks of a sequence are one merge group");
+
+template <int D, int S>
+__global__ __launch_bounds__(kSpreadWaves * 64, kWavesPerSimd) void decode_spread_kernel(SplitArgs a) {
+  static_assert(S <= kSpreadWaves, "S wavefronts of the workgroup stream");
+  constexpr int N = kWaves / S;  // workgroups of a chunk
+  constexpr int DB = D / 16, D4 = D / 4;
+  constexpr int kAuxDevice = 16;  // sc1: device scope
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+  const int c = blockIdx.x / N, wg = blockIdx.x % N, kvh = blockIdx.y, b = blockIdx.z;
+  const int ctx_raw = a.ctx_lens[b];
+  const int ctx = min(max(ctx_raw, 0), a.max_ctx);
+  const int n_pages = pages_of(ctx), nch = chunks_of(ctx, a.chunk_pages);
+  if (c >= nch) return;
+  // A few pages: one workgroup, a page per wavefront, and no round trips of
+  // partials and flags (about 1.6 us; with max_context_len 4096, 64 tokens
+  // took 6.6 us by them and take 5.3, 190 tokens 7.0 and 7.7).  The same
+  // bits: of kWaves wavefronts those without a page would add nothing, and
+  // the others fold in the order of their pages.
+  constexpr int kFew = S == kSpreadWaves ? 4 : 2;
+  static_assert(kFew <= kSpreadWaves, "a page per wavefront");
+  if (n_pages <= kFew) {
+    if (wg == 0) run_item<D, false, kSpreadWaves>(a, b, 0, kvh, wave, lane);
+    return;
+  }
+  const Rsrc wr = __builtin_amdgcn_make_buffer_rsrc(a.ws, 0, 0x7ffffff0, kRsrcWord3);
+  const uint32_t parts = static_cast<uint32_t>(a.B) * a.Hkv * a.max_chunks * kWaves * a.g;  // rows of partials
+  const uint32_t ml_off = parts * D * 4, fl_off = ml_off + parts * 8;
+  const uint32_t pair = static_cast<uint32_t>(b) * a.Hkv + kvh;
+  const uint32_t row0 = pair * a.max_chunks * kWaves * a.g;  // row of chunk s, wavefront v, head col: + (s kWaves + v) g + col
+  const uint32_t fl0 = fl_off + pair * a.max_chunks * N * 4;
+  if (wave < S) {
+    const int w = wg * S + wave;
+    int w0, w1;
+    wave_pages<kWaves>(n_pages, nch, c, w, w0, w1);
+    f32x4 o[DB];
+    float m, l;
+    stream_pages<D>(a, b, kvh, w0, w1 - w0, ctx, lane, o, m, l);
+    const int col = lane & 15, grp = lane >> 4;
+    const uint32_t row = row0 + static_cast<uint32_t>((c * kWaves + w) * a.g + col);
+    if (col < a.g) {
+#pragma unroll
+      for (int db = 0; db < DB; ++db)  // features 16 db + 4 grp .. + 3
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o[db]), wr, (row * D + 16 * db + 4 * grp) * 4, 0,
+                                               kAuxDevice);
+      if (grp == 0)
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, f32x2{m, l}), wr, ml_off + row * 8, 0, kAuxDevice);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();  // every partial store of the workgroup done
+  __shared__ int s_merge;
+  const int nf = nch * N;  // flags of this sequence and KV head
+  if (wave == 0) {
+    if (lane == 0) __builtin_amdgcn_raw_buffer_store_b32(a.ticket, wr, fl0 + (c * N + wg) * 4, 0, kAuxDevice);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    bool seen = true;
+    for (int f = lane; f < nf; f += 64)
+      seen = seen && __builtin_amdgcn_raw_buffer_load_b32(wr, fl0 + f * 4, 0, kAuxDevice) == a.ticket;
+    const bool all = __all(seen);
+    if (lane == 0) s_merge = all ? 1 : 0;
+  }
+  __syncthreads();
+  if (!s_merge) return;
+
+  for (int u = static_cast<int>(threadIdx.x); u < a.g * D4; u += kSpreadWaves * 64) {
+    const int col = u / D4, d = 4 * (u - col * D4);
+    // Chunk s's wavefronts: (m, l) and 4 features of O, then their fold.
+    f32x2 ml[kWaves];
+    auto load_ml = [&](int s) {
+#pragma unroll
+      for (int v = 0; v < kWaves; ++v)
+        ml[v] = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(
+                                              wr, ml_off + (row0 + (s * kWaves + v) * a.g + col) * 8, 0, kAuxDevice));
+    };
+    auto max_m = [&] {
+      float x = -INFINITY;
+#pragma unroll
+      for (int v = 0; v < kWaves; ++v) x = fmaxf(x, ml[v][0]);
+      return x;
+    };
+    auto fold = [&](int s, float& M, float& L, f32x4& O) {
+      f32x4 x[kWaves];
+      load_ml(s);
+#pragma unroll
+      for (int v = 0; v < kWaves; ++v)
+        x[v] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                             wr, ((row0 + (s * kWaves + v) * a.g + col) * D + d) * 4, 0, kAuxDevice));
+      M = max_m();
+      L = 0.f;
+      O = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int v = 0; v < kWaves; ++v) {
+        const float sc = M == -INFINITY ? 0.f : fast_exp2(ml[v][0] - M);
+        L = __builtin_fmaf(ml[v][1], sc, L);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) O[e] = __builtin_fmaf(x[v][e], sc, O[e]);
+      }
+    };
+    float M = -INFINITY, L = 0.f;
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (nch == 1) {
+      fold(0, M, L, acc);
+    } else {
+      for (int s = 0; s < nch; ++s) {
+        load_ml(s);
+        M = fmaxf(M, max_m());
+      }
+      const float mu = M == -INFINITY ? 0.f : M;
+      for (int s = 0; s < nch; ++s) {
+        float Mc, Lc;
+        f32x4 Oc;
+        fold(s, Mc, Lc, Oc);
+        const float wt = fast_exp2(Mc - mu);
+        L = __builtin_fmaf(Lc, wt, L);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(Oc[e], wt, acc[e]);
+      }
+    }
+    const int64_t row = static_cast<int64_t>(b) * a.Hq + kvh * a.g + col;
+    const bool none = ctx == 0 || L == 0.f;
+    const float inv = ctx_raw > a.max_ctx ? NAN : none ? 0.f : 1.f / L;
+    f16x4 rv;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) rv[e] = to_f16(acc[e] * inv);
+    *reinterpret_cast<f16x4*>(a.out + row * D + d) = rv;
+    if (a.lse && d == 0) a.lse[row] = none ? -INFINITY : (M + log2f(L)) * kLn2;
+  }
+  for (int f = static_cast<int>(threadIdx.x); f < nf; f += kSpreadWaves * 64)
+    __builtin_amdgcn_raw_buffer_store_b32(0u, wr, fl0 + f * 4, 0, kAuxDevice);
 }
 
 // Dense decode: item x = ((b Hkv + kvh) max_chunks + c); every sequence has
@@ -1236,6 +1390,27 @@ bool merges_in_kernel(int B, int Hq, int Hkv, int D, int max_context_len, int sp
          spyre_paged_decode_attn_workspace_bytes(B, Hq, Hkv, D, max_context_len, split_tokens) < (size_t{1} << 31);
 }
 
+// Wavefronts per workgroup of decode_spread_kernel (1, 2 or 4) for a call of
+// these sizes, 0 where it does not pay: the least whose workgroups still
+// find a compute unit each.  Twice as many lost it: B 12 x 4096 tokens 36.3 us
+// at one each and 41.1 at two, B 24 (192 items) 62.7 unspread and 75.9.
+constexpr int kSpreadPages = 3;  // pages at least: below, one workgroup has a page per wavefront
+int spread_waves(int B, int Hkv, int D, int max_context_len, int split_tokens) {
+  const int64_t slots = split_slots(D);
+  const int64_t chunks = max_chunks_for(max_context_len, split_tokens);
+  if (slots <= 0 || pages_of(max_context_len) < kSpreadPages || chunks > kSpreadChunks) return 0;
+  const int64_t items = static_cast<int64_t>(B) * Hkv * chunks;
+  for (int S = 1; S < kWaves; S *= 2)
+    if (items * (kWaves / S) <= slots) return S;
+  return 0;
+}
+
+// Its workspace: a partial per wavefront, a flag per workgroup of one.
+size_t spread_bytes(int B, int Hq, int Hkv, int D, int max_context_len, int split_tokens) {
+  return static_cast<size_t>(B) * Hkv * max_chunks_for(max_context_len, split_tokens) * kWaves *
+         (static_cast<size_t>(Hq / Hkv) * (D + 2) + 1) * sizeof(float);
+}
+
 int launch_split(const Plan& p, hipStream_t st) {
   if (p.list && p.D == 128)
     decode_split_list_kernel<128><<<p.g1, kThreads, 0, st>>>(p.sa);
@@ -1306,6 +1481,51 @@ extern "C" int spyre_paged_decode_attn_kernels(int B, int Hq, int Hkv, int D, in
                 SPYRE_EINVAL, "bad decode sizes");
   if (max_chunks_for(max_context_len, split_tokens) <= 1) return 1;
   return merges_in_kernel(B, Hq, Hkv, D, max_context_len, split_tokens) ? 1 : 2;
+}
+
+extern "C" size_t spyre_paged_decode_attn_call_workspace_bytes(int B, int Hq, int Hkv, int D, int max_context_len,
+                                                                int split_tokens) {
+  const size_t base = spyre_paged_decode_attn_workspace_bytes(B, Hq, Hkv, D, max_context_len, split_tokens);
+  if (base == 0 || spread_waves(B, Hkv, D, max_context_len, split_tokens) == 0) return base;
+  return std::max(base, spread_bytes(B, Hq, Hkv, D, max_context_len, split_tokens));
+}
+
+extern "C" int spyre_paged_decode_attn_call_f16(const void* q, const void* k_cache, const void* v_cache,
+                                                const int32_t* block_table, int64_t bt_stride,
+                                                const int32_t* context_lens, void* out, float* lse,
+                                                void* workspace, size_t workspace_bytes, int B, int Hq, int Hkv,
+                                                int D, int page_size, int64_t num_pages, int max_context_len,
+                                                int split_tokens, float scale, void* stream) {
+  spyre_hip::clear_error();
+  Plan p;
+  const int rc = plan_attn(q, k_cache, v_cache, block_table, bt_stride, context_lens, out, lse, workspace,
+                           workspace_bytes, B, Hq, Hkv, D, page_size, num_pages, max_context_len, split_tokens,
+                           scale, true, true, p);
+  if (rc != SPYRE_OK) return rc;
+  const int S = spread_waves(B, Hkv, D, max_context_len, split_tokens);
+  if (S == 0 || reinterpret_cast<uintptr_t>(workspace) % 16 != 0 || reinterpret_cast<uintptr_t>(out) % 8 != 0 ||
+      workspace_bytes < spread_bytes(B, Hq, Hkv, D, max_context_len, split_tokens))
+    return spyre_paged_decode_attn_f16(q, k_cache, v_cache, block_table, bt_stride, context_lens, out, lse, workspace,
+                                       workspace_bytes, B, Hq, Hkv, D, page_size, num_pages, max_context_len,
+                                       split_tokens, scale, stream);
+  p.sa.ticket = spyre_hip::next_call_ticket();
+  const dim3 grid(static_cast<unsigned>(p.sa.max_chunks * (kWaves / S)), Hkv, B);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  auto go = [&](auto d_c) {
+    constexpr int DD = decltype(d_c)::value;
+    switch (S) {
+      case 1: decode_spread_kernel<DD, 1><<<grid, kSpreadWaves * 64, 0, st>>>(p.sa); break;
+      case 2: decode_spread_kernel<DD, 2><<<grid, kSpreadWaves * 64, 0, st>>>(p.sa); break;
+      default: decode_spread_kernel<DD, kSpreadWaves><<<grid, kSpreadWaves * 64, 0, st>>>(p.sa); break;
+    }
+  };
+  if (D == 128)
+    go(std::integral_constant<int, 128>{});
+  else
+    go(std::integral_constant<int, 64>{});
+  const hipError_t e = hipGetLastError();
+  SPYRE_REQUIRE(e == hipSuccess, SPYRE_EHIP, "decode spread launch failed: %s", hipGetErrorString(e));
+  return SPYRE_OK;
 }
 
 extern "C" int spyre_paged_decode_attn_f16(const void* q, const void* k_cache, const void* v_cache,

@@ -174,16 +174,16 @@ std::tuple<at::Tensor, at::Tensor> paged_decode_attention(const at::Tensor& q, c
   if (max_context_len < 0) max_context_len = B ? context_lens.max().item<int32_t>() : 0;  // synchronises
   TORCH_CHECK_VALUE(max_context_len <= block_table.size(1) * kPage, "max_context_len ", max_context_len,
                     " exceeds the block table's ", block_table.size(1), " pages");
-  const size_t need = spyre_paged_decode_attn_workspace_bytes(B, Hq, Hkv, D, max_context_len, split_tokens);
+  const size_t need = spyre_paged_decode_attn_call_workspace_bytes(B, Hq, Hkv, D, max_context_len, split_tokens);
   at::Tensor ws = at::empty({static_cast<int64_t>(std::max<size_t>(need, 4))}, q.options().dtype(at::kByte));
   at::Tensor out = at::empty_like(q);
   at::Tensor lse = at::empty({B, Hq}, q.options().dtype(at::kFloat));
   check_rc("spyre_paged_decode_attn_f16",
-           spyre_paged_decode_attn_f16(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
-                                       block_table.data_ptr<int32_t>(), block_table.stride(0),
-                                       context_lens.data_ptr<int32_t>(), out.data_ptr(), lse.data_ptr<float>(),
-                                       ws.data_ptr(), ws.numel(), B, Hq, Hkv, D, kPage, num_pages, max_context_len,
-                                       split_tokens, static_cast<float>(scale), stream_of(q)));
+           spyre_paged_decode_attn_call_f16(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+                                            block_table.data_ptr<int32_t>(), block_table.stride(0),
+                                            context_lens.data_ptr<int32_t>(), out.data_ptr(), lse.data_ptr<float>(),
+                                            ws.data_ptr(), ws.numel(), B, Hq, Hkv, D, kPage, num_pages,
+                                            max_context_len, split_tokens, static_cast<float>(scale), stream_of(q)));
   return {out, lse};
 }
 
