@@ -260,3 +260,44 @@ def test_masked_decode_reads_inside_the_mask(cuda, case):
         kn[:, :, Skv - 64 - 64:], vn[:, :, Skv - 64 - 64:] = k[:, :, Skv - 64 - 64:], v[:, :, Skv - 64 - 64:]
     out = tsa.scaled_dot_product_attention(q.to(cuda), kn.to(cuda), vn.to(cuda), attn_mask=mask, enable_gqa=True)
     assert_close(out, OA.sdpa_cpu_fp32(q, k, v, attn_mask=keep))
+
+
+@pytest.mark.parametrize("key", [20, -3])
+@pytest.mark.parametrize("kind", ["f16", "f32"])
+@pytest.mark.parametrize("Sq,Skv,Hkv", [(1, 200, 2), (1, 4100, 8), (1, 20000, 8), (15, 65, 2), (40, 1040, 2),
+                                        (128, 4096, 2), (300, 777, 8), (1100, 1100, 8)])
+def test_nan_bias_reaches_its_row(cuda, Sq, Skv, Hkv, kind, key):
+    """A NaN in a bias makes its row NaN, also where every other score of its
+    keys' split or (fp32, or one query) step is -inf, and no other row.  fp16
+    biases of several queries skip steps by their largest number, so that NaN
+    keys under -inf do not count: their NaN lies among kept keys."""
+    import torch_spyre_amd as tsa
+
+    B, Hq, D = 2, 8, 128
+    q, k, v = (randn((B, h, s, D), SEED + 330 + i).to(cuda) for i, (h, s) in enumerate([(Hq, Sq), (Hkv, Skv), (Hkv, Skv)]))
+    mask = torch.full((B, Hq, Sq, Skv), -float("inf"), dtype=DTYPE[kind], device=cuda)
+    mask[..., :40] = 0
+    bad = torch.zeros((B, Hq, Sq), dtype=torch.bool, device=cuda)
+    bad[0, 1, 0] = bad[1, 7, Sq - 1] = True
+    if kind == "f16" and Sq > 1:
+        key = 20 if key > 0 else Skv - 20
+        mask[..., Skv - 30:] = 0
+    mask[..., key][bad] = float("nan")
+    got = torch.isnan(tsa.scaled_dot_product_attention(q, k, v, attn_mask=mask, enable_gqa=True))
+    assert torch.equal(got.all(-1), bad) and torch.equal(got.any(-1), bad)
+
+
+@pytest.mark.parametrize("kind", ["none", "bool"])
+@pytest.mark.parametrize("Sq,Skv", [(40, 1040), (128, 4096)])
+def test_nan_key_reaches_every_row_that_sees_it(cuda, kind, Sq, Skv):
+    """Key splits carry a NaN key of one split into the result."""
+    import torch_spyre_amd as tsa
+
+    B, Hq, Hkv, D = 2, 8, 2, 128
+    q, k, v = (randn((B, h, s, D), SEED + 340 + i).to(cuda) for i, (h, s) in enumerate([(Hq, Sq), (Hkv, Skv), (Hkv, Skv)]))
+    k[0, 0, Skv - 2, 5] = float("nan")
+    mask = torch.ones((Sq, Skv), dtype=torch.bool, device=cuda) if kind == "bool" else None
+    got = torch.isnan(tsa.scaled_dot_product_attention(q, k, v, attn_mask=mask, enable_gqa=True)).all(-1)
+    want = torch.zeros((B, Hq, Sq), dtype=torch.bool, device=cuda)
+    want[0, :Hq // Hkv] = True
+    assert torch.equal(got, want)

@@ -354,7 +354,7 @@ __device__ __forceinline__ bool mask_keeps(typename DenseMask<MK>::T x) {
   if constexpr (MK == kDecodeMaskBool)
     return x != 0;
   else
-    return static_cast<float>(x) > -INFINITY;
+    return static_cast<float>(x) != -INFINITY;  // a NaN is kept: it reaches the result
 }
 
 // N consecutive mask elements at any alignment.

@@ -404,6 +404,14 @@ __device__ __forceinline__ float max_xor32(float x) {
                __builtin_bit_cast(float, static_cast<unsigned>(r[1])));
 }
 
+// The same, NaN if either is.
+__device__ __forceinline__ float maximum_xor32(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, x),
+                                                  false, false);
+  return __builtin_elementwise_maximum(__builtin_bit_cast(float, static_cast<unsigned>(r[0])),
+                                       __builtin_bit_cast(float, static_cast<unsigned>(r[1])));
+}
+
 __device__ __forceinline__ float sum_xor32(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, x),
                                                   false, false);
@@ -765,13 +773,32 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   // (the first half of the next step's scores, computed before this
   // update); a move of m_use shifts both, and the tile.
   // The step's row max in the units of m_run.
+  // fp32 biases: NaN if a score is, so that no step with a NaN counts as
+  // blank (the per-wavefront kernel skips none).  fp16: a step whose kept
+  // scores are all NaN is one, as a cache's unused keys under -inf may be.
+  auto max_of = [](float x, float y) {
+    if constexpr (F32M)
+      return __builtin_elementwise_maximum(x, y);
+    else
+      return fmaxf(x, y);
+  };
+  auto max_halves = [](float x) {
+    if constexpr (F32M)
+      return maximum_xor32(x);
+    else
+      return max_xor32(x);
+  };
   auto row_max = [&](const f32x16 (&s)[2]) {
     float mx = -INFINITY;
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-      for (int rr = 0; rr < 16; ++rr) mx = fmaxf(mx, s[mt][rr]);
-    return PRESCALED ? max_xor32(mx) + m_use : max_xor32(mx) * scale_abs;
+      for (int rr = 0; rr < 16; ++rr) mx = max_of(mx, s[mt][rr]);
+    return PRESCALED ? max_halves(mx) + m_use : max_halves(mx) * scale_abs;
+  };
+  // Whether a masked step whose row max is mx adds anything to a real row.
+  auto adds = [&](float mx) {
+    return __builtin_amdgcn_ballot_w64(q_ok && !(mx == -INFINITY || mx < m_run - 32.f)) != 0;
   };
   // ahead2: with a mask, the second half of S(t+1) is complete too.
   auto update_max = [&](f32x16 (&s)[2], f32x16& ahead, f32x16* ahead2, float mx) {
@@ -998,10 +1025,10 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
       interleave_h(0, DK);
       float mx = -INFINITY;
 #pragma unroll
-      for (int rr = 0; rr < 16; ++rr) mx = fmaxf(mx, cur[rr]);
-      mx = PRESCALED ? max_xor32(mx) + m_use : max_xor32(mx) * (F32M ? 1.f : scale_abs);
+      for (int rr = 0; rr < 16; ++rr) mx = max_of(mx, cur[rr]);
+      mx = PRESCALED ? max_halves(mx) + m_use : max_halves(mx) * (F32M ? 1.f : scale_abs);
       // A step the mask blanks for every real row adds nothing (see step).
-      const bool live = MK == kNoMask || __builtin_amdgcn_ballot_w64(q_ok && mx > -INFINITY && mx >= m_run - 32.f) != 0;
+      const bool live = MK == kNoMask || adds(mx);
       if (live && __builtin_amdgcn_ballot_w64(mx > m_run + kLazy) != 0) {
         const float m_new = fmaxf(m_run, mx);
         const float alpha = m_new == -INFINITY ? 1.f : fast_exp2(m_run - m_new);
@@ -1136,7 +1163,7 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
         apply_mask(t, cur);
         if (edge(t)) mask_step(t, cur);
         const float mx = row_max(cur);
-        const bool live = __builtin_amdgcn_ballot_w64(q_ok && mx > -INFINITY && mx >= m_run - 32.f) != 0;
+        const bool live = adds(mx);
         nxt[0] = PRESCALED ? neg_m_tile : f32x16{};
         nxt[1] = PRESCALED ? neg_m_tile : f32x16{};
 #pragma unroll
@@ -1668,15 +1695,15 @@ __global__ __launch_bounds__(256) void sdpa_split_merge_kernel(MergeArgs a) {
     float Mn = M;
 #pragma unroll
     for (int j = 0; j < G; ++j)
-      if (ml[j][1] > 0.f) Mn = fmaxf(Mn, ml[j][0]);
-    if (Mn == -INFINITY) continue;  // nothing visible yet
-    const float c = exp2f(M - Mn);  // M = -inf: c = 0
+      if (ml[j][1] != 0.f) Mn = fmaxf(Mn, ml[j][0]);  // (a NaN sum counts: it reaches the row's result)
+    const float Mu = Mn == -INFINITY ? 0.f : Mn;  // nothing visible yet: weights 0
+    const float c = exp2f(M - Mu);  // M = -inf: c = 0
     L *= c;
     acc *= c;
 #pragma unroll
     for (int j = 0; j < G; ++j) {
-      if (!(ml[j][1] > 0.f)) continue;
-      const float w = exp2f(ml[j][0] - Mn);
+      if (ml[j][1] == 0.f) continue;
+      const float w = exp2f(ml[j][0] - Mu);
       L += ml[j][1] * w;
       acc += ov[j] * w;
     }
@@ -1692,17 +1719,16 @@ __global__ __launch_bounds__(256) void sdpa_split_merge_kernel(MergeArgs a) {
   M = -INFINITY;
 #pragma unroll
   for (int t = 0; t < SL; ++t)
-    if (s_l[t] > 0.f) M = fmaxf(M, s_m[t]);
+    if (s_l[t] != 0.f) M = fmaxf(M, s_m[t]);
   L = 0.f;
   acc = f32x4{0.f, 0.f, 0.f, 0.f};
-  if (M != -INFINITY) {
+  const float Mu = M == -INFINITY ? 0.f : M;
 #pragma unroll
-    for (int t = 0; t < SL; ++t) {
-      if (!(s_l[t] > 0.f)) continue;
-      const float w = exp2f(s_m[t] - M);
-      L += s_l[t] * w;
-      acc += s_acc[t][d4] * w;
-    }
+  for (int t = 0; t < SL; ++t) {
+    if (s_l[t] == 0.f) continue;
+    const float w = exp2f(s_m[t] - Mu);
+    L += s_l[t] * w;
+    acc += s_acc[t][d4] * w;
   }
   const int d = 4 * d4;
   const int64_t qi = r % a.Sq, bh = r / a.Sq;
@@ -1749,15 +1775,15 @@ __global__ __launch_bounds__(256) void sdpa_split_merge_rows_kernel(MergeArgs a)
     float Mn = M;
 #pragma unroll
     for (int j = 0; j < G; ++j)
-      if (ml[j][1] > 0.f) Mn = fmaxf(Mn, ml[j][0]);
-    if (Mn == -INFINITY) continue;  // nothing visible yet
-    const float c = exp2f(M - Mn);  // M = -inf: c = 0
+      if (ml[j][1] != 0.f) Mn = fmaxf(Mn, ml[j][0]);  // (a NaN sum counts: it reaches the row's result)
+    const float Mu = Mn == -INFINITY ? 0.f : Mn;  // nothing visible yet: weights 0
+    const float c = exp2f(M - Mu);  // M = -inf: c = 0
     L *= c;
     acc *= c;
 #pragma unroll
     for (int j = 0; j < G; ++j) {
-      if (!(ml[j][1] > 0.f)) continue;
-      const float w = exp2f(ml[j][0] - Mn);
+      if (ml[j][1] == 0.f) continue;
+      const float w = exp2f(ml[j][0] - Mu);
       L += ml[j][1] * w;
       acc += ov[j] * w;
     }
