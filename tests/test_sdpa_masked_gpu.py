@@ -301,3 +301,27 @@ def test_nan_key_reaches_every_row_that_sees_it(cuda, kind, Sq, Skv):
     want = torch.zeros((B, Hq, Sq), dtype=torch.bool, device=cuda)
     want[0, :Hq // Hkv] = True
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("kind", ["bool", "f16"])
+@pytest.mark.parametrize("shape", ["qk", "bhqk", "1h1k"])
+@pytest.mark.parametrize("Sq,Skv,D", [(40, 7, 64), (40, 9, 128), (130, 16, 64), (70, 17, 128), (33, 63, 64), (130, 65, 128),
+                                      (65, 95, 64), (40, 97, 128), (300, 129, 64), (20, 1023, 128), (333, 333, 128)])
+def test_mask_rows_of_any_alignment(cuda, Sq, Skv, D, shape, kind):
+    """Half steps read mask rows that start anywhere and end inside a 16-byte
+    unit as they lie: views into a buffer whose other elements are NaN (or
+    True), the last row ending with the buffer."""
+    import torch_spyre_amd as tsa
+
+    B, Hq, Hkv = 2, 8, 4
+    q = randn((B, Hq, Sq, D), SEED + 350)
+    k, v = randn((B, Hkv, Skv, D), SEED + 351), randn((B, Hkv, Skv, D), SEED + 352)
+    mask = make_mask(kind, shape, B, Hq, Sq, Skv, SEED + 353 + Sq + Skv)
+    wide = torch.full((*mask.shape[:-1], Skv + 3), True if kind == "bool" else float("nan"), dtype=mask.dtype, device=cuda)
+    view = wide[..., 3:]
+    view.copy_(mask)
+    out, lse = tsa.scaled_dot_product_attention(q.to(cuda), k.to(cuda), v.to(cuda), attn_mask=view, enable_gqa=True,
+                                                return_lse=True)
+    assert_close(out, OA.sdpa_cpu_fp32(q, k, v, attn_mask=mask))
+    _, lse64 = OA.sdpa_decomposition_fp64(q, k, v, attn_mask=mask.numpy(), return_lse=True)
+    assert np.allclose(lse.cpu().numpy(), lse64, atol=LSE_ATOL, rtol=0)

@@ -60,6 +60,7 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 using spyre_hip::fdiv;
 using spyre_hip::u32x4_t;
 
@@ -480,7 +481,16 @@ template <bool HALF> struct MaskTile<kNoMask, HALF> {
 // HALF (blocks of at most 128 rows, e.g. decode): wavefronts 2r and 2r + 1
 // share row tile r and take one 32-key half of every step each; the pair's
 // partials are folded in LDS at the end.
-template <int D, bool PRESCALED, int MK, int SLOTS, bool HALF, int W>
+// ANY (fp16 / boolean masks in half steps): rows of any alignment and length,
+// at least 16 bytes, through registers by ordinary loads and stores to the
+// mask block at the step's end.  Copied first with 16-byte rows, they cost
+// a launch and two passes: 32 heads, D 128, 1001 x 1001, fp16 63.6 -> 36.8 us,
+// boolean [1001, 1001] 35.1 -> 32.2; 333 x 333 boolean 16.0 -> 13.1; 4 x 16 heads
+// x 150, D 64, boolean 11.3 -> 8.2.  A kernel of its own: behind a flag the loads'
+// registers cost the others (2 x 12 heads x 512, D 64, boolean 9.7 -> 11.1).
+// fp32 rows this way instead of 4 bytes a lane: 21.7 -> 34.6 (2 x 16 heads x
+// 777, D 64).
+template <int D, bool PRESCALED, int MK, int SLOTS, bool HALF, int W, bool ANY = false>
 __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   static_assert(SLOTS == 2 || (SLOTS == 4 && MK == kNoMask), "four slots leave no room for a mask");
   // fp32 biases: half steps only (the 32-query block of a full step, 8 KB a
@@ -662,6 +672,46 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
       }
     }
   };
+  // ANY: the block's units of keys kb .. in registers, and from there to
+  // its slot.  A unit that crosses the row's end is read as the row's last 16
+  // bytes, shifted (rows have at least 16: the host's check).
+  u32x4 m_reg[MT::kLoads > 0 ? MT::kLoads : 1];
+  auto read_m = [&](int kb) {
+    if constexpr (ANY) {
+      const char* p = mbase + static_cast<int64_t>(kb) * MT::kEsz;
+#pragma unroll
+      for (int j = 0; j < MT::kLoads; ++j) {
+        m_reg[j] = u32x4{0, 0, 0, 0};
+        if (kb + kKT <= a.Skv) {
+          if (m_off[j] < kOob) __builtin_memcpy(&m_reg[j], p + m_off[j], 16);
+        } else {
+          const int u = 64 * j + lane;
+          const int at = (kb + 32 * hw) * MT::kEsz + 16 * ((u % MT::kU) ^ MT::swz(u / MT::kU));  // the unit's bytes in its row
+          const int past = at + 16 - a.Skv * MT::kEsz;  // of them past the row
+          if (m_off[j] < kOob && past < 16) {
+            const int back = max(past, 0);
+            uint64_t x[2];
+            __builtin_memcpy(x, p + (static_cast<int64_t>(m_off[j]) - back), 16);
+            if (back >= 8) {
+              x[0] = x[1] >> (8 * (back - 8));
+              x[1] = 0;
+            } else if (back > 0) {
+              x[0] = x[0] >> (8 * back) | x[1] << (64 - 8 * back);
+              x[1] >>= 8 * back;
+            }
+            __builtin_memcpy(&m_reg[j], x, 16);
+          }
+        }
+      }
+    }
+  };
+  auto write_m = [&](int slot) {
+    if constexpr (ANY) {
+#pragma unroll
+      for (int j = 0; j < MT::kLoads; ++j)
+        *reinterpret_cast<u32x4*>(mask_block(slot) + 512 * j + 8 * lane) = m_reg[j];
+    }
+  };
   // The loads must have landed before the barrier that publishes them.
   auto dma_wait = [] { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
 
@@ -758,7 +808,7 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   auto next_mask = [&](int t) {
     if constexpr (MK != kNoMask && kMaskSlots == 1) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      if (t + 1 < n_tiles) dma_m(kb0 + (t + 1) * kKT, 0);
+      if (t + 1 < n_tiles && !ANY) dma_m(kb0 + (t + 1) * kKT, 0);
     }
   };
   auto apply_mask = [&](int t, f32x16 (&s)[2]) {
@@ -993,7 +1043,8 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
     if constexpr (SLOTS == 2) {
       if (t + 2 < n_tiles) dma_k(t & 1);
       if (t + 1 < n_tiles) dma_v((t + 1) & 1);
-      if (kMaskSlots == 2 && t + 1 < n_tiles) dma_m(kb0 + (t + 1) * kKT, (t + 1) & 1);
+      if (kMaskSlots == 2 && t + 1 < n_tiles && !ANY) dma_m(kb0 + (t + 1) * kKT, (t + 1) & 1);
+      if (ANY && t + 1 < n_tiles) read_m(kb0 + (t + 1) * kKT);
     } else if ((t & 1) == 0) {
       if (t + 3 < n_tiles) dma_k((t + 3) % 4);
       if (t + 4 < n_tiles) dma_k(t % 4);
@@ -1063,6 +1114,7 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
     }
     if (SLOTS == 2 || (t & 1)) {
       dma_wait();
+      if (ANY && t + 1 < n_tiles) write_m((t + 1) & 1);
       __syncthreads();
     }
   };
@@ -1205,14 +1257,16 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   if (n_tiles > 0) {
     dma_k(0);
     dma_v(0);
-    dma_m(kb0, 0);
+    if (!ANY) dma_m(kb0, 0);
   }
   if (n_tiles > 1) dma_k(1);
   if constexpr (SLOTS == 4) {
     if (n_tiles > 1) dma_v(1);
     if (n_tiles > 2) dma_k(2);
   }
+  if (ANY && n_tiles > 0) read_m(kb0);
   dma_wait();
+  if (ANY && n_tiles > 0) write_m(0);
   __syncthreads();
   if (active(0)) {
     if constexpr (HALF) {
@@ -2044,17 +2098,17 @@ void launch_short(const Fwd2Args& f2, int D, bool prescaled, int waves, int mask
     launch_short_w<kWaves2>(f2, D, prescaled, mask_kind, st);
 }
 
-template <int MK, int SLOTS, bool HALF, int W>
+template <int MK, int SLOTS, bool HALF, int W, bool ANY = false>
 void launch_lds(const Fwd2Args& f2, int D, bool prescaled, hipStream_t st) {
   const dim3 grid(f2.n_items);
   if (D == 128 && prescaled)
-    sdpa_fwd_lds_kernel<128, true, MK, SLOTS, HALF, W><<<grid, W * 64, 0, st>>>(f2);
+    sdpa_fwd_lds_kernel<128, true, MK, SLOTS, HALF, W, ANY><<<grid, W * 64, 0, st>>>(f2);
   else if (D == 128)
-    sdpa_fwd_lds_kernel<128, false, MK, SLOTS, HALF, W><<<grid, W * 64, 0, st>>>(f2);
+    sdpa_fwd_lds_kernel<128, false, MK, SLOTS, HALF, W, ANY><<<grid, W * 64, 0, st>>>(f2);
   else if (prescaled)
-    sdpa_fwd_lds_kernel<64, true, MK, SLOTS, HALF, W><<<grid, W * 64, 0, st>>>(f2);
+    sdpa_fwd_lds_kernel<64, true, MK, SLOTS, HALF, W, ANY><<<grid, W * 64, 0, st>>>(f2);
   else
-    sdpa_fwd_lds_kernel<64, false, MK, SLOTS, HALF, W><<<grid, W * 64, 0, st>>>(f2);
+    sdpa_fwd_lds_kernel<64, false, MK, SLOTS, HALF, W, ANY><<<grid, W * 64, 0, st>>>(f2);
 }
 
 template <int W>
@@ -2340,6 +2394,29 @@ extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const
   const bool as_it_lies = mask_kind != kNoMask && direct && (dense || short_grid(B, Hq, Hkv, Sq, Skv, D, ws_room, gs));
   if (as_it_lies) mp.route = kRouteNone;
   const bool lds_path = mp.route != kRouteVt;
+  // Short query runs pack q heads of a KV head into one block's rows, so
+  // they share each K / V tile (decode: one block per (sequence, KV head)
+  // instead of g mostly idle ones).
+  // And (plan_grid) a key split when the blocks would not fill the device
+  // and the workspace holds its partials (after a mask's copy).
+  const size_t part_at = copy_room(mp);
+  const size_t part_room = ws_room > part_at ? ws_room - part_at : 0;
+  GridPlan gpl;
+  if (lds_path && !dense)
+    gpl = as_it_lies               ? gs
+          : mask_kind == kNoMask ? plan_grid(B, Hq, Hkv, Sq, Skv, D, is_causal != 0, part_room)
+                                 : masked_grid(mp, mask_kind, B, Hq, Hkv, Sq, Skv, D, part_room);
+  // Grids of half steps need no copy: they read rows of any alignment and
+  // of at least 16 bytes.
+  bool any_rows = false;
+  if (mp.route == kRouteCopied && (gpl.shape == kHalf8 || gpl.shape == kHalf4) && mask_strides[3] == 1 && Skv * mp.esz >= 16 &&
+      ((Sq - 1) * mask_strides[2] + (gpl.pack - 1) * mask_strides[1] + Skv) * mp.esz <= kBufRange) {
+    any_rows = true;
+    mp.route = kRouteStaged;
+    mp.sb = mask_strides[0];
+    mp.sh = mask_strides[1];
+    mp.sq = mask_strides[2];
+  }
   const int s64 = static_cast<int>(s64_of(Skv));
   const void* mask_ptr = attn_mask;
   if (mp.route == kRouteCopied) {
@@ -2431,16 +2508,6 @@ extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const
     f2.Sq = Sq;
     f2.Skv = Skv;
     f2.causal = fa.causal;
-    // Short query runs pack q heads of a KV head into one block's rows, so
-    // they share each K / V tile (decode: one block per (sequence, KV head)
-    // instead of g mostly idle ones).
-    // And (plan_grid) a key split when the blocks would not fill the device
-    // and the workspace holds its partials (after a mask's copy).
-    const size_t part_at = copy_room(mp);
-    const size_t part_room = ws_room > part_at ? ws_room - part_at : 0;
-    const GridPlan gpl = as_it_lies               ? gs
-                         : mask_kind == kNoMask ? plan_grid(B, Hq, Hkv, Sq, Skv, D, is_causal != 0, part_room)
-                                                : masked_grid(mp, mask_kind, B, Hq, Hkv, Sq, Skv, D, part_room);
     f2.pack = gpl.pack;
     f2.gp = fa.g / f2.pack;
     const int rows = shape_rows(gpl.shape);
@@ -2474,6 +2541,12 @@ extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const
     } else {
       auto go = [&](auto mk) {
         constexpr int MK = decltype(mk)::value;
+        if constexpr (MK != kNoMask)
+          if (any_rows) {
+            gpl.shape == kHalf8 ? launch_lds<MK, 2, true, 8, true>(f2, D, prescaled, st)
+                                : launch_lds<MK, 2, true, 4, true>(f2, D, prescaled, st);
+            return;
+          }
         switch (gpl.shape) {
           case k256: launch_lds<MK, 2, false, 8>(f2, D, prescaled, st); break;
           case kHalf8: launch_lds<MK, MK == kNoMask ? 4 : 2, true, 8>(f2, D, prescaled, st); break;
