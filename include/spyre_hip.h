@@ -300,7 +300,9 @@ size_t spyre_sdpa_fwd_workspace_bytes(int B, int Hkv, int Skv, int D);
  * bytes) for fp16 / bool masks other than those with key stride 1, a 16-byte
  * aligned pointer, b / h / i strides and Skv of whole 16 bytes (staged in
  * LDS beside K and V as they lie) a copy with 16-byte rows of the mask's
- * non-broadcast extent (then staged the same way); for fp32 masks, the larger
+ * non-broadcast extent (then staged the same way; grids of 64- and 128-row
+ * blocks read rows of at least 16 bytes as they lie, but the room is asked
+ * for whichever runs); for fp32 masks, the larger
  * of a key split's partials and spyre_sdpa_fwd_workspace_bytes (which fp32
  * masks whose keys are not contiguous use).  A
  * call whose fp16 / bool mask needs a copy but whose workspace holds only
