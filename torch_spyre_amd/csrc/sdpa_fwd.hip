@@ -1687,19 +1687,21 @@ __global__ __launch_bounds__(W * 64) void sdpa_decode_short_kernel(Fwd2Args a) {
         ov[jj] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(pr, ((r0 + s2) * D + 4 * d4) * 4, 0,
                                                                                  kAuxDevice));
       }
-      float mv[G];  // the split's max, or -inf when it carries no weight
+      // The split's max, or -inf when it carries no weight.  A NaN sum counts
+      // (and reaches the row whatever its weight: NaN times 0).
+      float mv[G];
 #pragma unroll
-      for (int jj = 0; jj < G; ++jj) mv[jj] = s0 + jj < a.nsplit && ml[jj][1] > 0.f ? ml[jj][0] : -INFINITY;
+      for (int jj = 0; jj < G; ++jj) mv[jj] = s0 + jj < a.nsplit && ml[jj][1] != 0.f ? ml[jj][0] : -INFINITY;
       float Mn = Mr;
 #pragma unroll
       for (int jj = 0; jj < G; ++jj) Mn = fmaxf(Mn, mv[jj]);
-      if (Mn == -INFINITY) continue;  // nothing visible yet
-      const float c = fast_exp2(Mr - Mn);  // Mr = -inf: c = 0
+      const float Mu = Mn == -INFINITY ? 0.f : Mn;  // nothing visible yet: weights 0
+      const float c = fast_exp2(Mr - Mu);  // Mr = -inf: c = 0
       Lr *= c;
       ac *= c;
 #pragma unroll
       for (int jj = 0; jj < G; ++jj) {
-        const float w = fast_exp2(mv[jj] - Mn);  // -inf: 0
+        const float w = fast_exp2(mv[jj] - Mu);  // -inf: 0
         Lr += ml[jj][1] * w;
         ac += ov[jj] * w;
       }
