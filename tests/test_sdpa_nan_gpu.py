@@ -1,11 +1,12 @@
 """NaN in masked SDPA calls: one in a key or a bias that a row keeps makes
-that row NaN, wherever its key lies."""
+that row NaN, wherever its key lies; what a row's mask drops does not."""
 
 import pytest
 import torch
 
+from oracle import attention as OA
 from tests.conftest import SEED
-from tests.test_sdpa_gpu import randn
+from tests.test_sdpa_gpu import assert_close, randn
 
 pytestmark = pytest.mark.gpu
 
@@ -18,11 +19,12 @@ def as_mask(kind, keep):
     return torch.zeros(keep.shape, dtype=DTYPE[kind]).masked_fill_(~keep, -float("inf"))
 
 
-def nan_rows(cuda, q, k, v, mask):
+def nan_rows(cuda, q, k, v, mask, scale=None):
     """Rows of the result that are NaN; a row is NaN in every feature or in none."""
     import torch_spyre_amd as tsa
 
-    out = tsa.scaled_dot_product_attention(q.to(cuda), k.to(cuda), v.to(cuda), attn_mask=mask.to(cuda), enable_gqa=True)
+    out = tsa.scaled_dot_product_attention(q.to(cuda), k.to(cuda), v.to(cuda), attn_mask=mask.to(cuda), scale=scale,
+                                           enable_gqa=True)
     got = torch.isnan(out)
     assert torch.equal(got.any(-1), got.all(-1))
     return got.all(-1).cpu()
@@ -50,3 +52,51 @@ def test_nan_in_the_only_split_with_kept_keys(cuda, case, first, kept, kind):
         mask[0, 1, Sq - 1, first] = float("nan")
         want[0, 1, Sq - 1] = True
         assert torch.equal(nan_rows(cuda, q, k, v, mask), want)
+
+
+# Half steps of 32 keys (Sq 40; 128 packed rows), with and without a key
+# split, and full steps of 64 (300, 1000).
+SQ = [(40, 300, 2), (40, 2048, 2), (128, 1000, 8), (128, 4096, 2), (300, 2048, 8), (1000, 1000, 8)]
+
+
+@pytest.mark.parametrize("scale", [None, 2.0])
+@pytest.mark.parametrize("kind", ["bool", "f16", "f32"])
+@pytest.mark.parametrize("Sq,Skv,Hkv", SQ)
+def test_nan_alone_in_its_step(cuda, Sq, Skv, Hkv, kind, scale):
+    """The one kept key of its step is NaN (keys 0 .. 64 are kept), then the
+    one number that is no -inf of its step is a NaN bias; q prescaled in fp16
+    and (scale 2) not."""
+    B, Hq, D = 2, 8, 128
+    q = randn((B, Hq, Sq, D), SEED + 510)
+    k, v = randn((B, Hkv, Skv, D), SEED + 511), randn((B, Hkv, Skv, D), SEED + 512)
+    keep = torch.zeros((Sq, Skv), dtype=torch.bool)
+    keep[:, :65] = True
+    bad = k.clone()
+    bad[1, 0, 64, 9] = float("nan")
+    want = torch.zeros((B, Hq, Sq), dtype=torch.bool)
+    want[1, :Hq // Hkv] = True
+    assert torch.equal(nan_rows(cuda, q, bad, v, as_mask(kind, keep), scale), want)
+    if kind != "bool":
+        mask = as_mask(kind, keep).expand(B, Hq, Sq, Skv).clone()
+        mask[0, 2, Sq // 2, 200] = float("nan")
+        want = torch.zeros((B, Hq, Sq), dtype=torch.bool)
+        want[0, 2, Sq // 2] = True
+        assert torch.equal(nan_rows(cuda, q, k, v, mask, scale), want)
+
+
+@pytest.mark.parametrize("low", [-float("inf"), torch.finfo(torch.float16).min])
+@pytest.mark.parametrize("Sq,Skv,Hkv", [(128, 1000, 8), (300, 2048, 8), (1000, 1000, 8)])
+def test_steps_of_dropped_keys_stay_skipped(cuda, Sq, Skv, Hkv, low):
+    """fp16 biases: NaN keys of whole steps that a bias drops (-inf or the
+    type's lowest number) after kept ones do not reach a row."""
+    import torch_spyre_amd as tsa
+
+    B, Hq, D = 1, 8, 128
+    q = randn((B, Hq, Sq, D), SEED + 520)
+    k, v = randn((B, Hkv, Skv, D), SEED + 521), randn((B, Hkv, Skv, D), SEED + 522)
+    mask = torch.zeros((Sq, Skv), dtype=torch.float16)
+    mask[:, 128:] = low
+    kn = k.clone()
+    kn[:, :, 192:] = float("nan")
+    out = tsa.scaled_dot_product_attention(q.to(cuda), kn.to(cuda), v.to(cuda), attn_mask=mask.to(cuda), enable_gqa=True)
+    assert_close(out, OA.sdpa_cpu_fp32(q, k, v, attn_mask=mask))

@@ -821,7 +821,6 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   auto apply_mask = [&](int t, f32x16 (&s)[2]) {
     apply_mask_half(t, 0, s[0]);
     apply_mask_half(t, 1, s[1]);
-    next_mask(t);
   };
   // The running max (log2 domain) moves only when a score of the step
   // exceeds it by more than 2^8, so P <= 256 (fine in fp16) and most steps
@@ -830,17 +829,15 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   // (the first half of the next step's scores, computed before this
   // update); a move of m_use shifts both, and the tile.
   // The step's row max in the units of m_run.
-  // fp32 biases: NaN if a score is, so that no step with a NaN counts as
-  // blank (the per-wavefront kernel skips none).  fp16: a step whose kept
-  // scores are all NaN is one, as a cache's unused keys under -inf may be.
+  // Masked: NaN if a score is, so that a NaN does not leave its step blank.
   auto max_of = [](float x, float y) {
-    if constexpr (F32M)
+    if constexpr (MK != kNoMask)
       return __builtin_elementwise_maximum(x, y);
     else
       return fmaxf(x, y);
   };
   auto max_halves = [](float x) {
-    if constexpr (F32M)
+    if constexpr (MK != kNoMask)
       return maximum_xor32(x);
     else
       return max_xor32(x);
@@ -853,9 +850,33 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
       for (int rr = 0; rr < 16; ++rr) mx = max_of(mx, s[mt][rr]);
     return PRESCALED ? max_halves(mx) + m_use : max_halves(mx) * scale_abs;
   };
-  // Whether a masked step whose row max is mx adds anything to a real row.
-  auto adds = [&](float mx) {
-    return __builtin_amdgcn_ballot_w64(q_ok && !(mx == -INFINITY || mx < m_run - 32.f)) != 0;
+  // Whether a masked step adds anything to a real row: mx is this lane's row
+  // max (of both lane halves), s its scores (half steps: one half, else two).
+  // A NaN does.  Boolean masks leave none on a dropped key; an fp16 bias may
+  // (a cache's unused keys), so a NaN under one that alone makes the weight 0
+  // (-inf, the type's lowest number) does not count: when no row has a number
+  // that adds something, the NaN rows are gone through with their biases.
+  auto adds = [&](int t, float mx, const f32x16* s) {
+    const bool row = q_ok && !(mx == -INFINITY || mx < m_run - 32.f);
+    const bool any = __builtin_amdgcn_ballot_w64(row) != 0;
+    if (MK == kMaskF16 && __builtin_expect(any && __builtin_amdgcn_ballot_w64(row && mx == mx) == 0, 0)) {
+      constexpr float kDropped = -1024.f;
+      const char* blk = reinterpret_cast<const char*>(mask_block(t & 1));
+      bool some = false;
+#pragma unroll
+      for (int hf = 0; hf < (HALF ? 1 : 2); ++hf)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const f16x4 m4 = *reinterpret_cast<const f16x4*>(blk + (m_lane ^ (64 * hf + 32 * (i >> 1))) + 8 * (i & 1));
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const float x = PRESCALED ? s[hf][4 * i + v] + m_use : s[hf][4 * i + v] * scale_abs;
+            some = some || (x != x ? !(static_cast<float>(m4[v]) <= kDropped) : x > -INFINITY && x >= m_run - 32.f);
+          }
+        }
+      return __builtin_amdgcn_ballot_w64(row && some) != 0;
+    }
+    return any;
   };
   // ahead2: with a mask, the second half of S(t+1) is complete too.
   auto update_max = [&](f32x16 (&s)[2], f32x16& ahead, f32x16* ahead2, float mx) {
@@ -1068,6 +1089,7 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
         if (i + kPrefetch < kNFH) fr[i + kPrefetch] = frag_h(i + kPrefetch);
       };
       if constexpr (MK != kNoMask) {
+        static_assert(!HALF || MK != kMaskF16 || kMaskSlots == 2, "adds() reads the block after next_mask");
         apply_mask_half(t, 0, cur);
         next_mask(t);
       }
@@ -1086,7 +1108,7 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
       for (int rr = 0; rr < 16; ++rr) mx = max_of(mx, cur[rr]);
       mx = PRESCALED ? max_halves(mx) + m_use : max_halves(mx) * (F32M ? 1.f : scale_abs);
       // A step the mask blanks for every real row adds nothing (see step).
-      const bool live = MK == kNoMask || adds(mx);
+      const bool live = MK == kNoMask || adds(t, mx, &cur);
       if (live && __builtin_amdgcn_ballot_w64(mx > m_run + kLazy) != 0) {
         const float m_new = fmaxf(m_run, mx);
         const float alpha = m_new == -INFINITY ? 1.f : fast_exp2(m_run - m_new);
@@ -1222,7 +1244,11 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
         apply_mask(t, cur);
         if (edge(t)) mask_step(t, cur);
         const float mx = row_max(cur);
-        const bool live = adds(mx);
+        bool live = true;
+        if (kMaskSlots == 1) {
+          live = adds(t, mx, cur);
+          next_mask(t);
+        }
         nxt[0] = PRESCALED ? neg_m_tile : f32x16{};
         nxt[1] = PRESCALED ? neg_m_tile : f32x16{};
 #pragma unroll
@@ -1231,6 +1257,7 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
           mfma(2 * ks + 1, qv[ks], nxt[1]);
         }
         interleave_reads(0, 2 * DK);
+        if (kMaskSlots == 2) live = adds(t, mx, cur);
         if (live) {
           update_max(cur, nxt[0], &nxt[1], mx);
           const float neg_m = m_run == -INFINITY ? 0.f : -m_run;
