@@ -100,3 +100,26 @@ def test_steps_of_dropped_keys_stay_skipped(cuda, Sq, Skv, Hkv, low):
     kn[:, :, 192:] = float("nan")
     out = tsa.scaled_dot_product_attention(q.to(cuda), kn.to(cuda), v.to(cuda), attn_mask=mask.to(cuda), enable_gqa=True)
     assert_close(out, OA.sdpa_cpu_fp32(q, k, v, attn_mask=mask))
+
+
+@pytest.mark.parametrize("kind", ["bool", "f16", "f32"])
+@pytest.mark.parametrize("case", [(1, 32, 8, 1, 200, 128), (1, 32, 8, 1, 2048, 128), (2, 8, 2, 3, 500, 64),
+                                  (1, 8, 8, 1, 4000, 64), (16, 32, 8, 1, 2048, 128)], ids=str)
+def test_decode_ignores_unused_cache(cuda, case, kind):
+    """A padded decode over a cache never written past its 64-token run of
+    real keys: NaN in K and V there does not reach the result."""
+    import torch_spyre_amd as tsa
+
+    B, Hq, Hkv, Sq, Skv, D = case
+    q = randn((B, Hq, Sq, D), SEED + 530)
+    k, v = randn((B, Hkv, Skv, D), SEED + 531), randn((B, Hkv, Skv, D), SEED + 532)
+    lens = [70 + 7 * b for b in range(B)]
+    keep = torch.zeros((B, 1, 1, Skv), dtype=torch.bool)
+    kn, vn = k.clone(), v.clone()
+    for b, n in enumerate(lens):
+        keep[b, ..., :n] = True
+        end = (n + 63) // 64 * 64
+        kn[b, :, end:], vn[b, :, end:] = float("nan"), float("nan")
+    mask = as_mask(kind, keep)
+    out = tsa.scaled_dot_product_attention(q.to(cuda), kn.to(cuda), vn.to(cuda), attn_mask=mask.to(cuda), enable_gqa=True)
+    assert_close(out, OA.sdpa_cpu_fp32(q, k, v, attn_mask=mask))

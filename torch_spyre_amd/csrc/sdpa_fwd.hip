@@ -1518,7 +1518,23 @@ __global__ __launch_bounds__(W * 64) void sdpa_decode_short_kernel(Fwd2Args a) {
   f32x16 o[DM];
 #pragma unroll
   for (int dm = 0; dm < DM; ++dm) o[dm] = f32x16{};
-  if (rows_here > 0) {
+  // A slice whose mask drops every key for every row is left out (m -inf, l
+  // 0): what K and V hold there, an unused cache's NaN, does not count.
+  bool live = rows_here > 0;
+  if constexpr (MK != kNoMask) {
+    constexpr uint32_t kNone = MK == kMaskBool ? 0u : MK == kMaskF16 ? 0xfc00fc00u : 0xff800000u;  // a word of dropped keys
+    bool kept = false;
+    if (live) {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int w = 0; w < kMW; ++w) kept = kept || mw[mt][i][w] != kNone;
+    }
+    live = __builtin_amdgcn_ballot_w64(q_ok && kept) != 0;
+  }
+  if (live) {
     // S^T tile mt: keys 32mt .. 32mt + 31 of the slice; lane (row, half)
     // holds keys key32_of(8i + 4half + v) in register 4i + v.
     f32x16 s[MT];
