@@ -737,7 +737,18 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   float m_run = -INFINITY, l_run = 0.f;
   // PRESCALED: scores are carried relative to m_use (m_run, or 0 while no
   // finite score has been seen); neg_m_tile holds -m_use in every row.
+  // fp16 biases: 0 too while m_run is below kLow, a row's dropped keys at the
+  // type's lowest number (about -94500 here, where fp32 steps by 2^-7): the
+  // scores of its first kept keys would be accumulated there.  Relative
+  // error of 300 keys, the last 40 of them kept: 4.3e-3, with this 3.6e-4.
+  constexpr bool kClamp = PRESCALED && MK == kMaskF16;
+  constexpr float kLow = -1024.f;
   float m_use = 0.f;
+  bool low = false;  // some row's m_run is below kLow
+  auto reference = [&](float m) {  // m_use for m_run = m
+    if (kClamp) low = __builtin_amdgcn_ballot_w64(m < kLow && m > -INFINITY) != 0;
+    return m == -INFINITY || (kClamp && m < kLow) ? 0.f : m;
+  };
   f32x16 neg_m_tile = f32x16{};
   f32x16 o[DM];
 #pragma unroll
@@ -857,24 +868,27 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   // (-inf, the type's lowest number) does not count: when no row has a number
   // that adds something, the NaN rows are gone through with their biases.
   auto adds = [&](int t, float mx, const f32x16* s) {
-    const bool row = q_ok && !(mx == -INFINITY || mx < m_run - 32.f);
-    const bool any = __builtin_amdgcn_ballot_w64(row) != 0;
-    if (MK == kMaskF16 && __builtin_expect(any && __builtin_amdgcn_ballot_w64(row && mx == mx) == 0, 0)) {
-      constexpr float kDropped = -1024.f;
-      const char* blk = reinterpret_cast<const char*>(mask_block(t & 1));
-      bool some = false;
+    const bool number = mx >= fmaxf(m_run - 32.f, -__FLT_MAX__);  // (-inf is not)
+    bool any = __builtin_amdgcn_ballot_w64(q_ok && number) != 0;
+    if (__builtin_expect(!any && __builtin_amdgcn_ballot_w64(q_ok && mx != mx) != 0, 0)) {
+      any = true;
+      if constexpr (MK == kMaskF16) {
+        constexpr float kDropped = -1024.f;
+        const char* blk = reinterpret_cast<const char*>(mask_block(t & 1));
+        bool some = false;
 #pragma unroll
-      for (int hf = 0; hf < (HALF ? 1 : 2); ++hf)
+        for (int hf = 0; hf < (HALF ? 1 : 2); ++hf)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const f16x4 m4 = *reinterpret_cast<const f16x4*>(blk + (m_lane ^ (64 * hf + 32 * (i >> 1))) + 8 * (i & 1));
+          for (int i = 0; i < 4; ++i) {
+            const f16x4 m4 = *reinterpret_cast<const f16x4*>(blk + (m_lane ^ (64 * hf + 32 * (i >> 1))) + 8 * (i & 1));
 #pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const float x = PRESCALED ? s[hf][4 * i + v] + m_use : s[hf][4 * i + v] * scale_abs;
-            some = some || (x != x ? !(static_cast<float>(m4[v]) <= kDropped) : x > -INFINITY && x >= m_run - 32.f);
+            for (int v = 0; v < 4; ++v) {
+              const float x = PRESCALED ? s[hf][4 * i + v] + m_use : s[hf][4 * i + v] * scale_abs;
+              some = some || (x != x ? !(static_cast<float>(m4[v]) <= kDropped) : x > -INFINITY && x >= m_run - 32.f);
+            }
           }
-        }
-      return __builtin_amdgcn_ballot_w64(row && some) != 0;
+        any = __builtin_amdgcn_ballot_w64(q_ok && mx != mx && some) != 0;
+      }
     }
     return any;
   };
@@ -888,7 +902,7 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
       for (int dm = 0; dm < DM; ++dm) o[dm] *= alpha;
       m_run = m_new;
       if constexpr (PRESCALED) {
-        const float m_use_new = m_new == -INFINITY ? m_use : m_new;  // lanes still without a score keep 0
+        const float m_use_new = reference(m_new);
         const float d = m_use_new - m_use;
         m_use = m_use_new;
 #pragma unroll
@@ -900,6 +914,15 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
           neg_m_tile[rr] = -m_use;
         }
       }
+    }
+  };
+  // kClamp: the scores of rows below kLow made relative to m_run, which they
+  // are not carried against.
+  auto rebase = [&](f32x16& s) {
+    if (kClamp && __builtin_expect(low, 0)) {
+      const float d = m_use - (m_run == -INFINITY ? m_use : m_run);  // 0 in the other rows
+#pragma unroll
+      for (int rr = 0; rr < 16; ++rr) s[rr] += d;
     }
   };
   // P (fp16) of half mt; the row sum adds the same fp16 values the PV
@@ -1117,7 +1140,7 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
         for (int dm = 0; dm < DM; ++dm) o[dm] *= alpha;
         m_run = m_new;
         if constexpr (PRESCALED) {
-          const float m_use_new = m_new == -INFINITY ? m_use : m_new;
+          const float m_use_new = reference(m_new);
           const float d = m_use_new - m_use;
           m_use = m_use_new;
 #pragma unroll
@@ -1129,6 +1152,7 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
         }
       }
       if (live) {
+        rebase(cur);
         const float neg_m = m_run == -INFINITY ? 0.f : -m_run;
         f16x8 p[2];
         softmax_half(cur, neg_m, p);
@@ -1260,6 +1284,8 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
         if (kMaskSlots == 2) live = adds(t, mx, cur);
         if (live) {
           update_max(cur, nxt[0], &nxt[1], mx);
+          rebase(cur[0]);
+          rebase(cur[1]);
           const float neg_m = m_run == -INFINITY ? 0.f : -m_run;
           f16x8 p0[2], p1[2];
           softmax_half(cur[0], neg_m, p0);
