@@ -63,3 +63,14 @@ def test_dense_to_pages(cuda, case, form, dtype):
     P = max(1, -(-S // PAGE))
     assert torch.equal(table.cpu(), torch.arange(B * P, dtype=torch.int32).view(B, P))
     assert (cache.num_pages, cache.Hkv, cache.D) == (B * P, Hkv, D)
+
+
+@pytest.mark.parametrize("S", [0, 100])
+def test_empty_batch(cuda, S):
+    """No sequences: empty pages and an empty table."""
+    import torch_spyre_amd as tsa
+
+    k = torch.empty((0, 8, S, 128), dtype=torch.float16, device=cuda)
+    cache, table = tsa.dense_to_pages(k, k)
+    assert cache.k.shape == (0, 8, 2, PAGE, 64) and cache.v.shape == (0, 8, 128, PAGE)
+    assert cache.num_pages == 0 and table.shape == (0, max(1, -(-S // PAGE)))

@@ -111,10 +111,11 @@ extern "C" int spyre_dense_to_pages_f16(const void* k, const int64_t* k_strides,
                                         const int64_t* v_strides, void* k_pages, void* v_pages, int B, int Hkv,
                                         int S, int D, void* stream) {
   spyre_hip::clear_error();
-  SPYRE_REQUIRE(k_strides && v_strides && k_pages && v_pages && (S == 0 || (k && v)), SPYRE_EINVAL,
-                "null pointer argument");
   SPYRE_REQUIRE(B >= 0 && Hkv > 0 && S >= 0, SPYRE_EINVAL, "bad sizes B=%d Hkv=%d S=%d", B, Hkv, S);
   SPYRE_REQUIRE(D > 0 && D % 64 == 0, SPYRE_EUNSUPPORTED, "head_dim %d not a multiple of 64", D);
+  if (B == 0) return SPYRE_OK;  // no page: empty tensors have no address
+  SPYRE_REQUIRE(k_strides && v_strides && k_pages && v_pages && (S == 0 || (k && v)), SPYRE_EINVAL,
+                "null pointer argument");
   auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   SPYRE_REQUIRE(aligned(k) && aligned(v) && aligned(k_pages) && aligned(v_pages), SPYRE_EINVAL,
                 "k, v and the pages must be 16-byte aligned");
@@ -124,7 +125,6 @@ extern "C" int spyre_dense_to_pages_f16(const void* k, const int64_t* k_strides,
   const int64_t P = S > 0 ? (static_cast<int64_t>(S) + kPage - 1) / kPage : 1;
   const int64_t units = B * P * Hkv * (D / 64);
   SPYRE_REQUIRE(units < (int64_t{1} << 31) - kUnitWaves, SPYRE_EUNSUPPORTED, "too many pages");
-  if (units == 0) return SPYRE_OK;
   PagesArgs a{static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v), k_strides[0], k_strides[1],
               k_strides[2], v_strides[0], v_strides[1], v_strides[2], static_cast<uint16_t*>(k_pages),
               static_cast<uint16_t*>(v_pages), static_cast<uint32_t>(Hkv), static_cast<uint32_t>(P),
