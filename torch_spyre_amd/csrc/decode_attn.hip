@@ -43,6 +43,8 @@
 // (sequence, KV head) combines them (merge_in_kernel).
 
 #include <hip/hip_runtime.h>
+#include <time.h>
+#include <unistd.h>
 
 #include <algorithm>
 #include <atomic>
@@ -1564,10 +1566,41 @@ extern "C" int spyre_paged_decode_attn_f16(const void* q, const void* k_cache, c
 
 namespace spyre_hip {
 
+namespace {
+
+// A value that another process, or another run of this one, would not take:
+// the time, the process, and where its stack and this library lie.
+uint64_t ticket_seed() {
+  timespec t{};
+  clock_gettime(CLOCK_REALTIME, &t);
+  return static_cast<uint64_t>(t.tv_sec) * 1000000007u + static_cast<uint64_t>(t.tv_nsec) * 4294967311u +
+         static_cast<uint64_t>(getpid()) * 2654435761u + reinterpret_cast<uintptr_t>(&t) / 16 * 40503u +
+         reinterpret_cast<uintptr_t>(&ticket_seed) / 4096;
+}
+
+// One-to-one on 32 bits: odd multipliers (Fibonacci hashing: 2^32 over the
+// golden ratio) and exclusive ors with the value's own high half.
+uint32_t mix32(uint32_t x) {
+  for (int i = 0; i < 3; ++i) {
+    x ^= x >> 16;
+    x *= 0x9e3779b1u;
+  }
+  return x ^ x >> 15;
+}
+
+}  // namespace
+
+// Flags lie in memory that is never cleared first, so a value must not be one
+// that other data leaves there (lengths, positions, page numbers): a counter
+// would be.  A one-to-one mix of a counter that starts somewhere else in
+// every process: no value again in 2^32 calls, and any word equals it by
+// a chance of 2^-32.
 uint32_t next_call_ticket() {
-  static std::atomic<uint32_t> tickets{0};
-  uint32_t t = tickets.fetch_add(1, std::memory_order_relaxed) + 1;
-  if (t == 0) t = tickets.fetch_add(1, std::memory_order_relaxed) + 1;  // 0: a cleared flag
+  static const uint32_t seed = mix32(static_cast<uint32_t>(ticket_seed())) ^ static_cast<uint32_t>(ticket_seed() >> 32);
+  static std::atomic<uint32_t> calls{0};
+  uint32_t t;
+  do t = mix32(calls.fetch_add(1, std::memory_order_relaxed) + seed);
+  while (t == 0);  // 0: a cleared flag
   return t;
 }
 

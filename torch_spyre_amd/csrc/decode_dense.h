@@ -26,8 +26,9 @@ struct DenseDecodePlan {
 // 64-512 tokens).
 DenseDecodePlan dense_decode_plan(int B, int Hq, int Hkv, int Skv, int D);
 
-// A nonzero value, new on every call (process-wide): the arrival-flag value
-// of a kernel whose workgroups merge their partials in the same launch.
+// A nonzero value, new on every call (process-wide) and unlike what other
+// data leaves in memory: the arrival-flag value of a kernel whose workgroups
+// merge their partials in the same launch, in a workspace never cleared.
 uint32_t next_call_ticket();
 
 // Launches the plan: q strides {b, h} and K / V strides {b, h, s} in
