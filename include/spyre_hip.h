@@ -344,6 +344,19 @@ int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const void* k,
                        size_t workspace_bytes, int B, int Hq, int Hkv, int Sq, int Skv, int D,
                        void* stream);
 
+/* spyre_sdpa_fwd_f16 with a workspace of its own for every call in flight:
+ * a call whose fp16 / bool mask is staged as it lies then also splits its
+ * keys, the partials and arrival flags in the workspace
+ * (spyre_sdpa_fwd_f16 leaves the workspace alone in those calls, so that
+ * they may share one; results within the SDPA tolerance of each other).
+ * Same arguments.  No reference counterpart. */
+int spyre_sdpa_fwd_own_f16(const void* q, const int64_t* q_strides, const void* k,
+                           const int64_t* k_strides, const void* v, const int64_t* v_strides,
+                           const void* attn_mask, int mask_kind, const int64_t* mask_strides,
+                           int is_causal, float scale, void* out, float* lse, void* workspace,
+                           size_t workspace_bytes, int B, int Hq, int Hkv, int Sq, int Skv, int D,
+                           void* stream);
+
 #ifdef __cplusplus
 }
 #endif

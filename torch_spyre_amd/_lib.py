@@ -106,6 +106,10 @@ SIGNATURES = {
                                    POINTER(c_int64), c_void_p, c_int, POINTER(c_int64), c_int, c_float,
                                    c_void_p, c_void_p, c_void_p, c_size_t, c_int, c_int, c_int, c_int,
                                    c_int, c_int, c_void_p]),
+    "spyre_sdpa_fwd_own_f16": (c_int, [c_void_p, POINTER(c_int64), c_void_p, POINTER(c_int64), c_void_p,
+                                   POINTER(c_int64), c_void_p, c_int, POINTER(c_int64), c_int, c_float,
+                                   c_void_p, c_void_p, c_void_p, c_size_t, c_int, c_int, c_int, c_int,
+                                   c_int, c_int, c_void_p]),
 }
 
 _lib = None

@@ -2459,12 +2459,11 @@ extern "C" size_t spyre_sdpa_fwd_min_workspace_bytes(const void* attn_mask, int 
   return mp.route == kRouteCopied ? std::min(mp.copy_bytes, vt) : vt;
 }
 
-extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const void* k,
-                                  const int64_t* k_strides, const void* v, const int64_t* v_strides,
-                                  const void* attn_mask, int mask_kind, const int64_t* mask_strides,
-                                  int is_causal, float scale, void* out, float* lse,
-                                  void* workspace, size_t workspace_bytes, int B, int Hq, int Hkv,
-                                  int Sq, int Skv, int D, void* stream) {
+// own: no other call in flight uses the workspace.
+static int sdpa_fwd(bool own, const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides,
+                    const void* v, const int64_t* v_strides, const void* attn_mask, int mask_kind,
+                    const int64_t* mask_strides, int is_causal, float scale, void* out, float* lse, void* workspace,
+                    size_t workspace_bytes, int B, int Hq, int Hkv, int Sq, int Skv, int D, void* stream) {
   spyre_hip::clear_error();
   SPYRE_REQUIRE(q_strides && k_strides && v_strides, SPYRE_EINVAL, "null stride argument");
   SPYRE_REQUIRE((Sq == 0 || (q && out)) && (Skv == 0 || (k && v)), SPYRE_EINVAL,
@@ -2508,7 +2507,10 @@ extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const
                 SPYRE_ENOSPC, "workspace %zu < %zu bytes (or misaligned)", workspace_bytes, need);
   if (Sq == 0) return SPYRE_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const size_t ws_room = workspace && aligned16(workspace) ? workspace_bytes : 0;
+  // A shared workspace stays untouched by calls whose mask is staged as it
+  // lies, so these may overlap; such a call has no key split.
+  const bool staged = mask_kind != kNoMask && mp.route == kRouteStaged;
+  const size_t ws_room = workspace && aligned16(workspace) && (own || !staged) ? workspace_bytes : 0;
   // Decode that reads its mask as it lies: no copy, no relayout of V.
   const bool direct = mask_kind == kNoMask || mask_strides[3] == 1;
   const spyre_hip::DenseDecodePlan dp =
@@ -2722,3 +2724,26 @@ extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const
   SPYRE_REQUIRE(e == hipSuccess, SPYRE_EHIP, "sdpa launch failed: %s", hipGetErrorString(e));
   return SPYRE_OK;
 }
+
+#define SPYRE_SDPA_ARGS                                                                                            \
+  q, q_strides, k, k_strides, v, v_strides, attn_mask, mask_kind, mask_strides, is_causal, scale, out, lse, workspace, \
+      workspace_bytes, B, Hq, Hkv, Sq, Skv, D, stream
+
+extern "C" int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const void* k,
+                                  const int64_t* k_strides, const void* v, const int64_t* v_strides,
+                                  const void* attn_mask, int mask_kind, const int64_t* mask_strides,
+                                  int is_causal, float scale, void* out, float* lse,
+                                  void* workspace, size_t workspace_bytes, int B, int Hq, int Hkv,
+                                  int Sq, int Skv, int D, void* stream) {
+  return sdpa_fwd(false, SPYRE_SDPA_ARGS);
+}
+
+extern "C" int spyre_sdpa_fwd_own_f16(const void* q, const int64_t* q_strides, const void* k,
+                                      const int64_t* k_strides, const void* v, const int64_t* v_strides,
+                                      const void* attn_mask, int mask_kind, const int64_t* mask_strides,
+                                      int is_causal, float scale, void* out, float* lse,
+                                      void* workspace, size_t workspace_bytes, int B, int Hq, int Hkv,
+                                      int Sq, int Skv, int D, void* stream) {
+  return sdpa_fwd(true, SPYRE_SDPA_ARGS);
+}
+#undef SPYRE_SDPA_ARGS

@@ -102,11 +102,11 @@ std::tuple<at::Tensor, at::Tensor> sdpa_fwd(const at::Tensor& query, const at::T
                                                kind != SPYRE_MASK_NONE ? mstrides : nullptr, B, Hq, Hkv, Sq, Skv, D);
   at::Tensor ws = need ? at::empty({static_cast<int64_t>(need)}, f16.dtype(at::kByte)) : at::Tensor();
   check_rc("spyre_sdpa_fwd_f16",
-           spyre_sdpa_fwd_f16(q.data_ptr(), qs, k.data_ptr(), ks, v.data_ptr(), vs,
-                              kind != SPYRE_MASK_NONE ? mask.data_ptr() : nullptr, kind,
-                              kind != SPYRE_MASK_NONE ? mstrides : nullptr, is_causal ? 1 : 0,
-                              static_cast<float>(s), out.data_ptr(), return_lse ? lse.data_ptr<float>() : nullptr,
-                              need ? ws.data_ptr() : nullptr, need, B, Hq, Hkv, Sq, Skv, D, stream_of(q)));
+           spyre_sdpa_fwd_own_f16(q.data_ptr(), qs, k.data_ptr(), ks, v.data_ptr(), vs,
+                                  kind != SPYRE_MASK_NONE ? mask.data_ptr() : nullptr, kind,
+                                  kind != SPYRE_MASK_NONE ? mstrides : nullptr, is_causal ? 1 : 0,
+                                  static_cast<float>(s), out.data_ptr(), return_lse ? lse.data_ptr<float>() : nullptr,
+                                  need ? ws.data_ptr() : nullptr, need, B, Hq, Hkv, Sq, Skv, D, stream_of(q)));
   return {out.transpose(1, 2), lse};
 }
 

@@ -171,7 +171,8 @@ def scaled_dot_product_attention(query: torch.Tensor, key: torch.Tensor, value: 
     Runs the C++ kernel of ``spyre::sdpa_fwd`` (checks, outputs and the
     call's workspace from the caching allocator, launch on the current
     stream); with a ``workspace`` of the caller's, the library call is made
-    here with that workspace."""
+    here with that workspace, which calls with a float16 / boolean mask of
+    whole 16-byte rows leave untouched (and so take no key split)."""
     if dropout_p > 0.0:
         raise Unsupported("Attention dropout not implemented")
     if workspace is not None:
@@ -205,7 +206,8 @@ class SdpaCall:
                  enable_gqa: bool = False, return_lse: bool = False, workspace: Optional[torch.Tensor] = None):
         self._args, self.out, self.lse, self._keep = _prepare(query, key, value, attn_mask, 0.0, is_causal,
                                                               scale, enable_gqa, return_lse, workspace, False)
-        self._fn = _lib.lib().spyre_sdpa_fwd_f16
+        # A caller's workspace may serve other calls at the same time.
+        self._fn = _lib.lib().spyre_sdpa_fwd_own_f16 if workspace is None else _lib.lib().spyre_sdpa_fwd_f16
         self._device = query.device
         self._return_lse = return_lse
 
