@@ -24,6 +24,7 @@ from typing import Optional
 import torch
 
 from . import _lib
+from ._workspace import StreamWorkspaces
 from .layout import DataFormats, SpyreTensorLayout, get_device_dtype
 from .relayout import _require_cuda, _require_on, _stream_ptr, h2d_buffer
 
@@ -156,11 +157,12 @@ class _DecodeArgs:
         # caller's may be shared by calls in flight, as one-chunk calls allow.
         L = _lib.lib()
         self.call_fn = L.spyre_paged_decode_attn_call_f16 if workspace is None else L.spyre_paged_decode_attn_f16
+        self.own_ws = False  # the single call writes a workspace of this object's own
         if workspace is None:
             with torch.cuda.device(q.device):
-                need = max(need, L.spyre_paged_decode_attn_call_workspace_bytes(B, Hq, Hkv, D, max_context_len,
-                                                                                split_tokens))
-            workspace = torch.empty(max(need, 4), dtype=torch.uint8, device=q.device)
+                spread = L.spyre_paged_decode_attn_call_workspace_bytes(B, Hq, Hkv, D, max_context_len, split_tokens)
+            self.own_ws = spread > need or max_context_len > CHUNK_WAVES * split_tokens
+            workspace = torch.empty(max(need, spread, 4), dtype=torch.uint8, device=q.device)
         elif workspace.numel() * workspace.element_size() < need:
             raise ValueError(f"workspace holds {workspace.numel() * workspace.element_size()} bytes, need {need}")
         self.q, self.k, self.v, self.table, self.lens = q, k_cache, v_cache, block_table, context_lens
@@ -216,14 +218,16 @@ class PagedDecode:
 
     Checks shapes, dtypes and the workspace once; each launch then only
     passes the stored device pointers to the library (the tensors must stay
-    alive and keep their storage; the launches of one object follow one
-    another, as they share its workspace).  ``__call__`` is the single-call
+    alive and keep their storage).  ``__call__`` is the single-call
     entry (one kernel when max_context_len fits one chunk); ``split()`` and
     ``merge()`` launch the two passes separately (the split pass then
-    writes every chunk's partial to the workspace).  Each launch goes to the
+    writes every chunk's partial to the workspace, the one they share).  Each launch goes to the
     stream current at that moment, so the calls can be captured into a HIP
     graph (the library allocates and clears nothing: the arrival flags of
-    chunks merged in the kernel are cleared by the call that sets them)."""
+    chunks merged in the kernel are cleared by the call that sets them).
+    Without a ``workspace`` of the caller's, the single call has one per
+    stream and per capture (StreamWorkspaces), allocated at the first launch
+    there: launches on several streams may overlap."""
 
     def __init__(self, q, k_cache, v_cache, block_table, context_lens, scale=None,
                  split_tokens: int = 512, max_context_len: Optional[int] = None, workspace=None,
@@ -249,10 +253,11 @@ class PagedDecode:
         self._merge_fn = L.spyre_paged_decode_attn_merge_f16
         lse_ptr = lse.data_ptr() if lse is not None else None
         self._device = q.device
-        self._call_args = (q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_table.data_ptr(),
-                           block_table.stride(0), context_lens.data_ptr(), self.out.data_ptr(), lse_ptr,
-                           a.ws.data_ptr(), a.ws_bytes, a.B, a.Hq, a.Hkv, a.D, PAGE, a.num_pages,
-                           a.max_ctx, a.split, a.scale)
+        before = (q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_table.data_ptr(),
+                  block_table.stride(0), context_lens.data_ptr(), self.out.data_ptr(), lse_ptr)
+        after = (a.ws_bytes, a.B, a.Hq, a.Hkv, a.D, PAGE, a.num_pages, a.max_ctx, a.split, a.scale)
+        self._call_args = (*before, a.ws.data_ptr(), *after)
+        self._spaces = StreamWorkspaces(before, a.ws, after, a.stream) if a.own_ws else None
         self._split_args = (q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_table.data_ptr(),
                             block_table.stride(0), context_lens.data_ptr(), a.ws.data_ptr(), a.ws_bytes,
                             a.B, a.Hq, a.Hkv, a.D, PAGE, a.num_pages, a.max_ctx, a.split, a.scale)
@@ -269,7 +274,13 @@ class PagedDecode:
         return self.out
 
     def __call__(self) -> torch.Tensor:
-        _lib.check("spyre_paged_decode_attn_f16", self._call_fn(*self._call_args, _stream_ptr(self._device)))
+        stream = _stream_ptr(self._device)
+        if self._spaces is None:
+            rc = self._call_fn(*self._call_args, stream)
+        else:
+            args, _held = self._spaces.on(stream)
+            rc = self._call_fn(*args)
+        _lib.check("spyre_paged_decode_attn_f16", rc)
         return self.out
 
 

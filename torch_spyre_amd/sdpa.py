@@ -32,6 +32,7 @@ from typing import Optional
 import torch
 
 from . import _lib
+from ._workspace import StreamWorkspaces
 from .relayout import _require_cuda, _require_on, _stream_ptr
 
 MASK_NONE, MASK_F16, MASK_F32, MASK_BOOL = 0, 1, 2, 3
@@ -157,6 +158,7 @@ def _prepare(query, key, value, attn_mask, dropout_p, is_causal, scale, enable_g
     return args, out.transpose(1, 2), lse, (q, k, v, mask, workspace)
 
 
+_WS_ARG = 13  # the workspace among _prepare's library arguments
 _SDPA_FWD = torch.ops.spyre.sdpa_fwd.default
 
 
@@ -199,7 +201,9 @@ class SdpaCall:
     caller may rewrite their contents between calls.  Every call writes the
     same ``out`` (and ``lse``), on the stream current at that moment, so the
     calls can be captured into a HIP graph (the library allocates and clears
-    nothing)."""
+    nothing).  Without a ``workspace`` of the caller's, a call that needs one
+    has one per stream and per capture (StreamWorkspaces), allocated at the
+    first launch there: launches on several streams may overlap."""
 
     def __init__(self, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
                  attn_mask: Optional[torch.Tensor] = None, is_causal: bool = False, scale: Optional[float] = None,
@@ -210,9 +214,20 @@ class SdpaCall:
         self._fn = _lib.lib().spyre_sdpa_fwd_own_f16 if workspace is None else _lib.lib().spyre_sdpa_fwd_f16
         self._device = query.device
         self._return_lse = return_lse
+        own = self._keep[-1] if workspace is None else None
+        self._spaces = None
+        if own is not None:
+            self._spaces = StreamWorkspaces(self._args[:_WS_ARG], own, self._args[_WS_ARG + 1:],
+                                            _stream_ptr(self._device))
 
     def __call__(self):
-        _lib.check("spyre_sdpa_fwd_f16", self._fn(*self._args, _stream_ptr(self._device)))
+        stream = _stream_ptr(self._device)
+        if self._spaces is None:
+            rc = self._fn(*self._args, stream)
+        else:
+            args, _held = self._spaces.on(stream)
+            rc = self._fn(*args)
+        _lib.check("spyre_sdpa_fwd_f16", rc)
         return (self.out, self.lse) if self._return_lse else self.out
 
 
