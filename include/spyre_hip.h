@@ -349,7 +349,16 @@ int spyre_sdpa_fwd_f16(const void* q, const int64_t* q_strides, const void* k,
  * keys, the partials and arrival flags in the workspace
  * (spyre_sdpa_fwd_f16 leaves the workspace alone in those calls, so that
  * they may share one; results within the SDPA tolerance of each other).
- * Same arguments.  No reference counterpart. */
+ * Same arguments; the workspace holds spyre_sdpa_fwd_own_workspace_bytes:
+ * spyre_sdpa_fwd_call_workspace_bytes less what the call's kernels do not
+ * use (V's relayout for fp32 masks with contiguous keys, a copy of a mask
+ * that a decode call of one row tile reads as it lies).  A call given less
+ * for its partials runs unsplit; SPYRE_ENOSPC for less than a copied mask's
+ * smaller form or, for fp32 masks whose keys are not contiguous, V's
+ * relayout.  No reference counterpart. */
+size_t spyre_sdpa_fwd_own_workspace_bytes(const void* attn_mask, int mask_kind,
+                                          const int64_t* mask_strides, int B, int Hq, int Hkv,
+                                          int Sq, int Skv, int D);
 int spyre_sdpa_fwd_own_f16(const void* q, const int64_t* q_strides, const void* k,
                            const int64_t* k_strides, const void* v, const int64_t* v_strides,
                            const void* attn_mask, int mask_kind, const int64_t* mask_strides,

@@ -241,6 +241,36 @@ def test_sdpa_call_workspace_routes(tsa):
     assert need(2, [0, 0, 160, 1], 160) == vt
 
 
+def test_sdpa_own_workspace_holds_what_is_read(tsa):
+    """A call with a workspace of its own: nothing for an fp32 mask with
+    contiguous keys but a key split's partials, V's relayout when its keys
+    are not contiguous; decode that reads the mask as it lies, its partials
+    alone.  Elsewhere what the shared entry asks for."""
+    from torch_spyre_amd import _lib
+
+    L = _lib.lib()
+
+    def need(kind, strides, B, Hq, Hkv, Sq, Skv, D, ptr=0x10000):
+        args = (ptr, kind, _lib.i64_array(strides), B, Hq, Hkv, Sq, Skv, D)
+        own, shared = L.spyre_sdpa_fwd_own_workspace_bytes(*args), L.spyre_sdpa_fwd_call_workspace_bytes(*args)
+        assert own <= shared
+        return own, shared
+
+    vt = L.spyre_sdpa_fwd_workspace_bytes(2, 2, 160, 128)
+    assert need(2, [0, 0, 160, 1], 2, 8, 2, 100, 160, 128) == (0, vt)
+    assert need(2, [0, 0, 1, 100], 2, 8, 2, 100, 160, 128) == (vt, vt)
+    own, shared = need(2, [0, 0, 2100, 1], 1, 8, 2, 40, 2100, 128)  # split keys: partials of [128 + 2] fp32
+    assert own > 0 and own % (8 * 40 * 130 * 4) == 0
+    # decode of one row tile: 4 sequences in one block each; 2048 keys in 16 splits
+    assert need(2, [0, 0, 160, 1], 4, 32, 8, 1, 160, 128) == (0, L.spyre_sdpa_fwd_workspace_bytes(4, 8, 160, 128))
+    assert need(3, [77, 0, 77, 1], 4, 32, 8, 1, 77, 128) == (0, 4 * 80)
+    assert need(2, [0, 0, 2048, 1], 1, 32, 8, 1, 2048, 128)[0] == (32 * 130 + 8) * 16 * 4
+    # fp16 / bool: as the shared entry
+    for kind, strides in ((1, [0, 0, 77, 1]), (3, [100 * 77, 0, 77, 1]), (1, [0, 0, 1, 100])):
+        own, shared = need(kind, strides, 2, 8, 2, 100, 77, 128)
+        assert own == shared > 0
+
+
 def test_paged_decode_workspace_and_kernel_count(tsa):
     """The paged decode's workspace (host code): fp32 chunk partials
     [B, Hkv, chunks, g, D + 2], then a 4-byte arrival flag per (sequence, KV

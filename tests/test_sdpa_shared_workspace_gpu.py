@@ -1,6 +1,7 @@
 """Dense SDPA calls and the workspace they are given: a masked call whose
 mask is staged as it lies leaves a caller's workspace alone, so such calls
-may be in flight at once on one workspace."""
+may be in flight at once on one workspace; calls that bring none allocate
+what their kernels use."""
 
 import pytest
 import torch
@@ -50,3 +51,28 @@ def test_staged_mask_leaves_a_callers_workspace_alone(cuda, case, kind):
     eager = tsa.scaled_dot_product_attention(*args, enable_gqa=True)
     assert_close(own(), ref)
     assert torch.equal(own.out.view(torch.int16), eager.view(torch.int16))
+
+
+@pytest.mark.parametrize("case", [(2, 16, 16, 300, 301, 64), (1, 32, 8, 1, 255, 128), (16, 32, 8, 1, 2048, 128),
+                                  (2, 8, 8, 1, 600, 64)], ids=str)
+def test_fp32_mask_allocates_no_copy_of_v(cuda, case):
+    import torch_spyre_amd as tsa
+    from torch_spyre_amd import _lib
+
+    B, Hq, Hkv, Sq, Skv, D = case
+    q = randn((B, Hq, Sq, D), SEED + 585)
+    k, v = randn((B, Hkv, Skv, D), SEED + 586), randn((B, Hkv, Skv, D), SEED + 587)
+    mask = torch.randn((1, Hq, Sq, Skv), generator=torch.Generator().manual_seed(SEED + 588))
+    args = (q.to(cuda), k.to(cuda), v.to(cuda), mask.to(cuda))
+    m = args[3].expand(B, Hq, Sq, Skv)
+    part = _lib.lib().spyre_sdpa_fwd_own_workspace_bytes(m.data_ptr(), 2, _lib.i64_array(m.stride()), B, Hq, Hkv, Sq,
+                                                         Skv, D)
+    assert part < _lib.lib().spyre_sdpa_fwd_workspace_bytes(B, Hkv, Skv, D)
+    tsa.scaled_dot_product_attention(*args, enable_gqa=True)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    out = tsa.scaled_dot_product_attention(*args, enable_gqa=True)
+    peak = torch.cuda.max_memory_allocated() - before
+    assert peak <= part + 2 * out.numel() + 4 * 512  # (the allocator rounds to 512 bytes)
+    assert_close(out, OA.sdpa_cpu_fp32(q, k, v, attn_mask=mask))

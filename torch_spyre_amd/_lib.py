@@ -102,6 +102,8 @@ SIGNATURES = {
                                                        c_int, c_int, c_int]),
     "spyre_sdpa_fwd_min_workspace_bytes": (c_size_t, [c_void_p, c_int, POINTER(c_int64), c_int, c_int, c_int,
                                                       c_int, c_int, c_int]),
+    "spyre_sdpa_fwd_own_workspace_bytes": (c_size_t, [c_void_p, c_int, POINTER(c_int64), c_int, c_int, c_int,
+                                                      c_int, c_int, c_int]),
     "spyre_sdpa_fwd_f16": (c_int, [c_void_p, POINTER(c_int64), c_void_p, POINTER(c_int64), c_void_p,
                                    POINTER(c_int64), c_void_p, c_int, POINTER(c_int64), c_int, c_float,
                                    c_void_p, c_void_p, c_void_p, c_size_t, c_int, c_int, c_int, c_int,

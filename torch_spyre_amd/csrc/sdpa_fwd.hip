@@ -2424,9 +2424,10 @@ extern "C" size_t spyre_sdpa_fwd_workspace_bytes(int B, int Hkv, int Skv, int D)
   return static_cast<size_t>(B) * Hkv * D * s64_of(Skv) * sizeof(_Float16);
 }
 
-extern "C" size_t spyre_sdpa_fwd_call_workspace_bytes(const void* attn_mask, int mask_kind,
-                                                      const int64_t* mask_strides, int B, int Hq, int Hkv,
-                                                      int Sq, int Skv, int D) {
+// The workspace of a call; own: of spyre_sdpa_fwd_own_f16, which asks for
+// nothing that the kernels the call runs leave alone.
+static size_t call_workspace(bool own, const void* attn_mask, int mask_kind, const int64_t* mask_strides, int B, int Hq,
+                             int Hkv, int Sq, int Skv, int D) {
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || Sq < 0 || Skv < 0 || (D != 64 && D != 128)) return 0;
   if (mask_kind == kNoMask) {  // a key split's partials (calls without the causal flag)
     const size_t split = plan_grid(B, Hq, Hkv, Sq, Skv, D, false, SIZE_MAX).part_bytes;
@@ -2435,17 +2436,31 @@ extern "C" size_t spyre_sdpa_fwd_call_workspace_bytes(const void* attn_mask, int
   }
   if (!mask_strides || mask_kind < kNoMask || mask_kind > kMaskBool) return 0;
   const MaskPlan mp = plan_mask(attn_mask, mask_kind, mask_strides, B, Hq, Sq, Skv);
-  // Decode that reads the mask as it lies takes its partials alone, but the
-  // call also holds what the kernels that stage or copy the mask would need.
+  // Decode that reads the mask as it lies takes its partials alone; the
+  // shared entry also asks for what the kernels that stage or copy the mask
+  // would need.
   GridPlan gs;
   if (mask_strides[3] == 1 && short_grid(B, Hq, Hkv, Sq, Skv, D, SIZE_MAX, gs))
-    return std::max(gs.part_bytes, min_room(mp, B, Hkv, Skv, D));
+    return own ? gs.part_bytes : std::max(gs.part_bytes, min_room(mp, B, Hkv, Skv, D));
   const spyre_hip::DenseDecodePlan dp = dense_route(B, Hq, Hkv, Sq, Skv, D, false, mask_kind, mask_strides);
   const size_t decode = dp.ok ? dp.ws_bytes : 0;
-  if (mp.route == kRouteVt) return std::max(decode, spyre_sdpa_fwd_workspace_bytes(B, Hkv, Skv, D));
+  const size_t vt = spyre_sdpa_fwd_workspace_bytes(B, Hkv, Skv, D);
+  if (mp.route == kRouteVt) return std::max(decode, vt);
   const size_t part = masked_grid(mp, mask_kind, B, Hq, Hkv, Sq, Skv, D, SIZE_MAX).part_bytes;
-  if (mp.route == kRouteF32) return std::max({decode, part, spyre_sdpa_fwd_workspace_bytes(B, Hkv, Skv, D)});
+  if (mp.route == kRouteF32) return std::max({decode, part, own ? 0 : vt});
   return std::max(decode, part ? copy_room(mp) + part : mp.copy_bytes);
+}
+
+extern "C" size_t spyre_sdpa_fwd_call_workspace_bytes(const void* attn_mask, int mask_kind,
+                                                      const int64_t* mask_strides, int B, int Hq, int Hkv,
+                                                      int Sq, int Skv, int D) {
+  return call_workspace(false, attn_mask, mask_kind, mask_strides, B, Hq, Hkv, Sq, Skv, D);
+}
+
+extern "C" size_t spyre_sdpa_fwd_own_workspace_bytes(const void* attn_mask, int mask_kind,
+                                                     const int64_t* mask_strides, int B, int Hq, int Hkv,
+                                                     int Sq, int Skv, int D) {
+  return call_workspace(true, attn_mask, mask_kind, mask_strides, B, Hq, Hkv, Sq, Skv, D);
 }
 
 extern "C" size_t spyre_sdpa_fwd_min_workspace_bytes(const void* attn_mask, int mask_kind,
@@ -2499,14 +2514,6 @@ static int sdpa_fwd(bool own, const void* q, const int64_t* q_strides, const voi
   MaskPlan mp = plan_mask(attn_mask, mask_kind, mask_strides, B, Hq, Sq, Skv);
   if (mp.route == kRouteCopied && (!workspace || workspace_bytes < mp.copy_bytes || !aligned16(workspace)))
     mp.route = kRouteVt;
-  // (fp32 masks ask for V's relayout whichever kernel runs.)
-  const size_t need = mp.route >= kRouteF32      ? spyre_sdpa_fwd_workspace_bytes(B, Hkv, Skv, D)
-                      : mp.route == kRouteCopied ? mp.copy_bytes
-                                                 : 0;
-  SPYRE_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && aligned16(workspace)),
-                SPYRE_ENOSPC, "workspace %zu < %zu bytes (or misaligned)", workspace_bytes, need);
-  if (Sq == 0) return SPYRE_OK;
-  hipStream_t st = static_cast<hipStream_t>(stream);
   // A shared workspace stays untouched by calls whose mask is staged as it
   // lies, so these may overlap; such a call has no key split.
   const bool staged = mask_kind != kNoMask && mp.route == kRouteStaged;
@@ -2520,6 +2527,17 @@ static int sdpa_fwd(bool own, const void* q, const int64_t* q_strides, const voi
                      (dp.ws_bytes == 0 || ws_room >= dp.ws_bytes);
   GridPlan gs;
   const bool as_it_lies = mask_kind != kNoMask && direct && (dense || short_grid(B, Hq, Hkv, Sq, Skv, D, ws_room, gs));
+  // (The shared entry asks for V's relayout for every fp32 mask and for a
+  // copied mask's copy whichever kernel runs.)
+  const size_t vt_bytes = spyre_sdpa_fwd_workspace_bytes(B, Hkv, Skv, D);
+  const size_t need = own && as_it_lies                             ? 0
+                      : mp.route == kRouteCopied                    ? mp.copy_bytes
+                      : mp.route >= (own ? kRouteVt : kRouteF32) ? vt_bytes
+                                                                    : 0;
+  SPYRE_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && aligned16(workspace)),
+                SPYRE_ENOSPC, "workspace %zu < %zu bytes (or misaligned)", workspace_bytes, need);
+  if (Sq == 0) return SPYRE_OK;
+  hipStream_t st = static_cast<hipStream_t>(stream);
   if (as_it_lies) mp.route = kRouteNone;
   const bool lds_path = mp.route != kRouteVt;
   // Short query runs pack q heads of a KV head into one block's rows, so

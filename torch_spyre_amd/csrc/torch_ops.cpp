@@ -98,8 +98,8 @@ std::tuple<at::Tensor, at::Tensor> sdpa_fwd(const at::Tensor& query, const at::T
   // The call's workspace (none for causal calls without a mask).
   size_t need = 0;
   if (kind != SPYRE_MASK_NONE || !is_causal)
-    need = spyre_sdpa_fwd_call_workspace_bytes(kind != SPYRE_MASK_NONE ? mask.data_ptr() : nullptr, kind,
-                                               kind != SPYRE_MASK_NONE ? mstrides : nullptr, B, Hq, Hkv, Sq, Skv, D);
+    need = spyre_sdpa_fwd_own_workspace_bytes(kind != SPYRE_MASK_NONE ? mask.data_ptr() : nullptr, kind,
+                                              kind != SPYRE_MASK_NONE ? mstrides : nullptr, B, Hq, Hkv, Sq, Skv, D);
   at::Tensor ws = need ? at::empty({static_cast<int64_t>(need)}, f16.dtype(at::kByte)) : at::Tensor();
   check_rc("spyre_sdpa_fwd_f16",
            spyre_sdpa_fwd_own_f16(q.data_ptr(), qs, k.data_ptr(), ks, v.data_ptr(), vs,

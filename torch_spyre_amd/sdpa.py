@@ -90,13 +90,13 @@ def _geometry_plan(q, k, v, mask, kind: int, is_causal: bool):
     B, Hq, Sq, D = q.shape
     _, Hkv, Skv, _ = k.shape
     mstrides = _lib.i64_array(mask.stride()) if mask is not None else None
-    # The call's workspace: a key split's partials when the blocks would not
-    # fill the device (none for causal calls), a copy with 16-byte rows of
-    # fp16 / bool masks the kernel cannot stage as they lie, room for V's
-    # relayout for fp32 masks.
+    # The workspace of a call that brings none: a key split's partials when
+    # the blocks would not fill the device (none for causal calls), a copy
+    # with 16-byte rows of fp16 / bool masks the kernel cannot stage as they
+    # lie, V's relayout for fp32 masks whose keys are not contiguous.
     need = 0
     if kind != MASK_NONE or not is_causal:
-        need = int(_lib.lib().spyre_sdpa_fwd_call_workspace_bytes(
+        need = int(_lib.lib().spyre_sdpa_fwd_own_workspace_bytes(
             mask.data_ptr() if mask is not None else None, kind, mstrides, B, Hq, Hkv, Sq, Skv, D))
     plan = (_lib.i64_array(q.stride()[:3]), _lib.i64_array(k.stride()[:3]), _lib.i64_array(v.stride()[:3]),
             mstrides, need)
@@ -144,7 +144,7 @@ def _prepare(query, key, value, attn_mask, dropout_p, is_causal, scale, enable_g
         _require_on(workspace, q.device, "workspace")
     if workspace is None and need:
         workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
-    elif workspace is not None and need and kind != MASK_NONE:
+    elif workspace is not None and kind != MASK_NONE:
         # less than the call asks for also serves (no key split; V's relayout instead of the mask's copy)
         floor = int(_lib.lib().spyre_sdpa_fwd_min_workspace_bytes(mask.data_ptr(), kind, mstrides, B, Hq, Hkv, Sq,
                                                                   Skv, D))
