@@ -98,3 +98,10 @@ def test_nests_that_overlap_keep_their_order(cuda):
     run([_nest([(64, 1, 1), (100, 70, 80)], 0, 0), _nest([(40, 1, 1), (90, 50, 75)], 9000, 30)])  # other strides
     run([_nest([(64, 1, 1), (50, 64, 100)], 0, 0), _nest([(36, 1, 1), (50, 64, 100)], 7000, 64)])  # apart
     run([_nest([(17 + i, 1, 1), (20, 40, 1000)], 900 * i, 50 * i) for i in range(10)])
+
+
+@pytest.mark.parametrize("rows", [8730, 8760])
+def test_items_to_a_lane(cuda, rows):
+    """Both sides of one or four items to a lane (rows of 120 items and a
+    remainder; 256 units x 16 blocks of 256 items are 8738.1 rows)."""
+    test_odd_sizes_and_offsets_vs_oracle(cuda, [rows, 1001], 1, torch.float16)

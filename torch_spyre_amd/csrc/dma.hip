@@ -220,8 +220,8 @@ __device__ __forceinline__ void small_block(const char* src, char* dst, const Sm
 // thousand items; as a launch of its own it took 5.6-6.1 us beside a main
 // nest of 14.  fp32 [3, 1021, 2500] to its device layout: 20.2 us in two
 // launches, 17.2 in one of the general kernel, 13.1 here; fp16 [1000, 1000]
-// 9.8 and 4.8.  ITEMS: 4, or 1 for nests that would not fill the device with
-// four to a lane.
+// 9.8 and 4.8.  ITEMS: 4, or 1 for nests that four to a lane leave with few
+// wavefronts in flight (launch_pair).
 template <int VB, int ITEMS>
 __global__ __launch_bounds__(kThreads) void dma_vec_pair_kernel(const char* __restrict__ src_arg,
                                                                 char* __restrict__ dst_arg, SmallNest a_arg,
@@ -1160,7 +1160,14 @@ bool launch_pair(const char* src, char* dst, const std::vector<VecNest>& vs, hip
   const VecNest& va = vs[swap ? 1 : 0];
   if (!small_nest(va, a) || (vs.size() == 2 && !small_nest(vs[swap ? 0 : 1], b))) return false;
   const int64_t cus = dma_device_cus() > 0 ? dma_device_cus() : 256;
-  const bool wide = a.total > 2 * cus * kThreads;
+  // One item to a lane until every unit has 16 blocks: four to a lane leave a
+  // unit a handful of wavefronts, one round trip after another.  fp16 [rows,
+  // 1000] to sticks / back, one / four to a lane, us: 1600 rows (3.2 MB) 2.9 / 4.3,
+  // 3.0 / 4.4; 2300 3.4 / 5.0, 3.4 / 4.8; 4200 4.5 / 5.4, 4.3 / 5.6; 8000 (16 MB,
+  // the line) 7.4 / 7.7, 6.7 / 7.6; past it the two are within 8 % either way
+  // with inputs from HBM (16000: 18.8 / 17.4, 13.9 / 15.2; fp32 [8000, 1000]
+  // 17.1 / 16.2, 13.2 / 14.0).
+  const bool wide = a.total > 16 * cus * kThreads;
   const uint32_t per = kThreads * (wide ? kItems : 1);
   const uint32_t blocks = (a.total + per - 1) / per;
   const dim3 grid(blocks + (b.total + kThreads - 1) / kThreads);
