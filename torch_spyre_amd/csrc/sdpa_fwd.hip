@@ -2017,10 +2017,14 @@ int shape_rows(Shape s) { return s == k256 ? 256 : s == kHalf4 ? 64 : 128; }
 //    but k256 at D 128 where its grid is whole rounds of even blocks (4096 x
 //    4096: 251.8 / 253.7; 8192: 942 / 960; 5000, 2.5 rounds: 408.0 / 383.6),
 //    or causal of two rounds, where each long block is followed by its
-//    complement, and heads that share K and V, which then stay in the L2
-//    (4096: 132.2 / 136.1, with inputs from HBM 136.6 / 136.9; 16 / 8 heads x
-//    8192: 245.8 / 252.1; 32 heads of their own K and V: 187.7 / 172.2; B 2,
-//    four rounds: 274.1 / 267.8);
+//    complement, heads that share K and V, and more than 8 blocks a head.
+//    With q, k, v in the 256 MB cache, as the projections before leave them,
+//    k256 / k128: 3841 rows 130.4 / 132.4, 4096 136.0 / 141.5, 16 / 8 heads x
+//    8192 250.4 / 261.8; from HBM the two are within 1 % (128.8 / 129.8, 140.5
+//    / 139.2, 259.3 / 257.4).  At 8 blocks a head (B 2 x 2048) 78.0 / 79.0, from
+//    HBM 82.9 / 81.5; below, k128 (B 4 x 1024 56.8 / 50.6, B 8 x 512 41.6 / 37.6).
+//    32 heads of their own K and V: 187.7 / 172.2; just past two rounds (4097)
+//    149.4 / 143.7; B 2, four rounds: 274.1 / 267.8;
 //  * key splits, whose blocks are even and end in a store of their partials:
 //    kHalf4 within one round (64 queries x 2000 keys: 25.4 / 20.1 / 20.4 /
 //    17.3; beyond it, B 4: 30.3 / 29.9 / 37.8 / 35.6); at D 128 k256 when its
@@ -2036,7 +2040,7 @@ Shape pick_shape(int64_t pairs, int64_t rows, int g, int keys, int nsplit, int D
   if (rows <= 64) return kHalf8;
   if (blocks(64) <= (nsplit > 1 ? 1 : D == 64 ? 3 : causal || mask_kind != kNoMask ? 2 : 1) * cus) return kHalf4;
   const bool whole = D == 128 && blocks(256) % cus == 0;
-  const bool paired = g > 1 && blocks(256) == 2 * cus && rows >= 14 * 256;
+  const bool paired = g > 1 && blocks(256) == 2 * cus && rows > 8 * 256;
   if (nsplit == 1) return whole && (!causal || paired) ? k256 : k128;
   if (rows <= 128) return D == 128 ? k256 : kHalf8;
   return whole ? k256 : k128;
