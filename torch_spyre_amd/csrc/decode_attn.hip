@@ -966,9 +966,9 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void decode_split_list_ker
 
 // A chunk's kWaves wavefronts spread over kWaves / S workgroups of S, for
 // grids that leave most compute units idle (spread_waves).  One compute unit
-// draws about 46 GB/s from memory however many of its wavefronts ask: a chunk
-// of 4096 tokens of one KV head took 59 us in one workgroup and takes 21 in
-// eight (B 1 x 32 / 8 heads: 700 tokens 14.4 -> 9.2 us, 4096 59.1 -> 20.7,
+// draws about 36 GB/s from memory however many of its wavefronts ask: a chunk
+// of 4096 tokens of one KV head (2.1 MB) took 59 us in one workgroup and takes 21
+// in eight (B 1 x 32 / 8 heads: 700 tokens 14.4 -> 9.2 us, 4096 59.1 -> 20.7,
 // 32768 63.5 -> 32.5; B 8 x 2048 32.0 -> 16.6, B 16 x 4096 60.5 -> 44.9).
 // Every wavefront streams the pages it would stream there, its partial goes
 // to the workspace, and whichever workgroup sees all of a (sequence, KV

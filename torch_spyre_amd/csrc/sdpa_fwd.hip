@@ -333,7 +333,7 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_fwd_kernel(FwdArgs a) {
   }
 }
 
-// ---- 3. attention with K/V tiles shared through LDS (no mask) -------------
+// ---- 3. attention with K/V tiles shared through LDS -------------------------
 //
 // A workgroup of W = 8 or 4 wavefronts takes W x 32 queries of one (sequence,
 // q head), wavefront w 32 of them (or, in half steps, W / 2 x 32 queries;
@@ -349,8 +349,8 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_fwd_kernel(FwdArgs a) {
 // VALU computes step t's softmax the matrix cores already compute step
 // t+1's scores and then step t's P V.  Two LDS slots each hold K(t+1) /
 // K(t+2) and V(t) / V(t+1); the next tiles travel from L2 straight into
-// LDS during a step's math.  LDS rows are padded so that the rows one
-// operand read touches fall in distinct bank groups.  Workgroups are
+// LDS during a step's math.  The 16-byte units of an LDS row are exchanged so
+// that those one operand read touches fall in distinct banks (Lds2).  Workgroups are
 // numbered so that those of one (sequence, KV head) run on one XCD (one L2),
 // and for causal attention each head's latest (heaviest) query block starts
 // first.
@@ -490,8 +490,7 @@ template <bool HALF> struct MaskTile<kNoMask, HALF> {
 // (the running max), so P = exp2(S) needs no per-score FMA.  Otherwise the
 // scale's sign is folded into Q and its magnitude into the exponent's FMA.
 // SLOTS: K / V slots in LDS.  Two: each step's tiles are loaded one step
-// ahead, a barrier per step.  Four (calls without a mask whose blocks have
-// fewer than 256 rows, e.g. decode, where one wavefront computes and the
+// ahead, a barrier per step.  Four (kHalf8 calls without a mask, e.g. decode, where one wavefront computes and the
 // step waits on its loads): loads two steps ahead, a barrier per two steps.
 // HALF (blocks of at most 128 rows, e.g. decode): wavefronts 2r and 2r + 1
 // share row tile r and take one 32-key half of every step each; the pair's
@@ -507,7 +506,7 @@ template <bool HALF> struct MaskTile<kNoMask, HALF> {
 // 777, D 64).
 template <int D, bool PRESCALED, int MK, int SLOTS, bool HALF, int W, bool ANY = false>
 __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
-  static_assert(SLOTS == 2 || (SLOTS == 4 && MK == kNoMask), "four slots leave no room for a mask");
+  static_assert(SLOTS == 2 || (SLOTS == 4 && HALF && MK == kNoMask), "four slots: half steps without a mask");
   // fp32 biases: half steps only (the 32-query block of a full step, 8 KB a
   // wavefront, leaves no room beside K and V), scores scaled and biased in
   // fp32 (log2 units), row sums of the fp32 probabilities and a running max
@@ -837,8 +836,8 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   // exceeds it by more than 2^8, so P <= 256 (fine in fp16) and most steps
   // skip the rescale of O; O / l is exact whatever max is used.
   // PRESCALED: s holds exponents relative to m_use, and so does `ahead`
-  // (the first half of the next step's scores, computed before this
-  // update); a move of m_use shifts both, and the tile.
+  // (the next step's scores, computed before this update); a move of m_use
+  // shifts both, and the tile.
   // The step's row max in the units of m_run.
   // Masked: NaN if a score is, so that a NaN does not leave its step blank.
   auto max_of = [](float x, float y) {
@@ -892,8 +891,8 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
     }
     return any;
   };
-  // ahead2: with a mask, the second half of S(t+1) is complete too.
-  auto update_max = [&](f32x16 (&s)[2], f32x16& ahead, f32x16* ahead2, float mx) {
+  // Masked full steps: s is S(t), ahead S(t+1), both complete.
+  auto update_max = [&](f32x16 (&s)[2], f32x16 (&ahead)[2], float mx) {
     if (__builtin_amdgcn_ballot_w64(mx > m_run + 8.f) != 0) {
       const float m_new = fmaxf(m_run, mx);
       const float alpha = m_new == -INFINITY ? 1.f : fast_exp2(m_run - m_new);
@@ -909,8 +908,8 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
         for (int rr = 0; rr < 16; ++rr) {
           s[0][rr] -= d;
           s[1][rr] -= d;
-          ahead[rr] -= d;
-          if (ahead2) (*ahead2)[rr] -= d;
+          ahead[0][rr] -= d;
+          ahead[1][rr] -= d;
           neg_m_tile[rr] = -m_use;
         }
       }
@@ -1097,6 +1096,10 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
       if (kMaskSlots == 2 && t + 1 < n_tiles && !ANY) dma_m(kb0 + (t + 1) * kKT, (t + 1) & 1);
       if (ANY && t + 1 < n_tiles) read_m(kb0 + (t + 1) * kKT);
     } else if ((t & 1) == 0) {
+      // Steps t, t + 1 read K(t+1), K(t+2), V(t), V(t+1) (slot = tile % 4);
+      // K(t+3), K(t+4), V(t+2), V(t+3) fill the other four slot halves,
+      // whose last readers were steps t - 2 and t - 1, and land by the
+      // barrier after step t + 1.
       if (t + 3 < n_tiles) dma_k((t + 3) % 4);
       if (t + 4 < n_tiles) dma_k(t % 4);
       if (t + 2 < n_tiles) dma_v((t + 2) % 4);
@@ -1179,22 +1182,11 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   // wavefront's last active step S(t+1) reads a stale K slot and is never
   // used.
   auto step = [&](int t, int par, f32x16 (&cur)[2], f32x16 (&nxt)[2]) {
-    if constexpr (SLOTS == 2) {
-      // K(t+2) replaces K(t) (read during step t-1), V(t+1) replaces
-      // V(t-1); both land during this step's math.
-      if (t + 2 < n_tiles) dma_k(t & 1);
-      if (t + 1 < n_tiles) dma_v((t + 1) & 1);
-      if (kMaskSlots == 2 && t + 1 < n_tiles) dma_m(kb0 + (t + 1) * kKT, (t + 1) & 1);
-    } else if ((t & 1) == 0) {
-      // Steps t, t + 1 read K(t+1), K(t+2), V(t), V(t+1) (slot = tile % 4);
-      // K(t+3), K(t+4), V(t+2), V(t+3) fill the other four slot halves,
-      // whose last readers were steps t - 2 and t - 1, and land by the
-      // barrier after step t + 1.
-      if (t + 3 < n_tiles) dma_k((t + 3) % 4);
-      if (t + 4 < n_tiles) dma_k(t % 4);
-      if (t + 2 < n_tiles) dma_v((t + 2) % 4);
-      if (t + 3 < n_tiles) dma_v((t + 3) % 4);
-    }
+    // K(t+2) replaces K(t) (read during step t-1), V(t+1) replaces
+    // V(t-1); both land during this step's math.
+    if (t + 2 < n_tiles) dma_k(t & 1);
+    if (t + 1 < n_tiles) dma_v((t + 1) & 1);
+    if (kMaskSlots == 2 && t + 1 < n_tiles) dma_m(kb0 + (t + 1) * kKT, (t + 1) & 1);
     if (active(t)) {
       f16x8 fr[kNF];
 #pragma unroll
@@ -1260,7 +1252,6 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
           for (int dm = 0; dm < DM; ++dm) mfma(2 * DK + 2 * DM + j * DM + dm, p1[j], o[dm]);
         interleave_reads(2 * DK + 2 * DM, kNF);
       } else {
-
         // A mask can leave a step nothing to add: every score of the
         // wavefront's real rows -inf or more than 32 below its row's running
         // max, so every P rounds to 0 in fp16.  Such a step computes only
@@ -1283,7 +1274,7 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
         interleave_reads(0, 2 * DK);
         if (kMaskSlots == 2) live = adds(t, mx, cur);
         if (live) {
-          update_max(cur, nxt[0], &nxt[1], mx);
+          update_max(cur, nxt, mx);
           rebase(cur[0]);
           rebase(cur[1]);
           const float neg_m = m_run == -INFINITY ? 0.f : -m_run;
@@ -1303,10 +1294,8 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
         }
       }
     }
-    if (SLOTS == 2 || (t & 1)) {
-      dma_wait();
-      __syncthreads();
-    }
+    dma_wait();
+    __syncthreads();
   };
 
   // Prologue: K(0), V(0) in slot 0 and K(1) in slot 1 (four slots: also
