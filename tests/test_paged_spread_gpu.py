@@ -25,6 +25,20 @@ def _run(fn, cache, table, lens, q, max_ctx, split, ws):
     return out.view(torch.int16), lse.view(torch.int32)
 
 
+# Pages of a one-chunk context from which it is spread over workgroups of
+# 1, 2 and 4 streaming wavefronts, the least that leave each of 256 units at
+# most one workgroup.
+FROM = {128: (4, 5, 7), 64: (7, 8, 14)}
+
+
+def _spreads(pairs, D, max_ctx, split):
+    chunks = -(-max_ctx // (8 * split))
+    for S, pages in zip((1, 2, 4), FROM[D]):
+        if pairs * chunks * (8 // S) <= 256:
+            return chunks > 1 or -(-max_ctx // PAGE) >= pages
+    return False
+
+
 # Sequences around one to nine pages, empty ones, one and several chunks
 # (split 64: 512 tokens each, split 512: 4096), 1 / 2 / 4 streaming
 # wavefronts per workgroup (by the number of pairs), 1 to 16 q heads per KV
@@ -41,6 +55,21 @@ def _run(fn, cache, table, lens, q, max_ctx, split, ws):
     ([300, 290, 64, 10] * 4, 32, 8, 128, 512, 300),
     ([900, 700, 10], 32, 8, 128, 512, 800),
     ([300] * 20, 32, 8, 128, 512, 300),
+    # both sides of each line: pairs that fit the device, pages that pay
+    ([192, 150], 32, 8, 128, 512, 192),
+    ([256, 193, 130, 64], 32, 8, 128, 512, 256),
+    ([256, 240] * 4, 32, 8, 128, 512, 256),
+    ([320, 257, 256, 129, 64, 1, 0, 300], 32, 8, 128, 512, 320),
+    ([384, 370] * 8, 32, 8, 128, 512, 384),
+    ([448, 385, 320, 257] * 4, 32, 8, 128, 512, 448),
+    ([448, 440] * 8 + [448], 32, 8, 128, 512, 448),
+    ([384, 350], 16, 16, 64, 512, 384),
+    ([448, 385], 16, 16, 64, 512, 448),
+    ([448, 400, 257], 16, 16, 64, 512, 448),
+    ([512, 449, 257, 200], 16, 16, 64, 512, 512),
+    ([832, 800] * 4, 16, 16, 64, 512, 832),
+    ([896, 833, 513, 257, 256, 129, 64, 0], 16, 16, 64, 512, 896),
+    ([700, 520, 130, 70] * 2, 16, 16, 64, 64, 832),
 ], ids=str)
 def test_spread_equals_one_workgroup(cuda, lens, Hq, Hkv, D, split, max_ctx):
     from torch_spyre_amd import _lib
@@ -54,13 +83,15 @@ def test_spread_equals_one_workgroup(cuda, lens, Hq, Hkv, D, split, max_ctx):
     l = torch.tensor(lens, dtype=torch.int32, device=cuda)
     base = L.spyre_paged_decode_attn_workspace_bytes(B, Hq, Hkv, D, max_ctx, split)
     need = L.spyre_paged_decode_attn_call_workspace_bytes(B, Hq, Hkv, D, max_ctx, split)
-    assert need >= base > 0
+    assert base > 0
+    spread = _spreads(B * Hkv, D, max_ctx, split)
+    assert (need > base) == spread
     ws = torch.full((need,), 0xff, dtype=torch.uint8, device=cuda)
     want = _run(L.spyre_paged_decode_attn_f16, cache, table, l, q, max_ctx, split, ws)
     for size in (need, need, base):  # the second meets the first one's workspace; too small: not spread
         got = _run(L.spyre_paged_decode_attn_call_f16, cache, table, l, q, max_ctx, split, ws[:size])
         assert all(torch.equal(x, y) for x, y in zip(got, want))
-    if need > base:  # an unaligned workspace is not spread either
+    if spread:  # an unaligned workspace is not spread either
         buf = torch.empty(need + 4, dtype=torch.uint8, device=cuda)[4:]
         got = _run(L.spyre_paged_decode_attn_call_f16, cache, table, l, q, max_ctx, split, buf)
         assert all(torch.equal(x, y) for x, y in zip(got, want))

@@ -994,11 +994,13 @@ __global__ __launch_bounds__(kSpreadWaves * 64, kWavesPerSimd) void decode_sprea
   const int n_pages = pages_of(ctx), nch = chunks_of(ctx, a.chunk_pages);
   if (c >= nch) return;
   // A few pages: one workgroup, a page per wavefront, and no round trips of
-  // partials and flags (about 1.6 us; with max_context_len 4096, 64 tokens
-  // took 6.6 us by them and take 5.3, 190 tokens 7.0 and 7.7).  The same
-  // bits: of kWaves wavefronts those without a page would add nothing, and
-  // the others fold in the order of their pages.
-  constexpr int kFew = S == kSpreadWaves ? 4 : 2;
+  // partials and flags (max_context_len 4096, us by flags / without: D 64, 16
+  // pairs, 3 and 4 pages 5.8 / 4.9, 5.8 / 5.1; 64 pairs 6.6 / 5.1, 6.9 / 5.3;
+  // D 128, 64 pairs 7.9 / 7.5, 8.2 / 7.9; 32 pairs 7.9 / 7.2 and, the other
+  // side of the line, 7.6 / 7.9).  The same bits: of kWaves wavefronts those
+  // without a page would add nothing, and the others fold in the order of
+  // their pages.
+  constexpr int kFew = D == 128 && S == 1 ? 3 : 4;
   static_assert(kFew <= kSpreadWaves, "a page per wavefront");
   if (n_pages <= kFew) {
     if (wg == 0) run_item<D, false, kSpreadWaves>(a, b, 0, kvh, wave, lane);
@@ -1392,18 +1394,31 @@ bool merges_in_kernel(int B, int Hq, int Hkv, int D, int max_context_len, int sp
          spyre_paged_decode_attn_workspace_bytes(B, Hq, Hkv, D, max_context_len, split_tokens) < (size_t{1} << 31);
 }
 
+// Pages of max_context_len from which a call whose contexts fit one chunk is
+// spread over workgroups of S wavefronts: below, the round trips of partials
+// and flags cost more than the idle units (us, one workgroup / spread, contexts
+// of max_context_len; pairs: sequences x KV heads):
+//  * D 128, S 1 (32 pairs): 3 pages 7.2 / 7.9, 4: 7.5 / 7.5, 5: 9.0 / 7.7;
+//    S 2 (64 pairs): 4: 7.6 / 8.2, 5: 9.2 / 8.7;
+//    S 4 (128 pairs): 6: 9.6 / 10.5, 7: 11.2 / 11.0, 10: 14.3 / 13.4;
+//  * D 64, S 1 (32 pairs): 6: 6.1 / 6.2, 7: 6.7 / 6.3;
+//    S 2 (64 pairs): 7: 6.8 / 6.9, 8: 7.0 / 6.9, 10: 8.9 / 7.8;
+//    S 4 (128 pairs): 5: 6.1 / 7.8, 12: 9.6 / 9.7, 14: 10.1 / 10.0, 28: 16.8 / 14.1.
+int spread_pages(int D, int S) {
+  return D == 128 ? (S == 1 ? 4 : S == 2 ? 5 : 7) : S == 1 ? 7 : S == 2 ? 8 : 14;
+}
+
 // Wavefronts per workgroup of decode_spread_kernel (1, 2 or 4) for a call of
 // these sizes, 0 where it does not pay: the least whose workgroups still
 // find a compute unit each.  Twice as many lost it: B 12 x 4096 tokens 36.3 us
 // at one each and 41.1 at two, B 24 (192 items) 62.7 unspread and 75.9.
-constexpr int kSpreadPages = 3;  // pages at least: below, one workgroup has a page per wavefront
 int spread_waves(int B, int Hkv, int D, int max_context_len, int split_tokens) {
   const int64_t slots = split_slots(D);
   const int64_t chunks = max_chunks_for(max_context_len, split_tokens);
-  if (slots <= 0 || pages_of(max_context_len) < kSpreadPages || chunks > kSpreadChunks) return 0;
+  if (slots <= 0 || chunks > kSpreadChunks) return 0;
   const int64_t items = static_cast<int64_t>(B) * Hkv * chunks;
   for (int S = 1; S < kWaves; S *= 2)
-    if (items * (kWaves / S) <= slots) return S;
+    if (items * (kWaves / S) <= slots) return chunks > 1 || pages_of(max_context_len) >= spread_pages(D, S) ? S : 0;
   return 0;
 }
 
