@@ -867,27 +867,25 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   // (-inf, the type's lowest number) does not count: when no row has a number
   // that adds something, the NaN rows are gone through with their biases.
   auto adds = [&](int t, float mx, const f32x16* s) {
-    const bool number = mx >= fmaxf(m_run - 32.f, -__FLT_MAX__);  // (-inf is not)
-    bool any = __builtin_amdgcn_ballot_w64(q_ok && number) != 0;
+    const float least = fmaxf(m_run - 32.f, -__FLT_MAX__);  // (-inf is below it)
+    if constexpr (MK != kMaskF16) return __builtin_amdgcn_ballot_w64(q_ok && !(mx < least)) != 0;
+    bool any = __builtin_amdgcn_ballot_w64(q_ok && mx >= least) != 0;
     if (__builtin_expect(!any && __builtin_amdgcn_ballot_w64(q_ok && mx != mx) != 0, 0)) {
-      any = true;
-      if constexpr (MK == kMaskF16) {
-        constexpr float kDropped = -1024.f;
-        const char* blk = reinterpret_cast<const char*>(mask_block(t & 1));
-        bool some = false;
+      constexpr float kDropped = -1024.f;
+      const char* blk = reinterpret_cast<const char*>(mask_block(t & 1));
+      bool some = false;
 #pragma unroll
-        for (int hf = 0; hf < (HALF ? 1 : 2); ++hf)
+      for (int hf = 0; hf < (HALF ? 1 : 2); ++hf)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const f16x4 m4 = *reinterpret_cast<const f16x4*>(blk + (m_lane ^ (64 * hf + 32 * (i >> 1))) + 8 * (i & 1));
+        for (int i = 0; i < 4; ++i) {
+          const f16x4 m4 = *reinterpret_cast<const f16x4*>(blk + (m_lane ^ (64 * hf + 32 * (i >> 1))) + 8 * (i & 1));
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-              const float x = PRESCALED ? s[hf][4 * i + v] + m_use : s[hf][4 * i + v] * scale_abs;
-              some = some || (x != x ? !(static_cast<float>(m4[v]) <= kDropped) : x > -INFINITY && x >= m_run - 32.f);
-            }
+          for (int v = 0; v < 4; ++v) {
+            const float x = PRESCALED ? s[hf][4 * i + v] + m_use : s[hf][4 * i + v] * scale_abs;
+            some = some || (x != x ? !(static_cast<float>(m4[v]) <= kDropped) : x > -INFINITY && x >= m_run - 32.f);
           }
-        any = __builtin_amdgcn_ballot_w64(q_ok && mx != mx && some) != 0;
-      }
+        }
+      any = __builtin_amdgcn_ballot_w64(q_ok && mx != mx && some) != 0;
     }
     return any;
   };
