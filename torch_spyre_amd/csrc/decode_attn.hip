@@ -525,10 +525,10 @@ __device__ __forceinline__ void stream_pages(const SplitArgs& a, int b, int kvh,
   };
   f16x8 ka[4][DS];
   VT va[VR][2];
-  int run = next_run(0);
+  int next = next_run(0);  // masked: the run that step streams
   {
     Rsrc kr, vr;
-    locate(run, kr, vr);
+    locate(next, kr, vr);
     if (DENSE && ctx < kPage) {
       if constexpr (DENSE) {  // the one short run
         load_k_dense<D, false>(ka, kr, lo, k_row);
@@ -545,6 +545,7 @@ __device__ __forceinline__ void stream_pages(const SplitArgs& a, int b, int kvh,
   // sets of registers at D = 64, where they fit, measured slower: 46.7 ->
   // 48.9 us for B 32 x 16 heads x 2048 tokens.)
   auto step = [&](int it) {
+    const int run = MK == kDecodeNoMask ? run_of(it) : next;
     int lo_tok, valid;  // this run's own window tokens: [lo_tok, valid)
     window(run, lo_tok, valid);
     // The mask of this lane's tokens, in flight during the QK products.
@@ -570,15 +571,15 @@ __device__ __forceinline__ void stream_pages(const SplitArgs& a, int b, int kvh,
     // The K registers are consumed: start the next run's K loads into them
     // now, so they are in flight during this run's softmax and PV.
     const int nx = it + 1;
-    const bool more = nx < n_run;
+    const bool more = nx < (MK == kDecodeNoMask ? n_it : n_run);
     Rsrc kr, vr;
     if (more) {
-      run = next_run(nx);
+      next = next_run(nx);
       if (!DENSE && (nx & 63) == 0) {  // the page ids of the next 64 runs
         const int q = nx + lane;
         ids = q < n_it ? trow[q] : 0;
       }
-      locate(run, kr, vr);
+      locate(next, kr, vr);
       issue_k(ka, kr);
     }
 
@@ -664,7 +665,7 @@ __device__ __forceinline__ void stream_pages(const SplitArgs& a, int b, int kvh,
     if (more) issue_v(va, vr);
   };
 
-  for (int it = 0; it < n_run; ++it) step(it);
+  for (int it = 0; it < (MK == kDecodeNoMask ? n_it : n_run); ++it) step(it);
   if (poisoned) l_run = NAN;  // propagates to the merged output: NaN, not a fault
   l_run += wave_xor(l_run, 16);
   l_run += wave_xor(l_run, 32);
