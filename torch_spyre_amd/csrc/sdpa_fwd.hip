@@ -831,6 +831,7 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
   auto apply_mask = [&](int t, f32x16 (&s)[2]) {
     apply_mask_half(t, 0, s[0]);
     apply_mask_half(t, 1, s[1]);
+    next_mask(t);
   };
   // The running max (log2 domain) moves only when a score of the step
   // exceeds it by more than 2^8, so P <= 256 (fine in fp16) and most steps
@@ -861,31 +862,27 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
     return PRESCALED ? max_halves(mx) + m_use : max_halves(mx) * scale_abs;
   };
   // Whether a masked step adds anything to a real row: mx is this lane's row
-  // max (of both lane halves), s its scores (half steps: one half, else two).
-  // A NaN does.  Boolean masks leave none on a dropped key; an fp16 bias may
-  // (a cache's unused keys), so a NaN under one that alone makes the weight 0
-  // (-inf, the type's lowest number) does not count: when no row has a number
-  // that adds something, the NaN rows are gone through with their biases.
-  auto adds = [&](int t, float mx, const f32x16* s) {
+  // max (of both lane halves).  A NaN does.  Boolean masks leave none on a
+  // dropped key; an fp16 bias may (a cache's unused keys), so in a step where
+  // no row has a number that adds something, a NaN row counts only if it
+  // keeps a key, i.e. has a bias other than one that alone makes the weight 0
+  // (-inf, the type's lowest number).  Read from memory, since the block in
+  // LDS may be the next step's by now.
+  auto adds = [&](int t, float mx) {
     const float least = fmaxf(m_run - 32.f, -__FLT_MAX__);  // (-inf is below it)
     if constexpr (MK != kMaskF16) return __builtin_amdgcn_ballot_w64(q_ok && !(mx < least)) != 0;
     bool any = __builtin_amdgcn_ballot_w64(q_ok && mx >= least) != 0;
     if (__builtin_expect(!any && __builtin_amdgcn_ballot_w64(q_ok && mx != mx) != 0, 0)) {
       constexpr float kDropped = -1024.f;
-      const char* blk = reinterpret_cast<const char*>(mask_block(t & 1));
-      bool some = false;
-#pragma unroll
-      for (int hf = 0; hf < (HALF ? 1 : 2); ++hf)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const f16x4 m4 = *reinterpret_cast<const f16x4*>(blk + (m_lane ^ (64 * hf + 32 * (i >> 1))) + 8 * (i & 1));
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const float x = PRESCALED ? s[hf][4 * i + v] + m_use : s[hf][4 * i + v] * scale_abs;
-            some = some || (x != x ? !(static_cast<float>(m4[v]) <= kDropped) : x > -INFINITY && x >= m_run - 32.f);
-          }
-        }
-      any = __builtin_amdgcn_ballot_w64(q_ok && mx != mx && some) != 0;
+      const int at = kb0 + t * kKT + (HALF ? 32 * hw : 0) + 8 * half, n = HALF ? 2 : 4;
+      bool keeps = false;
+      if (q_ok) {
+        const _Float16* row = static_cast<const _Float16*>(a.mask) + b * a.m_sb + h * a.m_sh + qi * a.m_sq + at;
+#pragma unroll 1
+        for (int k = 0; k < 16 * n; ++k)  // this lane's: 8 of every 16 keys
+          keeps = keeps || ((k & 8) == 0 && at + k <= key_last && !(static_cast<float>(row[k]) <= kDropped));
+      }
+      any = __builtin_amdgcn_ballot_w64(q_ok && mx != mx && keeps) != 0;
     }
     return any;
   };
@@ -1113,7 +1110,6 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
         if (i + kPrefetch < kNFH) fr[i + kPrefetch] = frag_h(i + kPrefetch);
       };
       if constexpr (MK != kNoMask) {
-        static_assert(!HALF || MK != kMaskF16 || kMaskSlots == 2, "adds() reads the block after next_mask");
         apply_mask_half(t, 0, cur);
         next_mask(t);
       }
@@ -1132,7 +1128,7 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
       for (int rr = 0; rr < 16; ++rr) mx = max_of(mx, cur[rr]);
       mx = PRESCALED ? max_halves(mx) + m_use : max_halves(mx) * (F32M ? 1.f : scale_abs);
       // A step the mask blanks for every real row adds nothing (see step).
-      const bool live = MK == kNoMask || adds(t, mx, &cur);
+      const bool live = MK == kNoMask || adds(t, mx);
       if (live && __builtin_amdgcn_ballot_w64(mx > m_run + kLazy) != 0) {
         const float m_new = fmaxf(m_run, mx);
         const float alpha = m_new == -INFINITY ? 1.f : fast_exp2(m_run - m_new);
@@ -1257,11 +1253,7 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
         apply_mask(t, cur);
         if (edge(t)) mask_step(t, cur);
         const float mx = row_max(cur);
-        bool live = true;
-        if (kMaskSlots == 1) {
-          live = adds(t, mx, cur);
-          next_mask(t);
-        }
+        const bool live = adds(t, mx);
         nxt[0] = PRESCALED ? neg_m_tile : f32x16{};
         nxt[1] = PRESCALED ? neg_m_tile : f32x16{};
 #pragma unroll
@@ -1270,7 +1262,6 @@ __global__ __launch_bounds__(W * 64, 2) void sdpa_fwd_lds_kernel(Fwd2Args a) {
           mfma(2 * ks + 1, qv[ks], nxt[1]);
         }
         interleave_reads(0, 2 * DK);
-        if (kMaskSlots == 2) live = adds(t, mx, cur);
         if (live) {
           update_max(cur, nxt, mx);
           rebase(cur[0]);
