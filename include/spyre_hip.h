@@ -281,8 +281,8 @@ int spyre_paged_decode_attn_noalloc_f16(const void* q, const void* k_cache, cons
  * a mask (plain or causal) need no workspace. */
 size_t spyre_sdpa_fwd_workspace_bytes(int B, int Hkv, int Skv, int D);
 
-/* The workspace one spyre_sdpa_fwd_f16 call needs (same arguments as the
- * call, less the causal flag).  Without a mask: the fp32 partials of a key
+/* The workspace that covers one spyre_sdpa_fwd_f16 or spyre_sdpa_fwd_own_f16
+ * call (same arguments as the call, less the causal flag).  Without a mask: the fp32 partials of a key
  * split, B * Hq * Sq * nsplit * (D + 2) * 4 bytes, when the call's blocks
  * would not fill the device (short query runs, few sequences, long keys),
  * plus, when each KV head's g q heads x Sq queries fit one 32-row tile (the
@@ -318,7 +318,8 @@ size_t spyre_sdpa_fwd_call_workspace_bytes(const void* attn_mask, int mask_kind,
  * arguments): 0 without a mask or for a mask staged as it lies; the smaller
  * of its copy and V's relayout for other fp16 / bool masks; V's relayout for
  * fp32 masks.  What spyre_sdpa_fwd_call_workspace_bytes asks beyond it only
- * makes the call faster. */
+ * makes the call faster (for masks staged as they lie: of
+ * spyre_sdpa_fwd_own_f16). */
 size_t spyre_sdpa_fwd_min_workspace_bytes(const void* attn_mask, int mask_kind,
                                           const int64_t* mask_strides, int B, int Hq, int Hkv,
                                           int Sq, int Skv, int D);
